@@ -1,0 +1,59 @@
+// Device helpers shared by the kernel translation units: mesh gathers and the
+// batched kernels' view of a case.
+#pragma once
+#include "simplic_device.hpp"
+#include "simplic_types.hpp"
+
+namespace svp {
+
+static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
+
+// where a gathered empty-patch flag of face f is read: f itself for a
+// boundary face; for an interior face (never empty, and its flag unused) the
+// first boundary face's, clamped into the array when there is none
+__device__ inline int empty_slot(const DevMesh& m, int f) { return min(max(f, m.nIF), m.nF - 1); }
+
+// volPointInterpolation value at a point: the weighted sum of its source
+// values in source order.  A point of up to PU_SLOTS sources (every interior
+// point of a hexahedral mesh) loads all source labels and weights, then all
+// their values, before the sum, instead of waiting on two loads per source.
+constexpr int PU_SLOTS = 8;
+__device__ inline V3 point_u(const DevMesh& m, const DevState& st, int p) {
+    const int o0 = m.psOff[p], n = m.psOff[p + 1] - o0;
+    V3 t = VZERO;
+    if (n >= 1 && n <= PU_SLOTS) {
+        int src[PU_SLOTS];
+        double w[PU_SLOTS];
+        V3 u[PU_SLOTS];
+#pragma unroll
+        for (int k = 0; k < PU_SLOTS; ++k) {
+            src[k] = m.psSrc[o0 + min(k, n - 1)];
+            w[k] = m.psW[o0 + min(k, n - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < PU_SLOTS; ++k) {
+            // a source is a cell (>= 0) or a boundary face (~face)
+            const double* base = src[k] >= 0 ? st.U : st.Ub;
+            const int idx = src[k] >= 0 ? src[k] : (~src[k]) - m.nIF;
+            u[k] = ld3(base, idx);
+        }
+#pragma unroll
+        for (int k = 0; k < PU_SLOTS; ++k)
+            if (k < n) t = t + w[k] * u[k];
+        return t;
+    }
+    for (int k = o0; k < o0 + n; ++k) {
+        const int s = m.psSrc[k];
+        const V3 u = (s >= 0) ? ld3(st.U, s) : ld3(st.Ub, (~s) - m.nIF);
+        t = t + m.psW[k] * u;
+    }
+    return t;
+}
+
+// state view of a batched case: buffers as they are (swapped 0) or with alpha
+// and alphaOld exchanged, bounding half of pass number `pass` of the step
+__device__ inline const DevState& batch_view(const BatchCase& c, const BatchStepInfo& si, int swapped, int pass) {
+    return c.st[((si.aPar ^ swapped) << 1) | (si.hPar ^ (pass & 1))];
+}
+
+}  // namespace svp

@@ -561,129 +561,6 @@ __device__ __attribute__((always_inline)) inline void combineSubCell(const FaceC
     (void)Cc;
 }
 
-// combineSubCell for a lane group that holds one face per lane (lane l: face
-// l of the cell, records rec[0..nF) in LDS, written by their lanes).  The
-// per-face terms that do not depend on the running sums are computed by the
-// face's own lane: the first interface segment of a cut face (its centre sum,
-// normal and area) and the pyramid volume against cEst; every lane then adds
-// them in the reference's face order, so the sums and the result are those
-// of combineSubCell.  seg/pyr: the group's scratch in LDS (nF entries each).
-struct SegTerm {
-    V3 c, nn;
-    double ar;
-};
-
-__device__ __attribute__((always_inline)) inline void combineSubCellGroup(const FaceCut* fc, SegTerm* seg, double* pyr,
-                                                                           int nF, int l, double Vc, CellCut& out) {
-    bool fullySubmerged = true, fullyEmpty = true;
-    int nSubmergedFaces = 0;
-    for (int f = 0; f < nF; ++f) {
-        if (fc[f].status == 0) {
-            fullySubmerged = false;
-            fullyEmpty = false;
-        } else if (fc[f].status == -1) {
-            fullyEmpty = false;
-            nSubmergedFaces++;
-        } else {
-            fullySubmerged = false;
-        }
-    }
-    out.ifCentre = VZERO;
-    out.ifArea = VZERO;
-    if (!fullySubmerged && !fullyEmpty) {
-        out.status = 0;
-        // calcInterfaceCentreAndArea (cutCell.C:37-100)
-        V3 fCentre = VZERO;
-        int nEdgePoints = 0;
-        for (int f = 0; f < nF; ++f) {
-            if (fc[f].status != 0) continue;
-            for (int k = 0; k < fc[f].nIf; ++k) {
-                fCentre = fCentre + fc[f].ifPts[k];
-                nEdgePoints++;
-            }
-        }
-        if (nEdgePoints > 0) fCentre = fCentre / (double)nEdgePoints;
-        if (l < nF && fc[l].status == 0 && fc[l].nIf >= 2) {
-            const V3 a = fc[l].ifPts[0], b = fc[l].ifPts[1];
-            seg[l].c = a + b + fCentre;
-            const V3 nn = cross(b - a, fCentre - a);
-            seg[l].nn = nn;
-            seg[l].ar = mag(nn);
-        }
-        __builtin_amdgcn_wave_barrier();
-        V3 sumN = VZERO, sumAc = VZERO;
-        double sumA = 0.0;
-        for (int f = 0; f < nF; ++f) {
-            if (fc[f].status != 0) continue;
-            for (int k = 0; k < fc[f].nIf - 1; ++k) {
-                V3 c, nn;
-                double ar;
-                if (k == 0) {
-                    c = seg[f].c;
-                    nn = seg[f].nn;
-                    ar = seg[f].ar;
-                } else {
-                    const V3 a = fc[f].ifPts[k], b = fc[f].ifPts[k + 1];
-                    c = a + b + fCentre;
-                    nn = cross(b - a, fCentre - a);
-                    ar = mag(nn);
-                }
-                sumN = sumN + sgn(dot(nn, sumN)) * nn;
-                sumA += ar;
-                sumAc = sumAc + ar * c;
-            }
-        }
-        if (sumA < SVP_ROOTVSMALL) {
-            out.ifCentre = fCentre;
-            out.ifArea = VZERO;
-        } else {
-            out.ifCentre = (1.0 / 3.0) * sumAc / sumA;
-            out.ifArea = 0.5 * sumN;
-        }
-        if (dot(out.ifArea, out.ifCentre - VZERO) < 0.0) out.ifArea = (-1.0) * out.ifArea;
-        if (mag(out.ifArea) < SVP_TSMALL) {
-            if (nSubmergedFaces == 0) {
-                out.status = 1;
-                out.VOF = 0.0;
-            } else {
-                out.status = -1;
-                out.VOF = 1.0;
-            }
-            return;
-        }
-        // calcSubCellCentreAndVolume (cutCell.C:103-137)
-        V3 sum = VZERO;
-        int cnt = 0;
-        for (int f = 0; f < nF; ++f)
-            if (fc[f].status != 1) {
-                sum = sum + fc[f].centre;
-                cnt++;
-            }
-        sum = sum + out.ifCentre;
-        cnt++;
-        const V3 cEst = sum / (double)cnt;
-        if (l < nF && fc[l].status != 1) pyr[l] = fmax(fabs(dot(fc[l].area, fc[l].centre - cEst)), SVP_VSMALL);
-        __builtin_amdgcn_wave_barrier();
-        double vol = 0.0;
-        for (int f = 0; f < nF; ++f) {
-            if (fc[f].status == 1) continue;
-            vol += pyr[f];
-        }
-        {
-            const double pyr3Vol = fmax(fabs(dot(out.ifArea, out.ifCentre - cEst)), SVP_VSMALL);
-            vol += pyr3Vol;
-        }
-        vol /= 3.0;
-        out.VOF = vol / Vc;
-    } else if (fullyEmpty) {
-        out.status = 1;
-        out.VOF = 0.0;
-    } else {
-        out.status = -1;
-        out.VOF = 1.0;
-    }
-}
-
 // Cut the whole cell sequentially (one lane)
 template <class Poly>
 __device__ inline bool calcSubCell(const Poly& P, V3 Cc, double Vc, V3 normal, double distance,

@@ -6,12 +6,9 @@
 // (compiled with -ffp-contract=off); each kernel cites the reference lines it
 // follows.  Control flow that the reference runs on the host (mixed-cell count,
 // bounding passes) stays on the device, so a step never waits for the host.
-#include "simplic_device.hpp"
-#include "simplic_types.hpp"
+#include "mesh_device.hpp"
 
 namespace svp {
-
-static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
 // ---------------------------------------------------------------------------
 // Mesh geometry (OpenFOAM primitiveMeshTools), computed once at create time
@@ -124,11 +121,6 @@ int detect_blocks(int nC) { return cdiv(nC, DETECT_BLOCK); }
 // published.  Counts stay below 2^30.
 constexpr unsigned long long LOOK_AGG = 1ull << 30, LOOK_PREFIX = 2ull << 30;
 constexpr int LOOK_SPIN_LIMIT = 1 << 22;
-
-// where a gathered empty-patch flag of face f is read: f itself for a
-// boundary face; for an interior face (never empty, and its flag unused) the
-// first boundary face's, clamped into the array when there is none
-__device__ inline int empty_slot(const DevMesh& m, int f) { return min(max(f, m.nIF), m.nF - 1); }
 
 // The block's ticket (thread 0 only).  The counter only grows, by nBlocks per
 // launch (every launch of a kernel on one counter has the same grid, and every
@@ -1020,369 +1012,18 @@ __global__ void __launch_bounds__(64) k_find_signed_distance(DevMesh m, DevState
     }
 }
 
-// findSignedDistance with one G-lane group per mixed cell and one lane per
-// cell face (cells of at most G faces and 16 points, faces as stored; G is
-// the mesh's largest face count: 4 for tetrahedra (16 cells per wave), 6 for
-// hexahedra (10 cells per wave, 4 lanes idle), else 8).  A
-// plane cut = every lane cuts its face (points in registers), writes the face
-// record to LDS, and every lane of the group combines the records in face
-// order, so all lanes hold the same VOF and follow the same bracketing and
-// Newton steps as the one-lane version.  The vertex levels are sorted by rank
-// in LDS.  One wave per workgroup: LDS traffic of a wave is in order.
-
-// volPointInterpolation value at a point: the weighted sum of its source
-// values in source order.  A point of up to PU_SLOTS sources (every interior
-// point of a hexahedral mesh) loads all source labels and weights, then all
-// their values, before the sum, instead of waiting on two loads per source.
-constexpr int PU_SLOTS = 8;
-__device__ inline V3 point_u(const DevMesh& m, const DevState& st, int p) {
-    const int o0 = m.psOff[p], n = m.psOff[p + 1] - o0;
-    V3 t = VZERO;
-    if (n >= 1 && n <= PU_SLOTS) {
-        int src[PU_SLOTS];
-        double w[PU_SLOTS];
-        V3 u[PU_SLOTS];
-#pragma unroll
-        for (int k = 0; k < PU_SLOTS; ++k) {
-            src[k] = m.psSrc[o0 + min(k, n - 1)];
-            w[k] = m.psW[o0 + min(k, n - 1)];
-        }
-#pragma unroll
-        for (int k = 0; k < PU_SLOTS; ++k) {
-            // a source is a cell (>= 0) or a boundary face (~face)
-            const double* base = src[k] >= 0 ? st.U : st.Ub;
-            const int idx = src[k] >= 0 ? src[k] : (~src[k]) - m.nIF;
-            u[k] = ld3(base, idx);
-        }
-#pragma unroll
-        for (int k = 0; k < PU_SLOTS; ++k)
-            if (k < n) t = t + w[k] * u[k];
-        return t;
-    }
-    for (int k = o0; k < o0 + n; ++k) {
-        const int s = m.psSrc[k];
-        const V3 u = (s >= 0) ? ld3(st.U, s) : ld3(st.Ub, (~s) - m.nIF);
-        t = t + m.psW[k] * u;
-    }
-    return t;
-}
-
-__device__ __attribute__((always_inline)) inline void fsd_face_cut(int fsz, const V3 (&q4)[4], const V3 (&q3)[3], V3 n, double dist,
-                                    FaceCut& fc, bool& ok, const double* full, const double (&dots)[4]) {
-    if (fsz == 4) ok &= calcSubFaceN<4, true, true>(q4, n, dist, fc, full, dots);
-    else ok &= calcSubFaceN<3, true, true>(q3, n, dist, fc, full, dots);
-}
-
-// waves per SIMD the register allocation of the interface-cell kernels
+// waves per SIMD the register allocation of the interface-flux kernels
 // targets (build-time tuning; results do not depend on it)
-#ifndef SVP_FSD_WAVES
-#define SVP_FSD_WAVES 2
-#endif
 #ifndef SVP_FLUX_WAVES
 #define SVP_FLUX_WAVES 1
 #endif
 
-template <int G>
-__device__ __attribute__((always_inline)) inline void k_fsd_group_body(const DevMesh& m, const DevState& st, const int* wl, const int* wn) {
-    static_assert(G >= 3 && G <= 8, "groups of 3 to 8 lanes");
-    constexpr int NG = 64 / G;                         // groups per wave; lanes past NG * G idle
-    constexpr int PPL = (NS_CELL_POINTS + G - 1) / G;  // cell points per lane
-    __shared__ FaceCut rec[NG][G];
-    __shared__ double full[NG][G][6];   // the lane's face as a fully submerged sub-face
-    __shared__ SegTerm seg[NG][G];      // per-face terms of the cut combination
-    __shared__ double pyr[NG][G];
-    __shared__ double vraw[NG][NS_CELL_POINTS];
-    __shared__ double vsrt[NG][NS_CELL_POINTS];
-    const int g = threadIdx.x / G, l = threadIdx.x % G;
-    if (g >= NG) return;
-    const int nWork = wl ? *wn : *st.nMixed;
-    for (int wi = blockIdx.x * NG + g; wi < nWork; wi += gridDim.x * NG) {
-        const int i = wl ? wl[wi] : wi;
-        const int c = st.mixed[i];
-        const int fb = m.cOff[c], nF = m.cOff[c + 1] - fb;
-        const int pb = m.cpOff[c], np = m.cpOff[c + 1] - pb;
-        const V3 normalI = ld3(st.ifN, i);
-        const double alphaI = st.alpha[c];
-        const V3 Cc = ld3(m.C, c);
-        const double Vc = m.V[c];
-        if (mag(normalI) < SVP_TSMALL) {
-            if (l == 0) {
-                st.status[i] = (int)sgn(0.5 - alphaI);
-                st.nCutPts[i] = 0;
-                st.faceClass[i] = 0ull;
-                if (!st.fsdKeep) {
-                    st.ifD[i] = 0.0;
-                    st3(st.ifC, i, VZERO);
-                    st3(st.ifS, i, VZERO);
-                }
-                st.un0[i] = 0.0;
-            }
-            continue;
-        }
-        // The lane's face (faces of 3 or 4 points) and its two cell points,
-        // every load unconditional (slots past the cell's faces or points,
-        // or past a triangle's third point, repeat the last one): the face
-        // chain and the point chain then go out together, where loads under
-        // a lane condition would each wait for all the loads before them.
-        const int fL = m.cFaces[fb + min(l, nF - 1)];
-        const int cpA = m.cPts[pb + min(l, np - 1)], cpB = m.cPts[pb + min(l + G, np - 1)];
-        const int s0 = m.fOff[fL], fszL = m.fOff[fL + 1] - s0;
-        int plL[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) plL[k] = m.fPts[s0 + min(k, fszL - 1)];
-        V3 qq[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) qq[k] = ld3(m.pts, plL[k]);
-        const V3 ptA = ld3(m.pts, cpA), ptB = ld3(m.pts, cpB);
-        double fcs[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) fcs[k] = m.fullCS[6L * fL + k];
-        int fsz = 0, myFace = -1;
-        V3 q4[4], q3[3];
-        int pl[4] = {0, 0, 0, 0};
-        if (l < nF) {
-            myFace = fL;
-            fsz = fszL;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) pl[k] = k < fsz ? plL[k] : 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) q4[k] = qq[k];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) q3[k] = qq[k];
-#pragma unroll
-            for (int k = 0; k < 6; ++k) full[g][l][k] = fcs[k];
-        }
-        // the plane's normal is fixed for the cell: dot(point, n) once
-        double dots[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) dots[k] = (fsz == 4) ? dot(q4[k], normalI) : (k < 3 ? dot(q3[k], normalI) : 0.0);
-        // vertex levels -n.x of the cell points, sorted descending by rank
-        // (points past PPL per lane cannot occur: np <= NS_CELL_POINTS = PPL * G)
-        double va = 0.0, vb = 0.0;
-        if (l < np) va = -dot(normalI, ptA);
-        if (l + G < np) vb = -dot(normalI, ptB);
-        if (l < np) vraw[g][l] = va;
-        if (l + G < np) vraw[g][l + G] = vb;
-        if constexpr (PPL > 2) {
-            for (int k = l + 2 * G; k < np; k += G) vraw[g][k] = -dot(normalI, ld3(m.pts, m.cPts[pb + k]));
-        }
-        __builtin_amdgcn_wave_barrier();
-        {
-            int ra = 0, rb = 0;
-            for (int j = 0; j < np; ++j) {
-                const double v = vraw[g][j];
-                ra += (v > va) || (v == va && j < l);
-                rb += (v > vb) || (v == vb && j < l + G);
-            }
-            if (l < np) vsrt[g][ra] = va;
-            if (l + G < np) vsrt[g][rb] = vb;
-            if constexpr (PPL > 2) {
-                for (int k = l + 2 * G; k < np; k += G) {
-                    const double vk = vraw[g][k];
-                    int rk = 0;
-                    for (int j = 0; j < np; ++j) {
-                        const double v = vraw[g][j];
-                        rk += (v > vk) || (v == vk && j < k);
-                    }
-                    vsrt[g][rk] = vk;
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        bool ok = true;
-        auto cut = [&](double dist, CellCut& cc) {
-            if (l < nF) fsd_face_cut(fsz, q4, q3, normalI, dist, rec[g][l], ok, &full[g][l][0], dots);
-            __builtin_amdgcn_wave_barrier();
-            combineSubCellGroup(&rec[g][0], &seg[g][0], &pyr[g][0], nF, l, Vc, cc);
-            __builtin_amdgcn_wave_barrier();
-        };
-        // cutCell::findSignedDistance (cutCell.C:611-799) as one loop around a
-        // single cut, so the cut's code exists once (the kernel's instruction
-        // footprint decides its speed): phase 0 bisects over the vertex
-        // levels, 1 and 2 cut at a third and two thirds of the last bracket,
-        // 3 is the final cut at the plane found
-        double lowDistance = vsrt[g][0], upDistance = vsrt[g][np - 1];
-        int lowLabel = 0, upLabel = np - 1;
-        double lowAlpha = 0.0, upAlpha = 1.0;
-        CellCut cc;
-        double dOut = 0.0, deltaDistance = 0.0, alphaOneThird = 0.0;
-        int phase = 0, midLabel = 0;
-        while (true) {
-            double dist;
-            if (phase == 0) {
-                if ((upLabel - lowLabel) > 1) {
-                    midLabel = (int)round(0.5 * (double)(upLabel + lowLabel));
-                    dist = vsrt[g][midLabel];
-                } else if (fabs(lowDistance - upDistance) < SVP_TSMALL) {
-                    dOut = 0.5 * (lowDistance + upDistance);
-                    dist = dOut;
-                    phase = 3;
-                } else {
-                    deltaDistance = (upDistance - lowDistance) / 3.0;
-                    dist = lowDistance + deltaDistance;
-                    phase = 1;
-                }
-            } else if (phase == 2) {
-                dist = lowDistance + 2.0 * deltaDistance;
-            } else {
-                dist = dOut;
-            }
-            cut(dist, cc);
-            if (phase == 0) {
-                const double midDistance = dist;
-                const double midAlpha = cc.VOF;
-                if (fabs(midAlpha - alphaI) < SVP_TSMALL) {
-                    dOut = midDistance;
-                    break;
-                }
-                if (midAlpha > alphaI) {
-                    upLabel = midLabel;
-                    upDistance = midDistance;
-                    upAlpha = midAlpha;
-                } else {
-                    lowLabel = midLabel;
-                    lowDistance = midDistance;
-                    lowAlpha = midAlpha;
-                }
-            } else if (phase == 1) {
-                alphaOneThird = cc.VOF - lowAlpha;
-                phase = 2;
-            } else if (phase == 2) {
-                const double alphaPrismatoid = upAlpha - lowAlpha;
-                const double alphaTwoThirds = cc.VOF - lowAlpha;
-                const double a = 13.5 * alphaOneThird - 13.5 * alphaTwoThirds + 4.5 * alphaPrismatoid;
-                const double b = -22.5 * alphaOneThird + 18.0 * alphaTwoThirds - 4.5 * alphaPrismatoid;
-                const double cq = 9.0 * alphaOneThird - 4.5 * alphaTwoThirds + 1.0 * alphaPrismatoid;
-                const double d = lowAlpha - alphaI;
-                double lambda = 0.5;
-                for (int iter = 0; iter < 100; iter++) {
-                    const double func = a * (lambda * lambda * lambda) + b * (lambda * lambda) + cq * lambda + d;
-                    const double funcPrime = 3.0 * a * (lambda * lambda) + 2.0 * b * lambda + cq;
-                    const double lambdaNew = lambda - (func / funcPrime);
-                    if (fabs(lambdaNew - lambda) < SVP_TSMALL) break;
-                    lambda = lambdaNew;
-                }
-                dOut = lowDistance - lambda * (lowDistance - upDistance);
-                phase = 3;
-            } else {
-                break;
-            }
-        }
-        if (l == 0) {
-            unsigned long long fcls = 0ull;
-            int ncp = 0;
-            for (int k = 0; k < nF; ++k) {
-                const int s2 = rec[g][k].status;
-                fcls |= (unsigned long long)(s2 + 1) << (2 * k);
-                if (s2 == 0) ncp += rec[g][k].nIf;
-            }
-            st.status[i] = cc.status;
-            st.nCutPts[i] = ncp;
-            st.faceClass[i] = fcls;
-            st.ifD[i] = dOut;
-            st3(st.ifC, i, cc.ifCentre);
-            st3(st.ifS, i, cc.ifArea);
-        }
-        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
-        __builtin_amdgcn_wave_barrier();
-        // Un0 = U(interface centre) . n for a cut cell (advection.C:126):
-        // interpolationCellPoint's tet search with one lane per face
-        double un0 = 0.0;
-        if (cc.status == 0) {
-            const double tol = SVP_SMALL;
-            const V3 pos = cc.ifCentre;
-            bool found = false;
-            double fw[4] = {0, 0, 0, 0}, bw[4] = {0, 0, 0, 0}, bestMin = -1e300;
-            int fp[3] = {0, 0, 0}, bp[3] = {0, 0, 0};
-            if (l < nF) {
-                const bool ownFace = (m.own[myFace] == c);
-#pragma unroll
-                for (int t = 1; t < 3; ++t) {
-                    if (t >= fsz - 1 || found) continue;
-                    int a0 = pl[0], a1 = (t == 1) ? pl[1] : pl[2], a2 = (t == 1) ? pl[2] : pl[3];
-                    V3 b0 = (fsz == 4) ? q4[0] : q3[0];
-                    V3 b1 = (fsz == 4) ? ((t == 1) ? q4[1] : q4[2]) : q3[1];
-                    V3 b2 = (fsz == 4) ? ((t == 1) ? q4[2] : q4[3]) : q3[2];
-                    if (!ownFace) {
-                        const int ti = a1; a1 = a2; a2 = ti;
-                        const V3 tv = b1; b1 = b2; b2 = tv;
-                    }
-                    const V3 e0 = Cc - b2, e1 = b0 - b2, e2 = b1 - b2;
-                    const double detT = dot(e0, cross(e1, e2));
-                    double w[4];
-                    if (fabs(detT) < SVP_SMALL) {
-                        w[0] = w[1] = w[2] = w[3] = -1.0;
-                    } else {
-                        const V3 r = pos - b2;
-                        w[0] = dot(r, cross(e1, e2)) / detT;
-                        w[1] = dot(e0, cross(r, e2)) / detT;
-                        w[2] = dot(e0, cross(e1, r)) / detT;
-                        w[3] = 1.0 - w[0] - w[1] - w[2];
-                    }
-                    const double mn = fmin(fmin(w[0], w[1]), fmin(w[2], w[3]));
-                    if (mn + tol > 0.0) {
-                        found = true;
-                        fw[0] = w[0]; fw[1] = w[1]; fw[2] = w[2]; fw[3] = w[3];
-                        fp[0] = a0; fp[1] = a1; fp[2] = a2;
-                    } else if (mn > bestMin) {
-                        bestMin = mn;
-                        bw[0] = w[0]; bw[1] = w[1]; bw[2] = w[2]; bw[3] = w[3];
-                        bp[0] = a0; bp[1] = a1; bp[2] = a2;
-                    }
-                }
-            }
-            // first face (in cell-face order) with a containing tet, else the
-            // tet of largest minimum weight, earliest on ties
-            const unsigned long long grpMask = ((1ull << G) - 1ull) << (g * G);
-            const unsigned long long foundMask = __ballot(found && l < nF) & grpMask;
-            int src = -1;
-            if (foundMask) {
-                src = __ffsll((long long)foundMask) - 1 - g * G;
-            } else {
-                double best = -1e300;
-                for (int k = 0; k < nF; ++k) {
-                    const double v = __shfl(bestMin, g * G + k);
-                    if (v > best) {
-                        best = v;
-                        src = k;
-                    }
-                }
-            }
-            double w[4];
-            int pp[3];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) w[q] = __shfl(foundMask ? fw[q] : bw[q], g * G + src);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) pp[q] = __shfl(foundMask ? fp[q] : bp[q], g * G + src);
-            // point values: lane q of the group evaluates point q
-            V3 pu = VZERO;
-            if (l < 3) pu = point_u(m, st, (l == 0) ? pp[0] : (l == 1 ? pp[1] : pp[2]));
-            V3 pv[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q)
-                pv[q] = v3(__shfl(pu.x, g * G + q), __shfl(pu.y, g * G + q), __shfl(pu.z, g * G + q));
-            const V3 Ui = w[0] * ld3(st.U, c) + w[1] * pv[0] + w[2] * pv[1] + w[3] * pv[2];
-            un0 = dot(Ui, normalI);
-        }
-        if (l == 0) st.un0[i] = un0;
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-template <int G>
-__global__ void __launch_bounds__(64, SVP_FSD_WAVES) k_fsd_group(DevMesh m, DevState st, const int* wl, const int* wn) {
-    k_fsd_group_body<G>(m, st, wl, wn);
-}
-
+// cells whose warped faces are split keep one lane per cell; all others take
+// a lane group per cell (plane_kernels.hip)
 void launch_find_signed_distance(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s,
                                  const int* wl, const int* wn) {
     if (p.splitWarpedFace) k_find_signed_distance<CellPolySP><<<1024, 64, 0, s>>>(m, st, 1, wl, wn);
-    else if (st.un0Fused && st.maxCellFaces <= 4) k_fsd_group<4><<<2048, 64, 0, s>>>(m, st, wl, wn);
-    else if (st.un0Fused && st.maxCellFaces <= 6) k_fsd_group<6><<<2048, 64, 0, s>>>(m, st, wl, wn);
-    else if (st.un0Fused) k_fsd_group<8><<<2048, 64, 0, s>>>(m, st, wl, wn);
-    else if (st.maxCellFaces <= NS_CELL_FACES && m.maxCellPoints <= NS_CELL_POINTS)
-        k_find_signed_distance<CellPolyNS><<<1024, 64, 0, s>>>(m, st, 0, wl, wn);
-    else k_find_signed_distance<CellPolyGen><<<1024, 64, 0, s>>>(m, st, 0, wl, wn);
+    else launch_fsd_group(m, st, s, wl, wn);
 }
 
 // ---------------------------------------------------------------------------
@@ -3267,7 +2908,8 @@ void launch_advect_stage(int stage, const DevMesh& m, const DevState& st, const 
             k_upwind<<<cdiv(m.nF, 256), 256, 0, s>>>(m, st, dt);
             break;
         case STAGE_IFLUX:
-            if (!st.un0Fused) k_un0<<<512, 64, 0, s>>>(m, st);
+            if (!st.placeGroup) k_un0<<<512, 64, 0, s>>>(m, st);
+            else if (!st.un0Fused) launch_un0_group(m, st, s);
             if (st.maxCellFaces > 4) {
                 k_flux_list<<<1024, 256, 0, s>>>(m, st, st.maxCellFaces);
                 if (m.triQuadFaces && st.fluxFan) k_flux_fan<<<4096, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
@@ -3330,10 +2972,6 @@ void launch_rho_phi(int nF, const double* ap, const double* phi, double rho1, do
 // taking a ticket, so each case's ticket counter still grows by its own
 // block count per launch.
 // ---------------------------------------------------------------------------
-__device__ inline const DevState& batch_view(const BatchCase& c, const BatchStepInfo& si, int swapped, int pass) {
-    return c.st[((si.aPar ^ swapped) << 1) | (si.hPar ^ (pass & 1))];
-}
-
 __global__ void __launch_bounds__(DETECT_LIST_THREADS) kb_detect_list(const BatchCase* __restrict__ bc,
                                                                       const BatchStepInfo* __restrict__ info,
                                                                       double tol) {
@@ -3349,15 +2987,6 @@ __global__ void __launch_bounds__(64, 1) kb_ls_normal(const BatchCase* __restric
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
     k_ls_normal_body(c.m, batch_view(c, si, 0, 0), nullptr, nullptr);
-}
-
-template <int G>
-__global__ void __launch_bounds__(64, SVP_FSD_WAVES) kb_fsd_group(const BatchCase* __restrict__ bc,
-                                                                  const BatchStepInfo* __restrict__ info) {
-    const BatchCase& c = bc[blockIdx.y];
-    const BatchStepInfo si = info[blockIdx.y];
-    if (!(si.dt > 0.0)) return;
-    k_fsd_group_body<G>(c.m, batch_view(c, si, 0, 0), nullptr, nullptr);
 }
 
 __global__ void __launch_bounds__(256) kb_upwind(const BatchCase* __restrict__ bc,
@@ -3466,9 +3095,7 @@ void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* inf
             kb_ls_normal<<<dim3(d.ls, n), 64, 0, s>>>(bc, info);
             break;
         case STAGE_FSD:
-            if (G == 4) kb_fsd_group<4><<<dim3(d.fsd, n), 64, 0, s>>>(bc, info);
-            else if (G == 6) kb_fsd_group<6><<<dim3(d.fsd, n), 64, 0, s>>>(bc, info);
-            else kb_fsd_group<8><<<dim3(d.fsd, n), 64, 0, s>>>(bc, info);
+            launch_batch_fsd_group(bc, info, n, d.fsd, G, s);
             break;
         case STAGE_UPWIND:
             kb_upwind<<<dim3(cdiv(maxF, 256), n), 256, 0, s>>>(bc, info);

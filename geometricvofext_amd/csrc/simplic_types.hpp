@@ -91,7 +91,8 @@ struct DevState {
     unsigned long long* detLook;  // per detection block: the same
     unsigned long long* detTicket;  // detection block tickets (grows by the block count per launch)
     unsigned long long* bndTicket;  // candidate-list block tickets (the same)
-    int un0Fused;       // plane placement by 8-lane groups, which also computes Un0
+    int placeGroup;     // lanes per cell of the plane placement: 4, 6, 8 or 32 (0: one lane per cell, split warped faces)
+    int un0Fused;       // the plane placement also computes Un0 (groups of 4, 6 and 8)
     int fluxFan;        // face flux with four lanes per face (most faces warped)
     int fsdKeep;        // 1: where findSignedDistance writes no d/C/S they keep their values (isoRDF)
     int gridRounds;     // bounding rounds run as grid-wide kernels before the one-workgroup tail
@@ -230,6 +231,10 @@ void launch_rdf_iteration(const DevMesh& m, const DevState& st, const Params& p,
 void launch_rdf_end(const DevMesh& m, const DevState& st, const RdfBufs& r, hipStream_t s);
 void launch_find_signed_distance(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s,
                                  const int* wl = nullptr, const int* wn = nullptr);
+// the lane-group plane placement (plane_kernels.hip)
+void launch_fsd_group(const DevMesh& m, const DevState& st, hipStream_t s, const int* wl, const int* wn);
+void launch_batch_fsd_group(const BatchCase* bc, const BatchStepInfo* info, int n, int x, int G, hipStream_t s);
+void launch_un0_group(const DevMesh& m, const DevState& st, hipStream_t s);
 // pipeline stages of one step, in launch order (also the profiler's slots)
 enum Stage : int {
     STAGE_DETECT = 0,

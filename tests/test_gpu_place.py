@@ -1,0 +1,89 @@
+"""Plane placement and interface velocity of every launch form, against the
+oracle: the lane groups per cell (4, 6, 8, 32) and, for each, interfaces on both
+sides of the counts at which the number of cells per wave changes."""
+import numpy as np
+import pytest
+
+from tests.helpers import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def merge_cells(mesh, group):
+    """The mesh whose cells are the groups of `mesh`'s cells (faces inside a
+    group dropped), internal faces in upper-triangular order."""
+    from geometricvofext_amd.mesh import PolyMesh
+    nif = mesh.n_internal_faces
+    faces = [mesh.face(f) for f in range(mesh.n_faces)]
+    own, nei, kept = [], [], []
+    for f in range(nif):
+        a, b = group[mesh.owner[f]], group[mesh.neighbour[f]]
+        if a == b:
+            continue
+        pts = faces[f] if a < b else np.concatenate([faces[f][:1], faces[f][:0:-1]])
+        kept.append((min(a, b), max(a, b), pts))
+    kept.sort(key=lambda e: (e[0], e[1]))
+    own = [e[0] for e in kept] + [group[c] for c in mesh.owner[nif:]]
+    nei = [e[1] for e in kept]
+    pts = [e[2] for e in kept] + faces[nif:]
+    offs = np.concatenate([[0], np.cumsum([len(p) for p in pts])]).astype(np.int32)
+    shift = len(kept) - nif
+    return PolyMesh(points=mesh.points, face_offsets=offs, face_points=np.concatenate(pts).astype(np.int32),
+                    owner=np.asarray(own, np.int32), neighbour=np.asarray(nei, np.int32), n_cells=int(max(group)) + 1,
+                    patch_names=mesh.patch_names, patch_start=np.asarray(mesh.patch_start) + shift,
+                    patch_size=mesh.patch_size, patch_type=mesh.patch_type, name=f"{mesh.name} merged")
+
+
+def merged_tets(N, perturb, seed):
+    """Cells of three face-connected Kuhn tetrahedra (8 triangular faces, 6 points)."""
+    import geometricvofext_amd as g
+    m = g.tet_box(N, perturb=perturb, seed=seed)
+    half = np.array([0, 0, 1, 1, 0, 1])
+    return merge_cells(m, 2 * (np.arange(m.n_cells) // 6) + half[np.arange(m.n_cells) % 6])
+
+
+def case_mesh(kind, N):
+    import geometricvofext_amd as g
+    if kind == "tet":
+        return g.tet_box(N, perturb=0.1, seed=N)
+    if kind == "merged":
+        return merged_tets(N, 0.1, N)
+    if kind == "refined":
+        return g.refined_hex_box(N)
+    return g.hex_box(N, perturb=0.25, seed=N)
+
+
+# mixed cells: a lone cell; a hexahedron takes 6 lane groups up to 1024 of them,
+# 3 up to 3072, 2 up to 5120, then 1 (past 40960 the workgroups loop); a
+# tetrahedron 2 up to 8192; merged cells 8 and 4 groups up to 1024 and 2048;
+# general polyhedra 2 groups up to 1024
+@pytest.mark.parametrize("kind,N,mixed", [("hex", 6, 1), ("hex", 10, 1000), ("hex", 11, 1331), ("hex", 16, 4096),
+                                          ("hex", 18, 5832), ("hex", 35, 42875), ("tet", 4, 384), ("tet", 12, 10368),
+                                          ("merged", 4, 128), ("merged", 9, 1458), ("merged", 12, 3456),
+                                          ("refined", 8, 900), ("refined", 10, None)])
+def test_place_every_split(oracle_lib, kind, N, mixed):
+    import geometricvofext_amd as g
+    print("place", kind, N, mixed, flush=True)
+    mesh = case_mesh(kind, N)
+    om = oracle_lib.OracleMesh(mesh)
+    rng = np.random.default_rng(N)
+    alpha = rng.uniform(0.0, 1.0, mesh.n_cells)
+    alpha[rng.integers(0, mesh.n_cells, mesh.n_cells // 8 + 1)] = rng.choice([2e-8, 1.0 - 2e-8, 0.5, 1e-3])
+    if mixed is not None and mixed < mesh.n_cells:
+        alpha[rng.permutation(mesh.n_cells)[mixed:]] = 0.0
+    U = rng.normal(size=(mesh.n_cells, 3))
+    phi = om.Sf @ np.array([0.3, -0.2, 0.1])
+    gpu = g.SolveVofEqu(mesh, dict(orientationMethod="LS", nAlphaBounds=1, clip=False))
+    ors = oracle_lib.OracleSolver(om, nAlphaBounds=1, clip=False, threads=8)
+    for s in (gpu, ors):
+        s.set_alpha(alpha)
+        s.set_flow(phi, U)
+        s.reconstruct()
+        s.advect(0.1 / mesh.n_cells)
+    gi, oi = gpu.interface(), ors.mixed()
+    for k in ("cells", "status", "faceclass", "ncutpts"):
+        assert np.array_equal(gi[k], oi[k]), k
+    for k in ("d", "C", "S"):
+        assert bits_equal(gi[k], oi[k]), k
+    assert bits_equal(gpu.un0(), oi["un0"])
+    gpu.synchronize()
