@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsimplic_amd.so")
-SOURCES = ["simplic_kernels.hip", "plane_kernels.hip", "harness_kernels.hip", "learned_kernels.hip", "simplic_api.cpp", "learned_api.cpp"]
+SOURCES = ["simplic_kernels.hip", "plane_kernels.hip", "flux_kernels.hip", "harness_kernels.hip", "learned_kernels.hip", "simplic_api.cpp", "learned_api.cpp"]
 HEADERS = ["simplic_device.hpp", "cut_device.hpp", "mesh_device.hpp", "simplic_types.hpp", "learned_device.hpp", "learned_kernels.hpp",
            "learned_model.hpp", "api_common.hpp"]
 

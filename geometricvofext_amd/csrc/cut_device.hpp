@@ -78,6 +78,15 @@ constexpr CutWalks make_cut_walks() {
 }
 static __device__ const CutWalks kCutWalks = make_cut_walks();
 
+// One of four values by index.  The values are arguments, so they are in
+// registers before the choice: a choice between elements of an array can
+// become a load through a chosen address, which moves the array to scratch.
+__device__ inline double pick4(double a, double b, double c, double d, int e) {
+    const double lo = (e & 1) ? b : a, hi = (e & 1) ? d : c;
+    return (e & 2) ? hi : lo;
+}
+__device__ inline double choose(bool c, double a, double b) { return c ? a : b; }
+
 __device__ inline V3 lds3(const double (&a)[3][64], int t) { return v3(a[0][t], a[1][t], a[2][t]); }
 __device__ inline void lds3_put(double (&a)[3][64], int t, V3 v) {
     a[0][t] = v.x;
@@ -130,9 +139,8 @@ struct FaceWalk {
     __device__ __attribute__((always_inline)) inline void listCrossing(const CutWalk& w, int k) const {
         const int e = (int)((w.info >> (8 + 2 * k)) & 3u);
         const int e1 = e + 1 == n ? 0 : e + 1;
-        const double dc = (e & 2) ? ((e & 1) ? d[3] : d[2]) : ((e & 1) ? d[1] : d[0]);
-        const double dn = (e1 & 2) ? ((e1 & 1) ? d[3] : d[2]) : ((e1 & 1) ? d[1] : d[0]);
-        lds3_put(ps[FP + k], t, crossPoint(e, e1, dc, dn));
+        lds3_put(ps[FP + k], t,
+                 crossPoint(e, e1, pick4(d[0], d[1], d[2], d[3], e), pick4(d[0], d[1], d[2], d[3], e1)));
     }
     __device__ inline V3 listEntry(const CutWalk& w, int k) const {
         const int c = (int)((w.codes >> (4 * k)) & 15u);
@@ -141,7 +149,7 @@ struct FaceWalk {
     __device__ inline double distOf(int e) const {
         double v = d[0];
 #pragma unroll
-        for (int k = 1; k < FP; ++k) v = e == k ? d[k] : v;
+        for (int k = 1; k < FP; ++k) v = choose(e == k, d[k], v);
         return v;
     }
     // the walk of a face of more than 4 points; record: its crossings to ps

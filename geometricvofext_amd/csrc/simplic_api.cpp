@@ -115,9 +115,9 @@ public:
         allocState();
         launch_geometry(m_, stream_);
         HIPCHECK(hipGetLastError());
-        // face flux with four lanes per face where most faces are warped
-        // (fan-integrated); SVP_FLUX_FAN=0/1 forces it off/on
-        if (m_.triQuadFaces && st_.un0Fused) {
+        // face flux with lanes for a face's fan triangles where most faces are
+        // warped; SVP_FLUX_FAN=0/1 forces it off/on
+        if (m_.triQuadFaces) {
             int nWarped = 0;
             launch_count_warped(m_, nonfinite_, stream_);
             HIPCHECK(hipMemcpyAsync(&nWarped, nonfinite_, sizeof(int), hipMemcpyDeviceToHost, stream_));
@@ -893,6 +893,9 @@ private:
         m_.triQuadFaces = 1;
         for (int f = 0; f < nF; ++f)
             if (fOff[f + 1] - fOff[f] > 4) m_.triQuadFaces = 0;
+        m_.facePoints = fOff[1];
+        for (int f = 0; f < nF; ++f)
+            if (fOff[f + 1] - fOff[f] != m_.facePoints) m_.facePoints = 0;
         // point interpolation sources: boundary points -> their non-empty
         // boundary faces (ascending); other points -> their cells (ascending)
         std::vector<std::vector<int>> bFaces(nP);
@@ -963,7 +966,7 @@ private:
         st_.ifS = dalloc<double>(3L * nC);
         st_.un0 = dalloc<double>(nC);
         st_.oobCount = dalloc<int>(OOB_SLOTS * OOB_STRIDE);
-        st_.fluxList = dalloc<int>(cellFaceEntries_);
+        st_.fluxList = dalloc<int2>(cellFaceEntries_);
         st_.fluxCount = dalloc<int>(1);
         st_.candCount = dalloc<int>(1);
         st_.candBits = dalloc<unsigned long long>((nC + 63) / 64);
@@ -1062,6 +1065,7 @@ public:
         G_ = f.batchGroup();
         MF_ = bound_faces(f.st_.maxCellFaces);
         triQuad_ = f.m_.triQuadFaces;
+        int nFan = 0;
         for (solveVofEqu* h : c_) {
             std::string why;
             if (h->device_ != device_) throw SvpError(SVP_E_ARG, "svp_batch_create: cases on different devices");
@@ -1075,6 +1079,17 @@ public:
                 throw SvpError(SVP_E_ARG, "svp_batch_create: the cases' cell types differ (hexahedra and "
                                           "tetrahedra go to separate batches)");
         }
+        // one kind of flux launch for all: each handles every mesh of the
+        // batch's cell type (triangles only, if all cases are)
+        bool listed = false;
+        for (solveVofEqu* h : c_) {
+            nFan += h->st_.fluxFan;
+            listed = listed || flux_listed(h->m_, h->st_.maxCellFaces);
+        }
+        fluxListed_ = listed;
+        DevMesh any = f.m_;
+        if (listed) any.facePoints = 0;
+        fluxKind_ = flux_kind(any, f.st_.maxCellFaces, 2 * nFan > n ? 1 : 0);
         HIPCHECK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
         // the cases' earlier work is done; from now on they use the batch's stream
         std::vector<BatchCase> host(n);
@@ -1191,7 +1206,7 @@ public:
 
     void launchStage(int sg) {
         launch_batch_stage(sg, (const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, size(), maxC_, maxF_,
-                           maxDet_, maxList_, dims_, params_, G_, MF_, triQuad_, stream_);
+                           maxDet_, maxList_, dims_, params_, G_, MF_, fluxKind_, fluxListed_, stream_);
     }
 
     void dropGraph() {
@@ -1356,6 +1371,8 @@ private:
     hipStream_t stream_ = nullptr;
     Params params_{};
     int G_ = 6, MF_ = NS_CELL_FACES, triQuad_ = 1;
+    int fluxKind_ = 0;
+    bool fluxListed_ = true;
     int maxC_ = 0, maxF_ = 0, maxDet_ = 0, maxList_ = 0;
     long maxN_ = 0;
     bool haveFlow_ = true;

@@ -1012,12 +1012,6 @@ __global__ void __launch_bounds__(64) k_find_signed_distance(DevMesh m, DevState
     }
 }
 
-// waves per SIMD the register allocation of the interface-flux kernels
-// targets (build-time tuning; results do not depend on it)
-#ifndef SVP_FLUX_WAVES
-#define SVP_FLUX_WAVES 1
-#endif
-
 // cells whose warped faces are split keep one lane per cell; all others take
 // a lane group per cell (plane_kernels.hip)
 void launch_find_signed_distance(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s,
@@ -1291,341 +1285,6 @@ __device__ inline V3 interpolate_u(const DevMesh& m, const DevState& st, V3 pos,
            bw[3] * point_u(m, st, bp[2]);
 }
 
-// cutFace::timeIntegratedArea (cutFace.C:392-506)
-__device__ inline double time_integrated_area(const V3* fPts, int n, V3 normal, double distance,
-                                              const double* pTimesIn, double Un0, double dt,
-                                              double magSf, bool& ok) {
-    double pt[MAX_FACE_POINTS];
-    for (int k = 0; k < n; ++k) pt[k] = pTimesIn[k];
-    for (int k = 1; k < n; ++k) {
-        const double v = pt[k];
-        int j = k - 1;
-        while (j >= 0 && pt[j] > v) {
-            pt[j + 1] = pt[j];
-            --j;
-        }
-        pt[j + 1] = v;
-    }
-    const double firstTime = pt[0], lastTime = pt[n - 1];
-    if (lastTime <= 0.0) return magSf * dt * pos0(Un0);
-    if (firstTime >= dt) return magSf * dt * (1.0 - pos0(Un0));
-    double tIntArea = 0.0;
-    double sortedTimes[MAX_FACE_POINTS + 2];
-    int nSorted = 0;
-    double prevTime;
-    double subAreaOld;
-    FaceCut fc;
-    if (firstTime > 0.0) {
-        subAreaOld = magSf * (1.0 - pos0(Un0));
-        tIntArea = subAreaOld * firstTime;
-        sortedTimes[nSorted++] = firstTime;
-        prevTime = firstTime;
-    } else {
-        sortedTimes[nSorted++] = 0.0;
-        prevTime = 0.0;
-        ok &= calcSubFace(fPts, n, normal, distance, fc);
-        subAreaOld = mag(fc.area);
-    }
-    const double smallTime = fmax(SVP_TSMALL / fabs(Un0), SVP_TSMALL);
-    for (int ti = 0; ti < n; ++ti) {
-        const double timeI = pt[ti];
-        if (timeI > (prevTime + smallTime) && timeI < dt) {
-            sortedTimes[nSorted++] = timeI;
-            prevTime = timeI;
-        }
-    }
-    if (lastTime > dt) sortedTimes[nSorted++] = dt;
-    else tIntArea += magSf * (dt - lastTime) * pos0(Un0);
-    for (int k = 0; k < nSorted - 1; k++) {
-        const double tauOld = sortedTimes[k], tauNew = sortedTimes[k + 1];
-        const double deltaTau = 0.5 * (tauNew - tauOld);
-        ok &= calcSubFace(fPts, n, normal, distance - tauNew * Un0, fc);
-        const double subAreaNew = mag(fc.area);
-        ok &= calcSubFace(fPts, n, normal, distance - (tauOld + deltaTau) * Un0, fc);
-        const double subAreaMid = mag(fc.area);
-        tIntArea += (deltaTau / 3.0) * (subAreaOld + 4.0 * subAreaMid + subAreaNew);
-        subAreaOld = subAreaNew;
-    }
-    return tIntArea;
-}
-
-// cutFace::timeIntegratedFaceFlux (cutFace.C:262-389)
-__device__ inline double time_integrated_face_flux(const DevMesh& m, int f, V3 normal, double distance,
-                                                   double Un0, double dt, double phi, double magSf,
-                                                   bool& ok) {
-    if (fabs(phi) <= SVP_TSMALL) return 0.0;
-    const int fs = m.fOff[f], n = m.fOff[f + 1] - fs;
-    V3 p[MAX_FACE_POINTS];
-    for (int k = 0; k < n; ++k) p[k] = ld3(m.pts, m.fPts[fs + k]);
-    const bool flat = m.flat[f] > (1.0 - SVP_TSMALL);
-    if (fabs(Un0 * dt) > SVP_TSMALL) {
-        double pTimes[MAX_FACE_POINTS];
-        for (int i = 0; i < n; ++i) {
-            const double t = (dot(p[i], normal) + distance) / Un0;
-            pTimes[i] = fabs(t) < SVP_TSMALL ? 0.0 : t;
-        }
-        if (flat) {
-            return phi / magSf * time_integrated_area(p, n, normal, distance, pTimes, Un0, dt, magSf, ok);
-        }
-        double dVf = 0.0;
-        V3 tri[3];
-        double tt[3];
-        tri[0] = ld3(m.Cf, f);
-        const double t0 = (dot(tri[0], normal) + distance) / Un0;
-        tt[0] = fabs(t0) < SVP_TSMALL ? 0.0 : t0;
-        for (int pi = 0; pi < n; ++pi) {
-            tri[1] = p[pi];
-            tt[1] = pTimes[pi];
-            tri[2] = p[(pi + 1) % n];
-            tt[2] = pTimes[(pi + 1) % n];
-            const double magSfTri = mag(triAreaNormal(tri[0], tri[1], tri[2]));
-            const double phiTri = phi * magSfTri / magSf;
-            dVf += phiTri / magSfTri *
-                   time_integrated_area(tri, 3, normal, distance, tt, Un0, dt, magSfTri, ok);
-        }
-        return dVf;
-    }
-    FaceCut fc;
-    if (flat) {
-        ok &= calcSubFace(p, n, normal, distance, fc);
-        const double alphaf = mag(fc.area) / magSf;
-        return (phi * dt * alphaf);
-    }
-    V3 tri[3];
-    tri[0] = ld3(m.Cf, f);
-    double dVf = 0.0;
-    for (int pi = 0; pi < n; ++pi) {
-        tri[1] = p[pi];
-        tri[2] = p[(pi + 1) % n];
-        const double magSfTri = mag(triAreaNormal(tri[0], tri[1], tri[2]));
-        const double phiTri = phi * magSfTri / magSf;
-        ok &= calcSubFace(tri, 3, normal, distance, fc);
-        const double alphafTri = mag(fc.area) / magSfTri;
-        dVf += (phiTri * dt * alphafTri);
-    }
-    return dVf;
-}
-
-// timeIntegratedArea for a face of N points in registers: the sorted arrival
-// times are walked once and every accepted sub-interval gets its Simpson term
-// right away; the additions to tIntArea keep the reference's order (leading
-// uncut segment, trailing uncut segment, then the Simpson terms in time order).
-// FULL: full points to the face's fully submerged sub-face (fullCS)
-template <int N, bool FULL = false>
-__device__ inline double tia_regs(const V3 (&P)[N], const double (&ptIn)[N], V3 normal, double distance,
-                                  double Un0, double dt, double magSf, bool& ok, const double* full = nullptr) {
-    // the plane normal is fixed over the time step: dot(point, n) once
-    double dots[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) dots[k] = dot(P[k], normal);
-    double pt[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) pt[k] = ptIn[k];
-    // ascending sort (values only): odd-even transposition, static indices
-#pragma unroll
-    for (int r = 0; r < N; ++r)
-#pragma unroll
-        for (int k = r & 1; k + 1 < N; k += 2) {
-            const double a = pt[k], b = pt[k + 1];
-            pt[k] = fmin(a, b);
-            pt[k + 1] = fmax(a, b);
-        }
-    const double firstTime = pt[0], lastTime = pt[N - 1];
-    if (lastTime <= 0.0) return magSf * dt * pos0(Un0);
-    if (firstTime >= dt) return magSf * dt * (1.0 - pos0(Un0));
-    double tIntArea = 0.0;
-    double prevTime, tauOld, subAreaOld;
-    FaceCut fc;
-    if (firstTime > 0.0) {
-        subAreaOld = magSf * (1.0 - pos0(Un0));
-        tIntArea = subAreaOld * firstTime;
-        prevTime = firstTime;
-        tauOld = firstTime;
-    } else {
-        prevTime = 0.0;
-        tauOld = 0.0;
-        ok &= calcSubFaceN<N, false, FULL, true>(P, normal, distance, fc, full, dots);
-        subAreaOld = mag(fc.area);
-    }
-    if (!(lastTime > dt)) tIntArea += magSf * (dt - lastTime) * pos0(Un0);
-    const double smallTime = fmax(SVP_TSMALL / fabs(Un0), SVP_TSMALL);
-    auto simpson = [&](double tauNew) {
-        const double deltaTau = 0.5 * (tauNew - tauOld);
-        ok &= calcSubFaceN<N, false, FULL, true>(P, normal, distance - tauNew * Un0, fc, full, dots);
-        const double subAreaNew = mag(fc.area);
-        ok &= calcSubFaceN<N, false, FULL, true>(P, normal, distance - (tauOld + deltaTau) * Un0, fc, full, dots);
-        const double subAreaMid = mag(fc.area);
-        tIntArea += (deltaTau / 3.0) * (subAreaOld + 4.0 * subAreaMid + subAreaNew);
-        subAreaOld = subAreaNew;
-        tauOld = tauNew;
-    };
-#pragma unroll
-    for (int ti = 0; ti < N; ++ti) {
-        const double timeI = pt[ti];
-        if (timeI > (prevTime + smallTime) && timeI < dt) {
-            simpson(timeI);
-            prevTime = timeI;
-        }
-    }
-    if (lastTime > dt) simpson(dt);
-    return tIntArea;
-}
-
-// timeIntegratedFaceFlux (cutFace.C:262-389) for a face of N points in registers
-template <int N>
-__device__ __attribute__((always_inline)) inline double tiff_regs(const DevMesh& m, int f, const V3 (&p)[N], V3 normal, double distance,
-                                   double Un0, double dt, double phi, double magSf, bool& ok) {
-    if (fabs(phi) <= SVP_TSMALL) return 0.0;
-    const bool flat = m.flat[f] > (1.0 - SVP_TSMALL);
-    if (fabs(Un0 * dt) > SVP_TSMALL) {
-        double pTimes[N];
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const double t = (dot(p[i], normal) + distance) / Un0;
-            pTimes[i] = fabs(t) < SVP_TSMALL ? 0.0 : t;
-        }
-        if (flat) return phi / magSf * tia_regs<N, true>(p, pTimes, normal, distance, Un0, dt, magSf, ok, &m.fullCS[6L * f]);
-        double dVf = 0.0;
-        const V3 fc = ld3(m.Cf, f);
-        const double t0 = (dot(fc, normal) + distance) / Un0;
-        const double tc = fabs(t0) < SVP_TSMALL ? 0.0 : t0;
-        // fan triangle pi uses points pi and pi+1: the arrays rotate one slot
-        // per triangle so that those are always slots 0 and 1
-        V3 rp[N];
-        double rt[N];
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            rp[i] = p[i];
-            rt[i] = pTimes[i];
-        }
-#pragma unroll 1
-        for (int pi = 0; pi < N; ++pi) {
-            const V3 tri[3] = {fc, rp[0], rp[1]};
-            const double tt[3] = {tc, rt[0], rt[1]};
-            rotate_left(rp, 1);
-            rotate_left(rt, 1);
-            const double magSfTri = mag(triAreaNormal(tri[0], tri[1], tri[2]));
-            const double phiTri = phi * magSfTri / magSf;
-            dVf += phiTri / magSfTri * tia_regs<3>(tri, tt, normal, distance, Un0, dt, magSfTri, ok);
-        }
-        return dVf;
-    }
-    FaceCut fcut;
-    if (flat) {
-        ok &= calcSubFaceN<N, false>(p, normal, distance, fcut);
-        const double alphaf = mag(fcut.area) / magSf;
-        return (phi * dt * alphaf);
-    }
-    const V3 fc = ld3(m.Cf, f);
-    double dVf = 0.0;
-#pragma unroll
-    for (int pi = 0; pi < N; ++pi) {
-        const V3 tri[3] = {fc, p[pi], p[(pi + 1) % N]};
-        const double magSfTri = mag(triAreaNormal(tri[0], tri[1], tri[2]));
-        const double phiTri = phi * magSfTri / magSf;
-        ok &= calcSubFaceN<3, false>(tri, normal, distance, fcut);
-        const double alphafTri = mag(fcut.area) / magSfTri;
-        dVf += (phiTri * dt * alphafTri);
-    }
-    return dVf;
-}
-
-// timeIntegratedFlux of the listed (cut cell, downwind face) pairs with four
-// lanes per face (faces of 3 or 4 points).  On a warped face, which the
-// reference integrates as the fan of triangles about the face centre
-// (cutFace.C:316-345 with a time step, 369-386 without), lane j integrates
-// triangle j (points j and j+1) and the group's first lane adds the
-// triangle volumes in fan order, the reference's sum; a flat face (one
-// timeIntegratedArea of the whole face) runs on the first lane alone.  Every
-// triangle's volume is the expression tiff_regs evaluates, so the face
-// volumes are identical to k_interface_flux_faces.
-constexpr int FAN_LANES = 4;
-
-__device__ __attribute__((always_inline)) inline void k_flux_fan_body(const DevMesh& m, const DevState& st, double dtStep, int slots) {
-    const long nWork = (long)*st.fluxCount;
-    const int lane = threadIdx.x & 63, j = lane & (FAN_LANES - 1), base = lane & ~(FAN_LANES - 1);
-    constexpr int PER_WAVE = 64 / FAN_LANES;
-    // one wave per workgroup; the loop bound is uniform across the wave, so
-    // every lane reaches the shuffles
-    for (long w0 = (long)blockIdx.x * PER_WAVE; w0 < nWork; w0 += (long)gridDim.x * PER_WAVE) {
-        const long wi = w0 + lane / FAN_LANES;
-        const bool live = wi < nWork;
-        int f = 0, i = 0, fsz = 3, s0 = 0;
-        double ph = 0.0;
-        if (live) {
-            const int w = st.fluxList[wi];
-            i = w / slots;
-            const int k = w % slots;
-            f = m.cFaces[m.cOff[st.mixed[i]] + k];
-            ph = st.phi[f];
-            s0 = m.fOff[f];
-            fsz = m.fOff[f + 1] - s0;
-        }
-        const double dt = dtStep;
-        const bool zero = !live || fabs(ph) <= SVP_TSMALL;
-        const bool flat = live && m.flat[f] > (1.0 - SVP_TSMALL);
-        const bool fan = !zero && !flat;
-        double term = 0.0;
-        bool ok = true;
-        if (!zero) {
-            const V3 n = ld3(st.ifN, i);
-            const double d = st.ifD[i], Un0 = st.un0[i];
-            const double magSf = m.magSf[f];
-            if (fan && j < fsz) {
-                const V3 fc = ld3(m.Cf, f);
-                const V3 pa = ld3(m.pts, m.fPts[s0 + j]);
-                const V3 pb = ld3(m.pts, m.fPts[s0 + (j + 1 == fsz ? 0 : j + 1)]);
-                const V3 tri[3] = {fc, pa, pb};
-                const double magSfTri = mag(triAreaNormal(tri[0], tri[1], tri[2]));
-                const double phiTri = ph * magSfTri / magSf;
-                if (fabs(Un0 * dt) > SVP_TSMALL) {
-                    auto arrival = [&](V3 q) {
-                        const double t = (dot(q, n) + d) / Un0;
-                        return fabs(t) < SVP_TSMALL ? 0.0 : t;
-                    };
-                    const double tt[3] = {arrival(fc), arrival(pa), arrival(pb)};
-                    term = phiTri / magSfTri * tia_regs<3>(tri, tt, n, d, Un0, dt, magSfTri, ok);
-                } else {
-                    FaceCut fcut;
-                    ok &= calcSubFaceN<3, false>(tri, n, d, fcut);
-                    const double alphafTri = mag(fcut.area) / magSfTri;
-                    term = (phiTri * dt * alphafTri);
-                }
-            } else if (!fan && j == 0) {
-                if (fsz == 4) {
-                    V3 p[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) p[q] = ld3(m.pts, m.fPts[s0 + q]);
-                    term = tiff_regs<4>(m, f, p, n, d, Un0, dt, ph, magSf, ok);
-                } else {
-                    V3 p[3];
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) p[q] = ld3(m.pts, m.fPts[s0 + q]);
-                    term = tiff_regs<3>(m, f, p, n, d, Un0, dt, ph, magSf, ok);
-                }
-            }
-        }
-        double v = term;
-        if (fan) {
-            v = 0.0;
-#pragma unroll
-            for (int t = 0; t < FAN_LANES; ++t) {
-                const double x = __shfl(term, base + t);
-                if (t < fsz) v += x;
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < FAN_LANES; ++t) (void)__shfl(term, base + t);
-        }
-        if (live && j == 0) st.dVf[f] = zero ? 0.0 : v;
-        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
-    }
-}
-
-__global__ void __launch_bounds__(64, SVP_FLUX_WAVES) k_flux_fan(DevMesh m, DevState st, double dtStep, int slots) {
-    k_flux_fan_body(m, st, dtStep, slots);
-}
-
 // faces whose flatness is below 1 - tSmall (the fan-integrated ones)
 __global__ void __launch_bounds__(256) k_count_warped(DevMesh m, int* count) {
     const int f = blockIdx.x * 256 + threadIdx.x;
@@ -1653,8 +1312,8 @@ __global__ void __launch_bounds__(64) k_un0(DevMesh m, DevState st) {
     }
 }
 
-// The (cut cell, cell face) pairs whose face is downwind of the cell, packed
-// as i * slots + k: about half of a cut cell's faces, so the flux kernel
+// The (mixed-list position, face) pairs of the cut cells' downwind faces:
+// about half of a cut cell's faces, so the flux kernel
 // below runs on full waves.  Block-aggregated appends (the order does not
 // matter: each face is downwind of one cell and gets one volume), one atomic
 // per block and round (a single counter serialises its atomics).  The count
@@ -1677,6 +1336,7 @@ __device__ __attribute__((always_inline)) inline void k_flux_list_body(const Dev
     for (long b0 = (long)blockIdx.x * blockDim.x; b0 < total; b0 += stride) {
         const long w = b0 + threadIdx.x;
         bool take = false;
+        int2 entry = make_int2(0, 0);
         if (w < total) {
             // the pair's cell, face and the face's cells loaded once (the
             // needBounding tags are stores, after which reloads would wait)
@@ -1686,6 +1346,7 @@ __device__ __attribute__((always_inline)) inline void k_flux_list_body(const Dev
             const int fb = m.cOff[c], nf = m.cOff[c + 1] - fb;
             if (k < nf) {
                 const int f = m.cFaces[fb + k];
+                entry = make_int2(i, f);
                 const int fo = m.own[f];
                 const int fn = f < m.nIF ? m.nbr[f] : -1;
                 const double ph = st.phi[f];
@@ -1710,76 +1371,13 @@ __device__ __attribute__((always_inline)) inline void k_flux_list_body(const Dev
         __syncthreads();
         int pre = sBase;
         for (int k = 0; k < wave; ++k) pre += wcnt[k];
-        if (take) st.fluxList[pre + __popcll(bal & ((1ull << lane) - 1ull))] = (int)w;
+        if (take) st.fluxList[pre + __popcll(bal & ((1ull << lane) - 1ull))] = entry;
         __syncthreads();
     }
 }
 
 __global__ void __launch_bounds__(256) k_flux_list(DevMesh m, DevState st, int slots) {
     k_flux_list_body(m, st, slots, st.epoch);
-}
-
-// timeIntegratedFlux with one thread per (cut cell, downwind face): each
-// downwind face's volume is independent of the others.  LISTED takes the
-// pairs from the work list; otherwise every (cut cell, face slot) pair is a
-// thread and the upwind faces drop out (cheaper for tetrahedra, whose light
-// faces do not repay the list).
-template <bool TRIQUAD, bool LISTED>
-__device__ __attribute__((always_inline)) inline void k_interface_flux_faces_body(const DevMesh& m, const DevState& st, double dtStep, int slots,
-                                                                                  int epoch) {
-    const long nWork = LISTED ? (long)*st.fluxCount : (long)*st.nMixed * slots;
-    for (long wi = (long)blockIdx.x * blockDim.x + threadIdx.x; wi < nWork; wi += (long)gridDim.x * blockDim.x) {
-        const int w = LISTED ? st.fluxList[wi] : (int)wi;
-        const int i = w / slots, k = w % slots;
-        // the pair's cell and face loaded once, before the needBounding
-        // stores (after which reloads of them would wait)
-        const int c = st.mixed[i];
-        const int fb = m.cOff[c];
-        if (!LISTED && k >= m.cOff[c + 1] - fb) continue;
-        const double dt = dtStep;
-        const int f = m.cFaces[fb + k];
-        const double ph = st.phi[f];
-        if (!LISTED) {
-            const int status = st.status[i];
-            const int fo = m.own[f];
-            const int fn = f < m.nIF ? m.nbr[f] : -1;
-            const unsigned char em = m.fEmpty[empty_slot(m, f)];
-            // needBounding: the cell (slot 0) and its neighbour across each
-            // internal face, for every status
-            if (k == 0) st.nbTag[c] = epoch;
-            if (f < m.nIF) st.nbTag[fo == c ? fn : fo] = epoch;
-            if (status != 0) continue;
-            bool down;
-            if (f < m.nIF) down = (fo == c) ? (ph >= 0.0) : (ph < 0.0);
-            else down = !em && (ph >= 0.0);
-            if (!down) continue;
-        }
-        const V3 n = ld3(st.ifN, i);
-        const double d = st.ifD[i], Un0 = st.un0[i];
-        const int s0 = m.fOff[f], fsz = m.fOff[f + 1] - s0;
-        bool ok = true;
-        double v;
-        if (fsz == 4) {
-            V3 p[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) p[q] = ld3(m.pts, m.fPts[s0 + q]);
-            v = tiff_regs<4>(m, f, p, n, d, Un0, dt, ph, m.magSf[f], ok);
-        } else if (TRIQUAD || fsz == 3) {
-            V3 p[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) p[q] = ld3(m.pts, m.fPts[s0 + q]);
-            v = tiff_regs<3>(m, f, p, n, d, Un0, dt, ph, m.magSf[f], ok);
-        } else {
-            v = time_integrated_face_flux(m, f, n, d, Un0, dt, ph, m.magSf[f], ok);
-        }
-        st.dVf[f] = v;
-        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
-    }
-}
-
-template <bool TRIQUAD, bool LISTED>
-__global__ void __launch_bounds__(64, SVP_FLUX_WAVES) k_interface_flux_faces(DevMesh m, DevState st, double dtStep, int slots) {
-    k_interface_flux_faces_body<TRIQUAD, LISTED>(m, st, dtStep, slots, st.epoch);
 }
 
 __device__ inline bool loop_oob(double a, double aTol) { return (a - 1.0 > aTol) || (a < -aTol); }
@@ -2910,15 +2508,8 @@ void launch_advect_stage(int stage, const DevMesh& m, const DevState& st, const 
         case STAGE_IFLUX:
             if (!st.placeGroup) k_un0<<<512, 64, 0, s>>>(m, st);
             else if (!st.un0Fused) launch_un0_group(m, st, s);
-            if (st.maxCellFaces > 4) {
-                k_flux_list<<<1024, 256, 0, s>>>(m, st, st.maxCellFaces);
-                if (m.triQuadFaces && st.fluxFan) k_flux_fan<<<4096, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
-                else if (m.triQuadFaces) k_interface_flux_faces<true, true><<<2048, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
-                else k_interface_flux_faces<false, true><<<2048, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
-            } else {
-                if (m.triQuadFaces) k_interface_flux_faces<true, false><<<2048, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
-                else k_interface_flux_faces<false, false><<<2048, 64, 0, s>>>(m, st, dt, st.maxCellFaces);
-            }
+            if (flux_listed(m, st.maxCellFaces)) k_flux_list<<<1024, 256, 0, s>>>(m, st, st.maxCellFaces);
+            launch_interface_flux(m, st, dt, s);
             break;
         case STAGE_UPDATE:
             launch_update(m, st, dt, Sp, Su, s);
@@ -3006,16 +2597,6 @@ __global__ void __launch_bounds__(256) kb_flux_list(const BatchCase* __restrict_
     k_flux_list_body(c.m, st, st.maxCellFaces, si.epoch);
 }
 
-template <bool TRIQUAD, bool LISTED>
-__global__ void __launch_bounds__(64, SVP_FLUX_WAVES) kb_interface_flux_faces(const BatchCase* __restrict__ bc,
-                                                                              const BatchStepInfo* __restrict__ info) {
-    const BatchCase& c = bc[blockIdx.y];
-    const BatchStepInfo si = info[blockIdx.y];
-    if (!(si.dt > 0.0)) return;
-    const DevState& st = batch_view(c, si, 1, 0);
-    k_interface_flux_faces_body<TRIQUAD, LISTED>(c.m, st, si.dt, st.maxCellFaces, si.epoch);
-}
-
 template <int MF>
 __global__ void __launch_bounds__(UPDATE_BLOCK) kb_update(const BatchCase* __restrict__ bc,
                                                           const BatchStepInfo* __restrict__ info) {
@@ -3086,7 +2667,7 @@ static void launch_batch_bound(const BatchCase* bc, const BatchStepInfo* info, i
 
 void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* info, int n, int maxC, int maxF,
                         int maxDetBlocks, int maxListBlocks, const BatchDims& d, const Params& p, int G, int MF,
-                        int triQuad, hipStream_t s) {
+                        int fluxKind, bool fluxListed, hipStream_t s) {
     switch (stage) {
         case STAGE_DETECT:
             kb_detect_list<<<dim3(maxDetBlocks, n), DETECT_LIST_THREADS, 0, s>>>(bc, info, p.mixedCellTol);
@@ -3101,14 +2682,8 @@ void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* inf
             kb_upwind<<<dim3(cdiv(maxF, 256), n), 256, 0, s>>>(bc, info);
             break;
         case STAGE_IFLUX:
-            if (G > 4) {
-                kb_flux_list<<<dim3(d.fluxList, n), 256, 0, s>>>(bc, info);
-                if (triQuad) kb_interface_flux_faces<true, true><<<dim3(d.fluxFaces, n), 64, 0, s>>>(bc, info);
-                else kb_interface_flux_faces<false, true><<<dim3(d.fluxFaces, n), 64, 0, s>>>(bc, info);
-            } else {
-                if (triQuad) kb_interface_flux_faces<true, false><<<dim3(d.fluxFaces, n), 64, 0, s>>>(bc, info);
-                else kb_interface_flux_faces<false, false><<<dim3(d.fluxFaces, n), 64, 0, s>>>(bc, info);
-            }
+            if (fluxListed) kb_flux_list<<<dim3(d.fluxList, n), 256, 0, s>>>(bc, info);
+            launch_batch_interface_flux(bc, info, n, d.fluxFaces, fluxKind, s);
             break;
         case STAGE_UPDATE:
             // MF: the bounding slots of the largest cell (4, 6, 8 or 24)

@@ -27,6 +27,7 @@ struct DevMesh {
     const int* cPts;
     int maxCellPoints;
     int triQuadFaces;       // 1 when every face has 3 or 4 points
+    int facePoints;         // points of every face when all have the same number, else 0
     // cell-point-cell stencil: the cell first, then the other cells ascending
     const int* stOff;
     const int* st;
@@ -72,7 +73,7 @@ struct DevState {
     double* un0;
     // bounding bookkeeping (limitFlux/boundFlux)
     int* oobCount;      // cells with alpha-1 > aTol or alpha < -aTol, spread over OOB_SLOTS counters
-    int* fluxList;      // (cut cell, downwind face) pairs of the interface flux, cell-face CSR size
+    int2* fluxList;     // (mixed-list position, downwind face) pairs of the interface flux, cell-face CSR size
     int* fluxCount;     // [1]
     int* candCount;     // [1] candidates of the last pass (diagnostics)
     unsigned long long* candBits;  // nC bits: alpha outside [-aTol,1+aTol] and needBounding
@@ -93,7 +94,7 @@ struct DevState {
     unsigned long long* bndTicket;  // candidate-list block tickets (the same)
     int placeGroup;     // lanes per cell of the plane placement: 4, 6, 8 or 32 (0: one lane per cell, split warped faces)
     int un0Fused;       // the plane placement also computes Un0 (groups of 4, 6 and 8)
-    int fluxFan;        // face flux with four lanes per face (most faces warped)
+    int fluxFan;        // face flux with lanes for four fan triangles per face (most faces warped)
     int fsdKeep;        // 1: where findSignedDistance writes no d/C/S they keep their values (isoRDF)
     int gridRounds;     // bounding rounds run as grid-wide kernels before the one-workgroup tail
     int bndGrid;        // workgroups of the grid-stride bounding kernels
@@ -235,6 +236,13 @@ void launch_find_signed_distance(const DevMesh& m, const DevState& st, const Par
 void launch_fsd_group(const DevMesh& m, const DevState& st, hipStream_t s, const int* wl, const int* wn);
 void launch_batch_fsd_group(const BatchCase* bc, const BatchStepInfo* info, int n, int x, int G, hipStream_t s);
 void launch_un0_group(const DevMesh& m, const DevState& st, hipStream_t s);
+// interface face volumes (flux_kernels.hip): the kind of launch a mesh takes
+// (lanes per face) and whether it reads the work list
+int flux_kind(const DevMesh& m, int maxCellFaces, int fluxFan);
+bool flux_listed(const DevMesh& m, int maxCellFaces);
+void launch_interface_flux(const DevMesh& m, const DevState& st, double dt, hipStream_t s);
+void launch_batch_interface_flux(const BatchCase* bc, const BatchStepInfo* info, int n, int x, int kind,
+                                 hipStream_t s);
 // pipeline stages of one step, in launch order (also the profiler's slots)
 enum Stage : int {
     STAGE_DETECT = 0,
@@ -280,7 +288,7 @@ DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
 // size shared by all cases
 void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC, int maxF,
                         int maxDetBlocks, int maxListBlocks, const BatchDims& d, const Params& p, int G, int MF,
-                        int triQuad, hipStream_t s);
+                        int fluxKind, bool fluxListed, hipStream_t s);
 void launch_batch_courant(const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC,
                           unsigned long long* out, hipStream_t s);
 void launch_batch_scale_flow(const BatchCase* bc, const BatchStepInfo* info, const double* factors, int nCases,
