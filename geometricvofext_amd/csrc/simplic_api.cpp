@@ -981,8 +981,6 @@ private:
             throw SvpError(SVP_E_UNSUPPORTED, "mesh too large for 31-bit bounding order keys");
         st_.corrPos = dalloc<int>(2L * nF);
         HIPCHECK(hipMemsetAsync(st_.corrPos, 0xFF, sizeof(int) * 2 * nF, stream_));
-        st_.touched = dalloc<int>(nC);
-        st_.touchedFlag = dalloc<int>(nC);
         st_.boundStats = dalloc<int>(4 * MAX_BOUND_PASSES);
         st_.boundTotals = dalloc<unsigned long long>(5);
         st_.bcount = dalloc<int>(32);

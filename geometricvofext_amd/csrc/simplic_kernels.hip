@@ -6,6 +6,7 @@
 // (compiled with -ffp-contract=off); each kernel cites the reference lines it
 // follows.  Control flow that the reference runs on the host (mixed-cell count,
 // bounding passes) stays on the device, so a step never waits for the host.
+#include "cut_device.hpp"
 #include "mesh_device.hpp"
 
 namespace svp {
@@ -1519,15 +1520,15 @@ __device__ inline bool face_downwind_of(const DevMesh& m, const double* phi, int
 //   prep              every candidate's first redistribution loop, which
 //                     decides whether it writes corrections and which faces
 //                     open correctedFaces; the record of each writing cell
+//                     and the order keys of those faces
 //   flow              all remaining boundFlux work in dependency order in
-//                     one launch, and the correctedFaces order keys and
-//                     touched cells (the default), or
+//                     one launch (the default), or
 //   scatter/round/tail  the same as Kahn rounds: grid-wide kernels, then the
 //                     remaining rounds inside one workgroup
 //   apply             corrections applied per cell in correctedFaces order,
 //                     dVf of the corrected faces, bitmap and bound count,
 //                     pass statistics
-// bcount: [0] candidates, [1] corrected faces (prep), [2] touched cells,
+// bcount: [0] candidates, [1] corrected faces (prep),
 // [3+r] frontier size of round r (r <= st.gridRounds; [3] = active cells of
 // the dataflow pass), [BND_CTRL-1] rounds, then the dataflow ticket and
 // completion count.
@@ -1540,6 +1541,19 @@ static_assert(BND_PROGRESS < 16, "bcount holds 16 counters");
 // correction of a face whose writer has not completed yet in the dataflow
 // pass: a NaN payload that no arithmetic produces (stored and compared as bits)
 constexpr unsigned long long CORR_PENDING = 0x7FF4D00DF00DD00Dull;
+
+// x / V > aTol for x >= 0 (aTol and V fixed for a cell) without dividing: x
+// outside the band of a few rounding errors about V aTol is decided by a
+// comparison, inside it (or for a volume outside the range where the band's
+// ends are exact to that) by the quotient itself.
+struct OverTol {
+    double lo, hi;
+};
+__device__ inline OverTol over_tol(double V, double aTol) {
+    const double thr = V * aTol;
+    const bool plain = V > 1e-250 && V < 1e250;
+    return OverTol{plain ? thr * (1.0 - 1e-15) : -1.0, plain ? thr * (1.0 + 1e-15) : __builtin_inf()};
+}
 
 // Record of candidate c for the dependent part of the pass, with iteration 0
 // of boundFlux's redistribution loop (advectionTemplates.C:260-330) already
@@ -1563,10 +1577,9 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
     if (fabs(alphaOvershoot) < aTol) return 0;
     const double fluidToPassOn = alphaOvershoot * Vi;
     int fid[MF], oth[MF];
-    double phf[MF], dvf[MF], smax[MF];
+    double phdt[MF], dvf[MF], smax[MF];
     unsigned int flg[(MF + 7) / 8];
     unsigned int first = 0u;
-    int n = 0;
     double dVftot = 0.0;
 #pragma unroll
     for (int w = 0; w < (MF + 7) / 8; ++w) flg[w] = 0u;
@@ -1587,10 +1600,12 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
         fem[k] = m.fEmpty[empty_slot(m, f)];
     }
     __builtin_amdgcn_sched_barrier(0);
+    const OverTol tol = over_tol(Vi, aTol);
+    bool near = false;
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
         oth[k] = -1;
-        phf[k] = 0.0;
+        phdt[k] = 0.0;
         dvf[k] = 0.0;
         smax[k] = 0.0;
         if (k < nf) {
@@ -1601,7 +1616,7 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
             const bool live = (f < m.nIF) || !fem[k];
             const double ph = live ? fph[k] : 0.0;
             const double dv = live ? fdv[k] : 0.0;
-            phf[k] = ph;
+            phdt[k] = ph * dt + 0.0;   // (never -0: its sign bit is sgn(phi))
             dvf[k] = dv;
             const bool down = own ? (ph >= 0) : (ph < 0);
             const bool writable = live;
@@ -1610,28 +1625,35 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
                            << (4 * (k & 7));
             if (down) {
                 const double dVff = dv + 0.0;
-                const double maxExtra = fabs(pos0(fluidToPassOn) * ph * dt - dVff);
-                if (maxExtra / Vi > aTol) {
-                    first |= 1u << k;
-                    n++;
-                    smax[k] = maxExtra;
-                    dVftot += fabs(ph * dt);
-                }
+                smax[k] = fabs((fluidToPassOn >= 0.0 ? phdt[k] : 0.0) - dVff);
+                if (smax[k] > tol.hi) first |= 1u << k;
+                near |= !(smax[k] > tol.hi) && !(smax[k] < tol.lo);
             }
         }
     }
+    if (near) {
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            const bool down = (flg[k >> 3] >> (4 * (k & 7))) & 2u;
+            if (k < nf && down) first = (first & ~(1u << k)) | (smax[k] / Vi > aTol ? 1u << k : 0u);
+        }
+    }
+    const int n = __popc(first);
     if (n == 0) return 0;
+#pragma unroll
+    for (int k = 0; k < MF; ++k)
+        if ((first >> k) & 1u) dVftot += fabs(phdt[k]);
     auto bits = [&](int k) { return flg[k >> 3] >> (4 * (k & 7)); };
     int nFaces = 0;
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
         R.cor0[k] = 0.0;
         if (!((first >> k) & 1u)) continue;
-        double fl = fabs(fluidToPassOn) * fabs(phf[k] * dt) / dVftot;
-        nFaces += (int)pos0(smax[k] - fl);
+        double fl = fabs(fluidToPassOn) * fabs(phdt[k]) / dVftot;
+        nFaces += smax[k] >= fl ? 1 : 0;
         fl = fmin(fl, smax[k]);
         double dVff = 0.0;
-        dVff += sgn(phf[k]) * sgn(fluidToPassOn) * fl;
+        dVff += sgn(phdt[k]) * sgn(fluidToPassOn) * fl;
         if (bits(k) & 4u) R.cor0[k] = dVff;
     }
     double nfd = 0.0;
@@ -1647,7 +1669,7 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
     for (int k = 0; k < MF; ++k) {
         R.fid[k] = fid[k];
         R.oth[k] = oth[k];
-        R.phf[k] = phf[k];
+        R.phdt[k] = phdt[k];
         R.dvf[k] = dvf[k];
         if (k < nf && (bits(k) & 6u) == 6u) st.corr[fid[k]] = __longlong_as_double((long long)CORR_PENDING);
     }
@@ -1660,78 +1682,144 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
     return n;
 }
 
-// boundFlux of one cell (advectionTemplates.C:243-347) from iteration 0 of
-// its record on: cin[k] is the correction of face slot k written by its
-// lower-numbered upwind neighbour (0 where the flags mark no such writer; a
-// higher-numbered writer has not run yet in the reference's ascending walk,
-// so it contributes zero); out(k, f, v) stores the final correction of
-// downwind face f in slot k.
-template <int MF, class Out>
-__device__ inline void bound_finish(const BndRec<MF>& R, const double (&cin)[MF], double dt, double rDeltaT,
-                                    Out out) {
-    const double aTol = 100.0 * SVP_SMALL;
-    unsigned int flg[(MF + 7) / 8];
-#pragma unroll
-    for (int w = 0; w < (MF + 7) / 8; ++w) flg[w] = R.flg[w];
-    const int nf = R.nf;
-    const double Vi = R.Vi;
-    auto bits = [&](int k) { return flg[k >> 3] >> (4 * (k & 7)); };
-    auto isOwn = [&](int k) { return (bits(k) & 1u) != 0u; };
-    auto down = [&](int k) { return (bits(k) & 2u) != 0u; };
-    auto writable = [&](int k) { return (bits(k) & 4u) != 0u; };
-    double phf[MF], cor[MF];
+// What the rest of boundFlux takes from a cell's record: formed once, before
+// the cell's corrections arrive.
+template <int MF>
+struct BndDiv {
+    Rcp V, den;
+    OverTol tol;
+    double rDeltaT;
+    bool down[MF], writes[MF];   // faces that can take fluid, faces written
+    unsigned flip[MF];           // sign bit of a face's share of the flux sum (neighbour faces subtract)
+    // divisors and flux volumes within the range of the shared reciprocals
+    bool plain, plainFlux;
+};
+template <int MF>
+__device__ __attribute__((always_inline)) inline BndDiv<MF> bound_divisors(const BndRec<MF>& R, double rDeltaT) {
+    BndDiv<MF> D;
+    D.V = rcp_of(R.Vi);
+    D.den = rcp_of(R.den);
+    D.tol = over_tol(R.Vi, 100.0 * SVP_SMALL);
+    D.rDeltaT = rDeltaT;
+    D.plain = fabs(R.Vi) > 1e-250 && fabs(R.Vi) < 1e250 && fabs(R.den) > 1e-250 && fabs(R.den) < 1e250;
+    D.plainFlux = true;
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
-        phf[k] = R.phf[k];
-        cor[k] = down(k) ? R.cor0[k] : cin[k];
+        const unsigned bits = R.flg[k >> 3] >> (4 * (k & 7));
+        D.down[k] = k < R.nf && (bits & 2u);
+        D.writes[k] = D.down[k] && (bits & 4u);
+        D.flip[k] = (bits & 1u) ? 0u : 0x80000000u;
+        const double x = fabs(R.phdt[k]);
+        D.plainFlux &= x == 0.0 || (x > 1e-140 && x < 1e140);
     }
-    double alphaOvershoot = 0.0, fluidToPassOn = 0.0;
-    auto settle = [&]() {
+    return D;
+}
+// x with its sign bit changed where f has it
+__device__ inline double flip_sign(double x, unsigned f) {
+    return __hiloint2double((int)((unsigned)__double2hiint(x) ^ f), __double2loint(x));
+}
+
+// boundFlux of one cell (advectionTemplates.C:243-347) from iteration 0 of
+// its record on, one redistribution loop at a time: start() with the
+// corrections its lower-numbered upwind neighbours wrote (cin[k], 0 where the
+// flags mark no such writer; a higher-numbered writer has not run yet in the
+// reference's ascending walk, so it contributes zero), then settle(), and
+// share() + settle() until settled(); publish() gives out(k, f, v), the final
+// correction of downwind face f in slot k.
+//
+// A level of the dependent pass costs this routine's instructions, whatever
+// the number of cells on it, so it divides once where the reference divides
+// per face: the test against aTol compares (OverTol), the shares of one loop
+// have one divisor, and the new alpha's two divisors are the cell's.  Where a
+// shared reciprocal could differ from '/' (a numerator below 1e-290) the new
+// alpha is within aTol of 0 and ends the loop either way; values out of the
+// reciprocals' range and non-finite results are formed by '/'.
+template <int MF>
+struct BndSolve {
+    double cor[MF];
+    double overshoot, fluid;
+    bool open;   // a face can still take fluid
+
+    __device__ __attribute__((always_inline)) inline void start(const BndRec<MF>& R, const BndDiv<MF>& D,
+                                                                const double (&cin)[MF]) {
+#pragma unroll
+        for (int k = 0; k < MF; ++k) cor[k] = R.cor0[k] + cin[k];   // (one of the two is 0)
+        open = R.nFaces0 != 0;
+    }
+    __device__ __attribute__((always_inline)) inline void settle(const BndRec<MF>& R, const BndDiv<MF>& D) {
         double nfc = 0.0;
 #pragma unroll
-        for (int k = 0; k < MF; ++k)
-            if (k < nf) nfc = isOwn(k) ? nfc + cor[k] : nfc - cor[k];
-        const double alpha1New = (R.num0 - nfc / Vi * rDeltaT) / R.den;
-        alphaOvershoot = pos0(alpha1New - 1.0) * (alpha1New - 1.0) + neg0(alpha1New) * alpha1New;
-        fluidToPassOn = alphaOvershoot * Vi;
-    };
-    settle();
-    int nFaces = R.nFaces0;
-    for (int iter = 1; iter < 10; iter++) {
-        if (fabs(alphaOvershoot) < aTol || nFaces == 0) break;
-        bool sel[MF];
-        double smax[MF];
-        double dVftot = 0.0;
-        nFaces = 0;
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            sel[k] = false;
-            smax[k] = 0.0;
-            if (k < nf && down(k)) {
-                const double dVff = R.dvf[k] + cor[k];
-                const double maxExtra = fabs(pos0(fluidToPassOn) * phf[k] * dt - dVff);
-                if (maxExtra / Vi > aTol) {
-                    sel[k] = true;
-                    smax[k] = maxExtra;
-                    dVftot += fabs(phf[k] * dt);
-                }
-            }
+        for (int k = 0; k < MF; ++k) nfc += flip_sign(cor[k], D.flip[k]);
+        double a = div_by(R.num0 - div_by(nfc, D.V) * D.rDeltaT, D.den);
+        // pos0(a - 1) (a - 1) + neg0(a) a
+        overshoot = a >= 1.0 ? a - 1.0 : (a <= 0.0 ? a : 0.0);
+        if (!D.plain || !(fabs(a) < 1e300)) {
+            a = (R.num0 - nfc / R.Vi * D.rDeltaT) / R.den;
+            overshoot = pos0(a - 1.0) * (a - 1.0) + neg0(a) * a;
         }
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            if (!sel[k]) continue;
-            double fl = fabs(fluidToPassOn) * fabs(phf[k] * dt) / dVftot;
-            nFaces += (int)pos0(smax[k] - fl);
-            fl = fmin(fl, smax[k]);
-            double dVff = cor[k];
-            dVff += sgn(phf[k]) * sgn(fluidToPassOn) * fl;
-            if (writable(k)) cor[k] = dVff;
-        }
-        settle();
+        fluid = overshoot * R.Vi;
     }
+    // nothing is left to pass on, or no face can take it
+    __device__ inline bool settled() const { return fabs(overshoot) < 100.0 * SVP_SMALL || !open; }
+    // one redistribution loop (advectionTemplates.C:260-330)
+    __device__ __attribute__((always_inline)) inline void share(const BndRec<MF>& R, const BndDiv<MF>& D) {
+        const double aTol = 100.0 * SVP_SMALL;
+        const double over = pos0(fluid);
+        double smax[MF], dVftot = 0.0;
+        bool on[MF], near = false;
 #pragma unroll
-    for (int k = 0; k < MF; ++k)
-        if (k < nf && down(k) && writable(k)) out(k, R.fid[k], cor[k]);
+        for (int k = 0; k < MF; ++k) {
+            smax[k] = fabs(over * R.phdt[k] - (R.dvf[k] + cor[k]));
+            on[k] = D.down[k] && smax[k] > D.tol.hi;
+            near |= D.down[k] && !on[k] && !(smax[k] < D.tol.lo);
+        }
+        if (near) {
+#pragma unroll
+            for (int k = 0; k < MF; ++k) on[k] = D.down[k] && smax[k] / R.Vi > aTol;
+        }
+#pragma unroll
+        for (int k = 0; k < MF; ++k) dVftot += on[k] ? fabs(R.phdt[k]) : -0.0;
+        const Rcp rTot = rcp_of(dVftot);
+        const double amount = fabs(fluid);
+        double fl[MF];
+#pragma unroll
+        for (int k = 0; k < MF; ++k) fl[k] = div_by(amount * fabs(R.phdt[k]), rTot);
+        if (!(D.plainFlux && amount > 1e-140 && amount < 1e140)) {
+#pragma unroll
+            for (int k = 0; k < MF; ++k) fl[k] = amount * fabs(R.phdt[k]) / dVftot;
+        }
+        open = false;
+        const unsigned sF = (unsigned)__double2hiint(fluid);
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            open |= on[k] && smax[k] >= fl[k];
+            const double f = fmin(fl[k], smax[k]);
+            // sgn(phi) sgn(fluid) fl
+            const double v = cor[k] + flip_sign(f, (sF ^ (unsigned)__double2hiint(R.phdt[k])) & 0x80000000u);
+            cor[k] = choose(on[k] && D.writes[k], v, cor[k]);
+        }
+    }
+    template <class Out>
+    __device__ __attribute__((always_inline)) inline void publish(const BndRec<MF>& R, const BndDiv<MF>& D,
+                                                                  Out out) const {
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if (D.writes[k]) out(k, R.fid[k], cor[k]);
+    }
+};
+constexpr int BOUND_ITERATIONS = 10;
+
+template <int MF, class Out>
+__device__ __attribute__((always_inline)) inline void bound_finish(const BndRec<MF>& R, const BndDiv<MF>& D,
+                                                                   const double (&cin)[MF], Out out) {
+    BndSolve<MF> S;
+    S.start(R, D, cin);
+    S.settle(R, D);
+    for (int iter = 1; iter < BOUND_ITERATIONS && !S.settled(); iter++) {
+        S.share(R, D);
+        S.settle(R, D);
+    }
+    S.publish(R, D, out);
 }
 
 // Ascending candidates of the pass from the bitmap in one launch: every
@@ -1863,12 +1951,25 @@ template <int MF>
 __device__ __attribute__((always_inline)) inline void k_bnd_prep_body(const DevMesh& m, const DevState& st, double dt,
                                                                       const double* Sp, const double* Su) {
     const int nCand = st.bcount[0];
+    const BndStore<MF> recs(st.bndRec, m.nC);
     int nOpen = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nCand; i += gridDim.x * blockDim.x) {
         const int c = st.cand[i];
-        const int n = bound_record<MF>(m, st, c, dt, Sp, Su, ((BndRec<MF>*)st.bndRec)[i]);
+        BndRec<MF> R;
+        const int n = bound_record<MF>(m, st, c, dt, Sp, Su, R);
         st.active[i] = n > 0 ? 1 : 0;
-        if (n > 0) st.actIdx[c] = i;
+        if (n > 0) {
+            st.actIdx[c] = i;
+            recs.put(i, R);
+            // correctedFaces lists the first-loop faces of the candidates in
+            // ascending cell order, so the key c * MF + (rank among the cell's
+            // first-loop faces) orders any two faces as their positions in
+            // that list would; only that order is used
+            int key = c * MF;
+#pragma unroll
+            for (int k = 0; k < MF; ++k)
+                if ((R.first >> k) & 1u) st.corrPos[R.fid[k]] = key++;
+        }
         nOpen += n;
     }
     // correctedFaces length of the pass (statistics)
@@ -1882,50 +1983,17 @@ __global__ void __launch_bounds__(256) k_bnd_prep(DevMesh m, DevState st, double
 }
 
 
-// correctedFaces keys and the cells they touch (both schedules), for candidate
-// c whose record is written.  correctedFaces lists the first-loop faces of
-// the candidates in ascending cell order, so the key c * MF + (rank among
-// the cell's first-loop faces) orders any two of its faces as their positions
-// in that list would; only that order is used.  The touched-cell claims are
-// issued together, then one counter add reserves the list entries.
-template <int MF>
-__device__ inline void bound_open_faces(const DevState& st, const BndRec<MF>& R, int c) {
-    const unsigned int first = R.first;
-    int key = c * MF;
-    // claims first, results read afterwards, so that the claims overlap
-    int old[MF];
-#pragma unroll
-    for (int k = 0; k < MF; ++k) {
-        old[k] = 1;
-        if (!((first >> k) & 1u)) continue;
-        st.corrPos[R.fid[k]] = key++;
-        if (R.oth[k] >= 0) old[k] = atomicCAS(&st.touchedFlag[R.oth[k]], 0, 1);
-    }
-    const int oldSelf = first ? atomicCAS(&st.touchedFlag[c], 0, 1) : 1;
-    unsigned long long won = 0ull;
-#pragma unroll
-    for (int k = 0; k < MF; ++k)
-        if (old[k] == 0) won |= 1ull << k;
-    const bool self = oldSelf == 0;
-    const int nWon = __popcll(won) + (self ? 1 : 0);
-    if (nWon == 0) return;
-    int slot = atomicAdd(&st.bcount[2], nWon);
-    if (self) st.touched[slot++] = c;
-#pragma unroll
-    for (int k = 0; k < MF; ++k)
-        if ((won >> k) & 1ull) st.touched[slot++] = R.oth[k];
-}
-
-// Kahn schedule: correctedFaces, successors of every active candidate,
+// Kahn schedule: successors of every active candidate,
 // predecessor counts and frontier 0
 template <int MF>
 __global__ void __launch_bounds__(256) k_bnd_scatter(DevMesh m, DevState st) {
     const int nCand = st.bcount[0];
+    const BndStore<MF> recs(st.bndRec, m.nC);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nCand; i += gridDim.x * blockDim.x) {
         if (!st.active[i]) continue;
-        BndRec<MF>& R = ((BndRec<MF>*)st.bndRec)[i];
+        BndRec<MF> R;
+        recs.get(i, R);
         const int c = st.cand[i];
-        bound_open_faces<MF>(st, R, c);
         int np = 0;
 #pragma unroll
         for (int k = 0; k < MF; ++k) {
@@ -1937,39 +2005,31 @@ __global__ void __launch_bounds__(256) k_bnd_scatter(DevMesh m, DevState st) {
                 if ((bits & 8u) && st.actIdx[o] >= 0) np++;
                 if ((bits & 2u) && o > c) sc = st.actIdx[o];
             }
-            R.succ[k] = sc;
+            recs.succ(k, i) = sc;
         }
         st.pend[i] = np;
         if (np == 0) st.queue[atomicAdd(&st.bcount[3], 1)] = i;
     }
 }
 
-// boundFlux of candidate i from its record
-template <int MF, class Out>
-__device__ inline void bound_candidate(const DevState& st, const BndRec<MF>& R, const double (&cin)[MF], int i,
-                                       double dt, double rDeltaT, Out out) {
-    (void)st;
-    (void)i;
-    bound_finish<MF>(R, cin, dt, rDeltaT, out);
-}
-
 // completes cell i of frontier r and releases its successors into frontier
 // r+1; release(a) drops one pending predecessor of candidate a and returns
 // true when it was the last, push(a) appends a to the next frontier
 template <int MF, class Release, class Push>
-__device__ inline void bnd_complete(const DevState& st, int i, double dt, double rDeltaT, Release release,
-                                    Push push) {
-    const BndRec<MF>& R = ((const BndRec<MF>*)st.bndRec)[i];
+__device__ inline void bnd_complete(const DevState& st, const BndStore<MF>& recs, int i, double rDeltaT,
+                                    Release release, Push push) {
+    BndRec<MF> R;
+    recs.get(i, R);
     // predecessors wrote these corrections in an earlier round: the previous
     // kernel of the grid rounds, or before the workgroup barrier of the tail
     double cin[MF];
 #pragma unroll
     for (int k = 0; k < MF; ++k)
         cin[k] = ((R.flg[k >> 3] >> (4 * (k & 7))) & 8u) ? st.corr[R.fid[k]] : 0.0;
-    bound_candidate<MF>(st, R, cin, i, dt, rDeltaT, [&](int, int f, double v) { st.corr[f] = v; });
+    bound_finish<MF>(R, bound_divisors<MF>(R, rDeltaT), cin, [&](int, int f, double v) { st.corr[f] = v; });
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
-        const int a = R.succ[k];
+        const int a = recs.succ(k, i);
         if (a < 0) continue;
         if (release(a)) push(a);
     }
@@ -1981,11 +2041,12 @@ __global__ void __launch_bounds__(256) k_bnd_round(DevMesh m, DevState st, int r
     const int* q = st.queue + (long)(r & 1) * m.nC;
     int* qnext = st.queue + (long)((r + 1) & 1) * m.nC;
     int* nNext = &st.bcount[3 + r + 1];
+    const BndStore<MF> recs(st.bndRec, m.nC);
     const double rDeltaT = 1.0 / dt;
     auto release = [&](int a) { return atomicSub(&st.pend[a], 1) == 1; };
     auto push = [&](int a) { qnext[atomicAdd(nNext, 1)] = a; };
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
-        bnd_complete<MF>(st, q[k], dt, rDeltaT, release, push);
+        bnd_complete<MF>(st, recs, q[k], rDeltaT, release, push);
 }
 
 // Remaining rounds in one workgroup of TAIL_THREADS (frontiers are small by now); every round
@@ -2007,6 +2068,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_bnd_tail(DevMesh m, DevState s
     __shared__ unsigned int sPend[TAIL_PEND_WORDS];
     __shared__ int sQueue[2][TAIL_Q];
     const int t = threadIdx.x;
+    const BndStore<MF> recs(st.bndRec, m.nC);
     const double rDeltaT = 1.0 / dt;
     const int R = st.gridRounds;
     const int nCand = st.bcount[0];
@@ -2047,8 +2109,8 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_bnd_tail(DevMesh m, DevState s
         };
         for (int k = t; k < qn; k += TAIL_THREADS) {
             const int i = k < TAIL_Q ? sQueue[cur][k] : gq[k];
-            if (ldsPend) bnd_complete<MF>(st, i, dt, rDeltaT, releaseLds, push);
-            else bnd_complete<MF>(st, i, dt, rDeltaT, releaseGlobal, push);
+            if (ldsPend) bnd_complete<MF>(st, recs, i, rDeltaT, releaseLds, push);
+            else bnd_complete<MF>(st, recs, i, rDeltaT, releaseGlobal, push);
         }
         __syncthreads();
         if (t == 0) {
@@ -2077,6 +2139,12 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_bnd_tail(DevMesh m, DevState s
 // wait on LDS.  The lowest unfinished candidate is always ready, so the
 // waits end; a wave that sees no completion anywhere in the grid for about a
 // second flags ERR_BOUND_STALL and the pass stops.
+// Bound by the chain of levels (20k candidates of the 128^3 perturbed case:
+// up to 45), each the instructions of one trip of the waiting loop (0.7 us,
+// 1.2 with a redistribution loop) and of the memory round trip between two
+// workgroups (1 to 2 us).  With one whole boundFlux per ready cell, a
+// grid-wide count per trip and the touched-cell claims at the end: 60 us a
+// pass there, now 38; 1k candidates 35 -> 25, 220 (64^3) 12 -> 10.
 // chunk of candidates per workgroup: one per thread of the computing waves;
 // 7 + 1 waves at two waves per SIMD for cells of up to 8 faces (held
 // records fill the registers), smaller chunks for larger cells (LDS)
@@ -2115,19 +2183,19 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
     // t*MF+k: cell t, face slot k); [CH*MF, 2*CH*MF): corrections read from
     // earlier chunks, copied in by the polling wave
     constexpr int NS = CH * MF;
-    __shared__ unsigned long long sVal[2 * NS];
+    __shared__ unsigned long long sVal[2 * NS + 1];   // the last one is always 0.0: slots without a writer read it
     __shared__ int sFid[NS];                 // faces the chunk's cells write
     __shared__ int sPoll[NS][2];             // polled corrections: face, LDS slot
     __shared__ int sBase, sNPoll;
-    // records of up to 8 faces stay in registers from the chunk's start, so
-    // a cell that turns ready reads nothing but its upwind corrections
-    constexpr bool kHold = MF <= 8;
+    // a cell's record stays in registers from the chunk's start, so a cell
+    // that turns ready reads nothing but its upwind corrections
     const int nCand = st.bcount[0];
     const int t = threadIdx.x, lane = t & 63;
     const bool poller = t >= CH;
     static_assert(NS <= 64 * 64, "a polling lane tracks at most 64 entries");
     int* progress = &st.bcount[BND_PROGRESS];
-    const BndRec<MF>* rec = (const BndRec<MF>*)st.bndRec;
+    const double rDeltaT = 1.0 / dt;
+    const BndStore<MF> recs(st.bndRec, m.nC);
     while (true) {
         __syncthreads();
         if (t == 0) {
@@ -2145,9 +2213,10 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
         bool pending = active;
         const unsigned long long act = __ballot(active);
         if (lane == 0 && act) atomicAdd(&st.bcount[3], __popcll(act));
-        BndRec<MF> held;
-        if (kHold && active) held = rec[i];
-        const BndRec<MF>& R = kHold ? held : rec[active ? i : 0];
+        // (every lane loads: a lane without an active candidate the chunk's
+        // first one's record, whose flags it drops)
+        BndRec<MF> R;
+        recs.get(active ? i : base, R);
         unsigned int flg[(MF + 7) / 8];
 #pragma unroll
         for (int w = 0; w < (MF + 7) / 8; ++w) flg[w] = active ? R.flg[w] : 0u;
@@ -2175,16 +2244,13 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
         // loop reads global memory, so the loop never waits on the global
         // stores of earlier completions.
         int src[MF];
-        unsigned int need = 0u;
-        double cin[MF];
+        if (t == 0) sVal[2 * NS] = 0ull;
 #pragma unroll
         for (int k = 0; k < MF; ++k) {
-            src[k] = -1;
-            cin[k] = 0.0;
+            src[k] = 2 * NS;
             const int p = wr[k];
             if (p < 0) continue;
             const int f = R.fid[k];
-            need |= 1u << k;
             if (p >= base) {
                 const int j = p - base;
                 for (int q = 0; q < MF; ++q)
@@ -2196,8 +2262,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
                 src[k] = NS + t * MF + k;
             }
         }
-        const double dtc = dt;
-        const double rdc = 1.0 / dtc;
+        const BndDiv<MF> D = bound_divisors<MF>(R, rDeltaT);
         __syncthreads();
         FlowStall stall;
         if (poller) {
@@ -2242,38 +2307,65 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
             __hip_atomic_store(&sVal[t * MF + k], u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             __hip_atomic_store((unsigned long long*)&st.corr[f], u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         };
+        // A trip of the loop starts the cells that turned ready, takes one
+        // redistribution loop of the others and publishes those that are
+        // done, so a cell of ten loops does not hold up its wave's others.
+        BndSolve<MF> S;
+        int iter = 0;   // 0: waiting for its corrections
+        int nDone = 0;
         while (!poller && __any(pending)) {
             bool fin = false;
-            if (pending) {
-                // corrections not seen yet; each one is read until it arrives
+            if (pending && iter > 0) {
+                S.share(R, D);
+                iter++;
+            } else if (pending) {
+                // all reads in flight together; a correction that has
+                // arrived stays
+                unsigned long long u[MF];
 #pragma unroll
-                for (int k = 0; k < MF; ++k) {
-                    if (!((need >> k) & 1u)) continue;
-                    const unsigned long long u =
-                        __hip_atomic_load(&sVal[src[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (u != CORR_PENDING) {
-                        cin[k] = __longlong_as_double((long long)u);
-                        need &= ~(1u << k);
-                    }
+                for (int k = 0; k < MF; ++k)
+                    u[k] = __hip_atomic_load(&sVal[src[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                bool ready = true;
+#pragma unroll
+                for (int k = 0; k < MF; ++k) ready &= u[k] != CORR_PENDING;
+                if (ready) {
+                    double cin[MF];
+#pragma unroll
+                    for (int k = 0; k < MF; ++k) cin[k] = __longlong_as_double((long long)u[k]);
+                    S.start(R, D, cin);
+                    iter = 1;
                 }
-                if (need == 0u) {
-                    bound_finish<MF>(R, cin, dtc, rdc, out);
+            }
+            const bool moved = pending && iter > 0;
+            if (moved) {
+                S.settle(R, D);
+                if (iter >= BOUND_ITERATIONS || S.settled()) {
+                    S.publish(R, D, out);
                     pending = false;
                     fin = true;
                 }
             }
             const unsigned long long done = __ballot(fin);
-            if (done) {
-                if (lane == 0) atomicAdd(progress, __popcll(done));
+            // the grid-wide count moves once per 16 of the wave's completions:
+            // it is one address for all waves, whose atomics queue (an add per
+            // trip made the pass of 20k candidates 63 us instead of 45)
+            nDone += __popcll(done);
+            if (nDone >= 16) {
+                if (lane == 0) atomicAdd(progress, 1);
+                nDone = 0;
+            }
+            // a wave that moves goes before the waves that only look
+            if (__any(moved)) {
+                __builtin_amdgcn_s_setprio(3);
                 stall.idle = 0;
                 continue;
             }
+            __builtin_amdgcn_s_setprio(0);
             if (stall.wait(progress, lane)) {
                 if (lane == 0) atomicOr(st.errFlag, ERR_BOUND_STALL);
                 break;
             }
         }
-        if (active) bound_open_faces<MF>(st, R, st.cand[i]);
     }
 }
 
@@ -2283,14 +2375,99 @@ __global__ void __launch_bounds__(flow_threads<MF>()) k_bnd_flow(DevMesh m, DevS
 }
 
 
-// alpha of every touched cell in correctedFaces order (advectionTemplates.C:164-192)
-// and the dVf of every corrected face (the first-loop faces of the active
-// candidates)
+// alpha of a cell with corrected faces, in correctedFaces order
+// (advectionTemplates.C:164-192), and its candidate bit; returns the change of
+// the out-of-bounds count.  face >= 0: only
+// if that face is the first of the cell's corrected faces in that order, so
+// that of all faces that lead to a cell one applies it.
+template <int MF>
+__device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevMesh& m, const DevState& st, int c,
+                                                                      int face, int epoch) {
+    const double aTol = 100.0 * SVP_SMALL;
+    const int b = m.cOff[c], nf = m.cOff[c + 1] - b;
+    // every load unconditional (slots past nf repeat the last face), in
+    // batches: labels; keys; corrections, owners, empty flags, alpha
+    int fid[MF], kpos[MF], kon[MF];
+    double kval[MF];
+    unsigned char kem[MF];
+#pragma unroll
+    for (int k = 0; k < MF; ++k) fid[k] = m.cFaces[b + min(k, nf - 1)];
+#pragma unroll
+    for (int k = 0; k < MF; ++k) kpos[k] = st.corrPos[fid[k]];
+    if (face >= 0) {
+        int bpos = 0x7fffffff, bf = -1;
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if (kpos[k] >= 0 && kpos[k] < bpos) {
+                bpos = kpos[k];
+                bf = fid[k];
+            }
+        if (bf != face) return 0;
+    }
+#pragma unroll
+    for (int k = 0; k < MF; ++k) {
+        kval[k] = st.corr[fid[k]];
+        kon[k] = m.own[fid[k]];
+        kem[k] = m.fEmpty[empty_slot(m, fid[k])];
+    }
+    const double before = st.alpha[c];
+    const double Vc = m.V[c];
+    __builtin_amdgcn_sched_barrier(0);
+    bool kown[MF];
+#pragma unroll
+    for (int k = 0; k < MF; ++k) {
+        if (k >= nf) kpos[k] = -1;
+        // face_value: empty-patch faces carry nothing
+        kval[k] = (kpos[k] >= 0 && (fid[k] < m.nIF || !kem[k])) ? kval[k] : 0.0;
+        kown[k] = kpos[k] >= 0 && kon[k] == c;
+    }
+    double a = before;
+    // corrections in ascending correctedFaces position (selection over
+    // the unrolled slots: positions are distinct)
+    int last = -1;
+    for (int q = 0; q < MF; ++q) {
+        int best = -1, bpos = 0x7fffffff;
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if (kpos[k] > last && kpos[k] < bpos) {
+                bpos = kpos[k];
+                best = k;
+            }
+        if (best < 0) break;
+        double v = 0.0;
+        bool own = false;
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if (k == best) {
+                v = kval[k];
+                own = kown[k];
+            }
+        a = own ? a - v / Vc : a + v / Vc;
+        last = bpos;
+    }
+    st.alpha[c] = a;
+    const bool candNew = cell_oob(a, aTol) && need_bounding(st, c, epoch);
+    const unsigned long long bit = 1ull << (c & 63);
+    const bool candOld = (st.candBits[c >> 6] & bit) != 0ull;
+    if (candNew != candOld) {
+        if (candNew) atomicOr(&st.candBits[c >> 6], bit);
+        else atomicAnd(&st.candBits[c >> 6], ~bit);
+    }
+    return (int)loop_oob(a, aTol) - (int)loop_oob(before, aTol);
+}
+
+// The corrections applied: one thread per (candidate, face slot) and one per
+// candidate.  A corrected face (a first-loop face of an active candidate)
+// takes dVf + correction; the cell across it is applied by the first of its
+// corrected faces, unless it is an active candidate itself, which applies
+// itself.  (A list of touched cells, with a compare-and-swap per face to enter
+// each once, cost the dependent pass up to 8 us: its atomics queue with the
+// corrections.)
 template <int MF>
 __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const DevMesh& m, const DevState& st, int pass,
                                                                        int epoch) {
-    const double aTol = 100.0 * SVP_SMALL;
-    const int nT = st.bcount[2], nCand = st.bcount[0];
+    const int nCand = st.bcount[0];
+    const BndStore<MF> recs(st.bndRec, m.nC);
     // pass statistics, and the candidate count for the next list's clearing
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st.bcount[BND_PREV_COUNT] = nCand;
@@ -2312,95 +2489,31 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
         // kernel counts into it)
         st.bcount[1] = 0;
     }
-    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < nT + nCand; idx += gridDim.x * blockDim.x) {
-        if (idx >= nT) {
-            const int i = idx - nT;
-            if (!st.active[i]) continue;
-            const BndRec<MF>& R = ((const BndRec<MF>*)st.bndRec)[i];
-            const unsigned int first = R.first;
-            // every slot's loads unconditional (the record's slots past the
-            // cell's faces repeat its last face), then the writes: the
-            // faces of the first redistribution take dVf + correction
-            // (face_value of both; empty-patch faces keep theirs)
-            int fid[MF];
-            double dv[MF], cr[MF];
-            unsigned char em[MF];
-#pragma unroll
-            for (int k = 0; k < MF; ++k) fid[k] = R.fid[k];
-#pragma unroll
-            for (int k = 0; k < MF; ++k) {
-                dv[k] = st.dVf[fid[k]];
-                cr[k] = st.corr[fid[k]];
-                em[k] = m.fEmpty[empty_slot(m, fid[k])];
+    // slot-major, so that a wave's lanes read neighbouring records; the bound
+    // is a multiple of 64, so a wave's lanes leave the loop together
+    const long nPad = ((long)nCand + 63) / 64 * 64, total = nPad * (MF + 1);
+    for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
+        const int k = (int)(idx / nPad), i = (int)(idx % nPad);
+        int c = -1, face = -1, dOob = 0;
+        if (i < nCand && st.active[i]) {
+            if (k == MF) {
+                c = st.cand[i];
+            } else if (((unsigned)recs.first(i) >> k) & 1u) {
+                const int f = recs.fid(k, i), o = recs.oth(k, i);
+                // face_value of both: empty-patch faces keep theirs
+                const double dv = st.dVf[f], cr = st.corr[f];
+                const unsigned char em = m.fEmpty[empty_slot(m, f)];
+                const bool other = o >= 0 && st.actIdx[max(o, 0)] < 0;
+                if (f < m.nIF || !em) st.dVf[f] = dv + cr;
+                c = other ? o : -1;
+                face = f;
             }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < MF; ++k)
-                if (((first >> k) & 1u) && (fid[k] < m.nIF || !em[k])) st.dVf[fid[k]] = dv[k] + cr[k];
-            continue;
         }
-        const int c = st.touched[idx];
-        const int b = m.cOff[c], nf = m.cOff[c + 1] - b;
-        // every load unconditional (slots past nf repeat the last face), in
-        // three batches: labels; keys, corrections, owners, empty flags; alpha
-        int fid[MF], kpos[MF], kon[MF];
-        double kval[MF];
-        unsigned char kem[MF];
-#pragma unroll
-        for (int k = 0; k < MF; ++k) fid[k] = m.cFaces[b + min(k, nf - 1)];
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            kpos[k] = st.corrPos[fid[k]];
-            kval[k] = st.corr[fid[k]];
-            kon[k] = m.own[fid[k]];
-            kem[k] = m.fEmpty[empty_slot(m, fid[k])];
-        }
-        const double before = st.alpha[c];
-        const double Vc = m.V[c];
-        __builtin_amdgcn_sched_barrier(0);
-        bool kown[MF];
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            if (k >= nf) kpos[k] = -1;
-            // face_value: empty-patch faces carry nothing
-            kval[k] = (kpos[k] >= 0 && (fid[k] < m.nIF || !kem[k])) ? kval[k] : 0.0;
-            kown[k] = kpos[k] >= 0 && kon[k] == c;
-        }
-        double a = before;
-        // corrections in ascending correctedFaces position (selection over
-        // the unrolled slots: positions are distinct)
-        int last = -1;
-        for (int q = 0; q < MF; ++q) {
-            int best = -1, bpos = 0x7fffffff;
-#pragma unroll
-            for (int k = 0; k < MF; ++k)
-                if (kpos[k] > last && kpos[k] < bpos) {
-                    bpos = kpos[k];
-                    best = k;
-                }
-            if (best < 0) break;
-            double v = 0.0;
-            bool own = false;
-#pragma unroll
-            for (int k = 0; k < MF; ++k)
-                if (k == best) {
-                    v = kval[k];
-                    own = kown[k];
-                }
-            a = own ? a - v / Vc : a + v / Vc;
-            last = bpos;
-        }
-        st.alpha[c] = a;
-        const int dOob = (int)loop_oob(a, aTol) - (int)loop_oob(before, aTol);
-        if (dOob) atomicAdd(&st.oobCount[OOB_STRIDE * ((c >> 8) & (OOB_SLOTS - 1))], dOob);
-        const bool candNew = cell_oob(a, aTol) && need_bounding(st, c, epoch);
-        const unsigned long long bit = 1ull << (c & 63);
-        const bool candOld = (st.candBits[c >> 6] & bit) != 0ull;
-        if (candNew != candOld) {
-            if (candNew) atomicOr(&st.candBits[c >> 6], bit);
-            else atomicAnd(&st.candBits[c >> 6], ~bit);
-        }
-        st.touchedFlag[c] = 0;
+        if (c >= 0) dOob = bound_apply_cell<MF>(m, st, c, face, epoch);
+        // one add per wave (a wave's cells lie together)
+        const int d = __popcll(__ballot(dOob > 0)) - __popcll(__ballot(dOob < 0));
+        if (d && (threadIdx.x & 63) == 0)
+            atomicAdd(&st.oobCount[OOB_STRIDE * ((idx >> 6) & (OOB_SLOTS - 1))], d);
     }
 }
 
@@ -2427,7 +2540,7 @@ void launch_bound_pass(const DevMesh& m, const DevState& st, int pass, double dt
         for (int r = 0; r < st.gridRounds; ++r) k_bnd_round<MF><<<grid, 256, 0, s>>>(m, st, r, dt);
         k_bnd_tail<MF><<<1, TAIL_THREADS, 0, s>>>(m, st, dt);
     }
-    k_bnd_apply<MF><<<grid, 256, 0, s>>>(m, st, pass);
+    k_bnd_apply<MF><<<std::max(1, std::min(4 * st.bndGrid, cdiv((long)m.nC * (MF + 1), 256))), 256, 0, s>>>(m, st, pass);
 }
 
 // The state of bounding pass number seq of a handle: its candidate list,
@@ -2458,10 +2571,10 @@ int bound_faces(int maxCellFaces) {
 
 size_t bound_record_bytes(int maxCellFaces) {
     switch (bound_faces(maxCellFaces)) {
-        case 4: return sizeof(BndRec<4>);
-        case 6: return sizeof(BndRec<6>);
-        case NS_CELL_FACES: return sizeof(BndRec<NS_CELL_FACES>);
-        default: return sizeof(BndRec<MAX_CELL_FACES>);
+        case 4: return BndStore<4>::bytes();
+        case 6: return BndStore<6>::bytes();
+        case NS_CELL_FACES: return BndStore<NS_CELL_FACES>::bytes();
+        default: return BndStore<MAX_CELL_FACES>::bytes();
     }
 }
 

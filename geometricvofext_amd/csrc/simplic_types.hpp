@@ -83,8 +83,6 @@ struct DevState {
     int* queue;         // 2*nC, Kahn frontiers
     int* actIdx;        // nC cells -> candidate index of active cells, else -1
     int* corrPos;       // nF faces -> order key in correctedFaces (cell * max faces + rank), else -1
-    int* touched;       // nC, cells whose alpha gets corrections
-    int* touchedFlag;   // nC
     int* boundStats;    // [4*maxPasses]: candidates, active, rounds, corrected faces
     unsigned long long* boundTotals;  // [5] running sums: candidates, active, rounds, corrected faces, passes
     int* bcount;        // [32] per-pass counters of the bounding kernels
@@ -100,7 +98,7 @@ struct DevState {
     int bndGrid;        // workgroups of the grid-stride bounding kernels
     int bndFlow;        // workgroups of the one-launch dataflow pass, 0 = rounds and tail
     int bndListWords;   // bitmap words per block of the candidate list (64..4096)
-    void* bndRec;       // nC records BndRec<MF> of the active bounding candidates
+    void* bndRec;       // BndStore<MF> of the active bounding candidates, capacity nC
     int maxCellFaces;
     double* minmax;     // [4]: min, max before bounding, min, max after
     int* errFlag;       // [1] device error bits
@@ -143,16 +141,14 @@ constexpr int OOB_STRIDE = 16;
 constexpr int DETECT_BLOCK = 256;
 
 // Face data of an active bounding candidate, gathered once per pass with the
-// first iteration of its redistribution loop done, so that the dependent
-// part reads one contiguous record.  flags: 4 bits per face (owner,
-// downwind, writable, upwind writer with a lower label).
+// first iteration of its redistribution loop done.  flags: 4 bits per face
+// (owner, downwind, writable, upwind writer with a lower label).
 template <int MF>
 struct BndRec {
-    double phf[MF], dvf[MF];
+    double phdt[MF], dvf[MF];   // flux times dt, face volume (empty-patch faces: zero)
     double cor0[MF];    // downwind corrections after iteration 0
     int fid[MF];
     int oth[MF];        // cell on the other side of the face, -1 on boundary faces
-    int succ[MF];       // Kahn schedule: candidate index of the active downwind neighbour with a higher label, else -1
     unsigned int flg[(MF + 7) / 8];
     int nf;
     unsigned int first;  // face slots of the first redistribution loop, in correctedFaces order
@@ -160,6 +156,65 @@ struct BndRec {
     double Vi;
     double num0;         // alpha_old/dt (+Su) - sum(dVf)/V/dt, the part of the new alpha's numerator without corrections
     double den;          // 1/dt (-Sp)
+};
+
+// The records in memory: one array per value over the candidates, so that a
+// wave's lanes read and write neighbouring words (a record of its own lines
+// per lane took a line per lane and load).
+template <int MF>
+struct BndStore {
+    static constexpr int NW = (MF + 7) / 8;
+    static constexpr int DOUBLES = 3 * MF + 3, INTS = 3 * MF + NW + 3;
+    double* d;
+    int* w;
+    long cap;
+    __host__ __device__ BndStore(void* base, long capacity)
+        : d((double*)base), w((int*)((double*)base + DOUBLES * capacity)), cap(capacity) {}
+    __device__ double& f64(int field, int i) const { return d[field * cap + i]; }
+    __device__ int& i32(int field, int i) const { return w[field * cap + i]; }
+    __device__ int& fid(int k, int i) const { return i32(k, i); }
+    __device__ int& oth(int k, int i) const { return i32(MF + k, i); }
+    // Kahn schedule: candidate index of the active downwind neighbour with a
+    // higher label, else -1
+    __device__ int& succ(int k, int i) const { return i32(2 * MF + k, i); }
+    __device__ int& first(int i) const { return i32(3 * MF + NW, i); }
+    __device__ void put(int i, const BndRec<MF>& R) const {
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            f64(k, i) = R.phdt[k];
+            f64(MF + k, i) = R.dvf[k];
+            f64(2 * MF + k, i) = R.cor0[k];
+            fid(k, i) = R.fid[k];
+            oth(k, i) = R.oth[k];
+        }
+        f64(3 * MF, i) = R.Vi;
+        f64(3 * MF + 1, i) = R.num0;
+        f64(3 * MF + 2, i) = R.den;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) i32(3 * MF + q, i) = (int)R.flg[q];
+        first(i) = (int)R.first;
+        i32(3 * MF + NW + 1, i) = R.nf;
+        i32(3 * MF + NW + 2, i) = R.nFaces0;
+    }
+    __device__ void get(int i, BndRec<MF>& R) const {
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            R.phdt[k] = f64(k, i);
+            R.dvf[k] = f64(MF + k, i);
+            R.cor0[k] = f64(2 * MF + k, i);
+            R.fid[k] = fid(k, i);
+            R.oth[k] = oth(k, i);
+        }
+        R.Vi = f64(3 * MF, i);
+        R.num0 = f64(3 * MF + 1, i);
+        R.den = f64(3 * MF + 2, i);
+#pragma unroll
+        for (int q = 0; q < NW; ++q) R.flg[q] = (unsigned)i32(3 * MF + q, i);
+        R.first = (unsigned)first(i);
+        R.nf = i32(3 * MF + NW + 1, i);
+        R.nFaces0 = i32(3 * MF + NW + 2, i);
+    }
+    static constexpr size_t bytes() { return DOUBLES * sizeof(double) + INTS * sizeof(int); }
 };
 
 // One case of a batch of independent handles advanced together (one launch

@@ -1,0 +1,59 @@
+"""Bounding of every cell type and candidate count against the oracle: fields
+that leave many cells out of bounds (a random alpha advected with a large
+step), so that a pass has fewer candidates than a workgroup takes, exactly
+about as many, and several workgroups' worth that read one another's
+corrections; with and without sources, under both schedules."""
+import numpy as np
+import pytest
+
+from tests.helpers import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def case_mesh(kind, N):
+    import geometricvofext_amd as g
+    if kind == "tet":
+        return g.tet_box(N, perturb=0.1, seed=N)
+    if kind == "refined":
+        return g.refined_hex_box(N)
+    return g.hex_box(N, perturb=0.2 if kind == "hexp" else 0.0, seed=N)
+
+
+@pytest.mark.parametrize("kind,N,passes,sources", [("hex", 2, 1, False), ("hexp", 5, 3, False), ("hexp", 9, 3, True),
+                                                   ("hexp", 14, 10, False), ("hex", 20, 3, False), ("tet", 4, 3, True),
+                                                   ("tet", 10, 4, False), ("refined", 8, 3, False),
+                                                   ("refined", 12, 3, True)])
+@pytest.mark.parametrize("schedule", ["flow", "rounds"])
+def test_bound_every_count(oracle_lib, monkeypatch, kind, N, passes, sources, schedule):
+    import geometricvofext_amd as g
+    print("bound", kind, N, passes, sources, schedule, flush=True)
+    if schedule == "rounds":
+        monkeypatch.setenv("SVP_BND_FLOW", "0")
+    mesh = case_mesh(kind, N)
+    om = oracle_lib.OracleMesh(mesh)
+    rng = np.random.default_rng(7 + N)
+    alpha = np.clip(rng.normal(0.5, 0.6, mesh.n_cells), 0.0, 1.0)
+    V = np.array([0.5, -0.4, 0.7])
+    U = np.tile(V, (mesh.n_cells, 1)) + 0.3 * rng.normal(size=(mesh.n_cells, 3))
+    phi = om.Sf @ V
+    dt = 0.6 * float(np.min(om.V)) ** (1.0 / 3.0)
+    Sp = Su = None
+    if sources:
+        Sp, Su = -0.3 * rng.random(mesh.n_cells), 0.2 * rng.random(mesh.n_cells)
+    gpu = g.SolveVofEqu(mesh, dict(orientationMethod="LS", nAlphaBounds=passes, clip=False))
+    ors = oracle_lib.OracleSolver(om, nAlphaBounds=passes, clip=False, threads=8)
+    for step in range(3):
+        for s in (gpu, ors):
+            if step == 0:
+                s.set_alpha(alpha)
+            s.set_flow(phi, U)
+            s.reconstruct()
+            if sources:
+                s.advect(dt, Sp, Su)
+            else:
+                s.advect(dt)
+        assert bits_equal(gpu.alpha(), ors.alpha()), step
+        assert bits_equal(gpu.alpha_phi(), ors.alpha_phi()), step
+    print("candidates", gpu.bound_stats()[:, 0].tolist(), flush=True)
+    gpu.synchronize()
