@@ -1018,6 +1018,10 @@ private:
             const int g = std::atoi(e);
             if (g >= 0 && g <= 4096) st_.bndFlow = g;
         }
+        // all passes in one workgroup up to this many cells (knob
+        // SVP_BND_SMALL; results do not depend on it)
+        st_.bndSmall = BOUND_SMALL_CELLS;
+        if (const char* e = std::getenv("SVP_BND_SMALL")) st_.bndSmall = std::atoi(e);
         st_.bndRec = (void*)dalloc<unsigned char>(bound_record_bytes(maxCellFaces_) * (size_t)nC);
         st_.un0Fused = (!dict_.split_warped_face && maxCellFaces_ <= 8 && m_.maxCellPoints <= NS_CELL_POINTS &&
                         m_.triQuadFaces) ? 1 : 0;
@@ -1085,6 +1089,10 @@ public:
             listed = listed || flux_listed(h->m_, h->st_.maxCellFaces);
         }
         fluxListed_ = listed;
+        bndSmall_ = true;
+        for (solveVofEqu* h : c_)
+            bndSmall_ = bndSmall_ && h->st_.bndFlow && h->st_.bndSmall > 0 &&
+                        h->m_.nC <= BOUND_SMALL_BATCH_CELLS;
         DevMesh any = f.m_;
         if (listed) any.facePoints = 0;
         fluxKind_ = flux_kind(any, f.st_.maxCellFaces, 2 * nFan > n ? 1 : 0);
@@ -1204,7 +1212,7 @@ public:
 
     void launchStage(int sg) {
         launch_batch_stage(sg, (const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, size(), maxC_, maxF_,
-                           maxDet_, maxList_, dims_, params_, G_, MF_, fluxKind_, fluxListed_, stream_);
+                           maxDet_, maxList_, dims_, params_, G_, MF_, fluxKind_, fluxListed_, bndSmall_, stream_);
     }
 
     void dropGraph() {
@@ -1371,6 +1379,7 @@ private:
     int G_ = 6, MF_ = NS_CELL_FACES, triQuad_ = 1;
     int fluxKind_ = 0;
     bool fluxListed_ = true;
+    bool bndSmall_ = false;
     int maxC_ = 0, maxF_ = 0, maxDet_ = 0, maxList_ = 0;
     long maxN_ = 0;
     bool haveFlow_ = true;

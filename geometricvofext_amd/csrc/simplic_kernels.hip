@@ -1842,6 +1842,37 @@ __device__ inline bool oob_any(const DevState& st) {
     return n != 0;
 }
 
+// What a pass (of this step or the last one) left in its half of the double
+// buffers: the corrections and correctedFaces keys on the faces of its active
+// cells and their candidate index, back to 0 / -1 (thread t of nt).
+__device__ __attribute__((always_inline)) inline void bound_clear(const DevMesh& m, const BndPrev& prev, int nPrev,
+                                                                  int t, int nt) {
+    for (int i = t; i < nPrev; i += nt) {
+        if (!prev.active[i]) continue;
+        const int c = prev.cand[i];
+        const int fb = m.cOff[c], nf = m.cOff[c + 1] - fb;
+        if (nf <= 8) {
+            // the face labels loaded together, then the stores
+            int fs[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) fs[k] = m.cFaces[fb + min(k, nf - 1)];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k < nf) {
+                    prev.corr[fs[k]] = 0.0;
+                    prev.corrPos[fs[k]] = -1;
+                }
+        } else {
+            for (int k = fb; k < fb + nf; ++k) {
+                const int f = m.cFaces[k];
+                prev.corr[f] = 0.0;
+                prev.corrPos[f] = -1;
+            }
+        }
+        prev.actIdx[c] = -1;
+    }
+}
+
 __device__ __attribute__((always_inline)) inline void k_bnd_list_body(const DevMesh& m, const DevState& st, int nWords,
                                                                       int nBlocks, const BndPrev& prev) {
     __shared__ int lds[16];
@@ -1851,37 +1882,11 @@ __device__ __attribute__((always_inline)) inline void k_bnd_list_body(const DevM
     __syncthreads();
     const int b = sTicket;
     const unsigned epoch = sEpoch;
-    // what the previous pass (of this step or the last one) left: the
-    // corrections and correctedFaces keys on the faces of its active cells
-    // and their candidate index, back to 0 / -1 before this pass's records.
-    // Done by the waves that wait while wave 0 looks back (thread t of nt
-    // clearing threads per block), off the look-back chain.
+    // what the previous pass left, cleared by the waves that wait while wave 0
+    // looks back (thread t of nt clearing threads per block), off the
+    // look-back chain
     auto clearPrevious = [&](int t, int nt) {
-        const int nPrev = st.bcount[BND_PREV_COUNT];
-        for (int i = b * nt + t; i < nPrev; i += nBlocks * nt) {
-            if (!prev.active[i]) continue;
-            const int c = prev.cand[i];
-            const int fb = m.cOff[c], nf = m.cOff[c + 1] - fb;
-            if (nf <= 8) {
-                // the face labels loaded together, then the stores
-                int fs[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) fs[k] = m.cFaces[fb + min(k, nf - 1)];
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (k < nf) {
-                        prev.corr[fs[k]] = 0.0;
-                        prev.corrPos[fs[k]] = -1;
-                    }
-            } else {
-                for (int k = fb; k < fb + nf; ++k) {
-                    const int f = m.cFaces[k];
-                    prev.corr[f] = 0.0;
-                    prev.corrPos[f] = -1;
-                }
-            }
-            prev.actIdx[c] = -1;
-        }
+        bound_clear(m, prev, st.bcount[BND_PREV_COUNT], b * nt + t, nBlocks * nt);
     };
     // the counters the later kernels of the pass count into (the corrected
     // faces of [1] are counted here, so the previous apply cleared them)
@@ -1942,6 +1947,30 @@ __global__ void __launch_bounds__(256) k_bnd_list(DevMesh m, DevState st, int nW
     k_bnd_list_body(m, st, nWords, nBlocks, prev);
 }
 
+// record of candidate i; returns the faces it opens in correctedFaces
+template <int MF>
+__device__ __attribute__((always_inline)) inline int bound_prepare(const DevMesh& m, const DevState& st,
+                                                                   const BndStore<MF>& recs, int i, double dt,
+                                                                   const double* Sp, const double* Su) {
+    const int c = st.cand[i];
+    BndRec<MF> R;
+    const int n = bound_record<MF>(m, st, c, dt, Sp, Su, R);
+    st.active[i] = n > 0 ? 1 : 0;
+    if (n > 0) {
+        st.actIdx[c] = i;
+        recs.put(i, R);
+        // correctedFaces lists the first-loop faces of the candidates in
+        // ascending cell order, so the key c * MF + (rank among the cell's
+        // first-loop faces) orders any two faces as their positions in that
+        // list would; only that order is used
+        int key = c * MF;
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if ((R.first >> k) & 1u) st.corrPos[R.fid[k]] = key++;
+    }
+    return n;
+}
+
 // every candidate's record (iteration 0 of boundFlux done) and, when it
 // writes corrections, its candidate index and the CORR_PENDING marks of the
 // faces it will write; one candidate per thread over the whole grid (the
@@ -1954,23 +1983,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_prep_body(const DevM
     const BndStore<MF> recs(st.bndRec, m.nC);
     int nOpen = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nCand; i += gridDim.x * blockDim.x) {
-        const int c = st.cand[i];
-        BndRec<MF> R;
-        const int n = bound_record<MF>(m, st, c, dt, Sp, Su, R);
-        st.active[i] = n > 0 ? 1 : 0;
-        if (n > 0) {
-            st.actIdx[c] = i;
-            recs.put(i, R);
-            // correctedFaces lists the first-loop faces of the candidates in
-            // ascending cell order, so the key c * MF + (rank among the cell's
-            // first-loop faces) orders any two faces as their positions in
-            // that list would; only that order is used
-            int key = c * MF;
-#pragma unroll
-            for (int k = 0; k < MF; ++k)
-                if ((R.first >> k) & 1u) st.corrPos[R.fid[k]] = key++;
-        }
-        nOpen += n;
+        nOpen += bound_prepare<MF>(m, st, recs, i, dt, Sp, Su);
     }
     // correctedFaces length of the pass (statistics)
     for (int o = 32; o > 0; o >>= 1) nOpen += __shfl_xor(nOpen, o);
@@ -2448,12 +2461,37 @@ __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevM
     st.alpha[c] = a;
     const bool candNew = cell_oob(a, aTol) && need_bounding(st, c, epoch);
     const unsigned long long bit = 1ull << (c & 63);
-    const bool candOld = (st.candBits[c >> 6] & bit) != 0ull;
+    // (an atomic load: the word changes by atomics, past the L1 that a kernel
+    // of several passes would read)
+    const bool candOld = (__hip_atomic_load(&st.candBits[c >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) != 0ull;
     if (candNew != candOld) {
         if (candNew) atomicOr(&st.candBits[c >> 6], bit);
         else atomicAnd(&st.candBits[c >> 6], ~bit);
     }
     return (int)loop_oob(a, aTol) - (int)loop_oob(before, aTol);
+}
+
+// slot k of candidate i (k = MF: the candidate's own cell)
+template <int MF>
+__device__ __attribute__((always_inline)) inline int bound_apply_item(const DevMesh& m, const DevState& st,
+                                                                      const BndStore<MF>& recs, int k, int i,
+                                                                      int nCand, int epoch) {
+    int c = -1, face = -1;
+    if (i < nCand && st.active[i]) {
+        if (k == MF) {
+            c = st.cand[i];
+        } else if (((unsigned)recs.first(i) >> k) & 1u) {
+            const int f = recs.fid(k, i), o = recs.oth(k, i);
+            // face_value of both: empty-patch faces keep theirs
+            const double dv = st.dVf[f], cr = st.corr[f];
+            const unsigned char em = m.fEmpty[empty_slot(m, f)];
+            const bool other = o >= 0 && st.actIdx[max(o, 0)] < 0;
+            if (f < m.nIF || !em) st.dVf[f] = dv + cr;
+            c = other ? o : -1;
+            face = f;
+        }
+    }
+    return c >= 0 ? bound_apply_cell<MF>(m, st, c, face, epoch) : 0;
 }
 
 // The corrections applied: one thread per (candidate, face slot) and one per
@@ -2493,23 +2531,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
     // is a multiple of 64, so a wave's lanes leave the loop together
     const long nPad = ((long)nCand + 63) / 64 * 64, total = nPad * (MF + 1);
     for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-        const int k = (int)(idx / nPad), i = (int)(idx % nPad);
-        int c = -1, face = -1, dOob = 0;
-        if (i < nCand && st.active[i]) {
-            if (k == MF) {
-                c = st.cand[i];
-            } else if (((unsigned)recs.first(i) >> k) & 1u) {
-                const int f = recs.fid(k, i), o = recs.oth(k, i);
-                // face_value of both: empty-patch faces keep theirs
-                const double dv = st.dVf[f], cr = st.corr[f];
-                const unsigned char em = m.fEmpty[empty_slot(m, f)];
-                const bool other = o >= 0 && st.actIdx[max(o, 0)] < 0;
-                if (f < m.nIF || !em) st.dVf[f] = dv + cr;
-                c = other ? o : -1;
-                face = f;
-            }
-        }
-        if (c >= 0) dOob = bound_apply_cell<MF>(m, st, c, face, epoch);
+        const int dOob = bound_apply_item<MF>(m, st, recs, (int)(idx / nPad), (int)(idx % nPad), nCand, epoch);
         // one add per wave (a wave's cells lie together)
         const int d = __popcll(__ballot(dOob > 0)) - __popcll(__ballot(dOob < 0));
         if (d && (threadIdx.x & 63) == 0)
@@ -2520,6 +2542,233 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
 template <int MF>
 __global__ void __launch_bounds__(256) k_bnd_apply(DevMesh m, DevState st, int pass) {
     k_bnd_apply_body<MF>(m, st, pass, st.epoch);
+}
+
+// one half of the bounding double buffers
+struct BndHalf {
+    int* cand;
+    unsigned char* active;
+    double* corr;
+    int* corrPos;
+    int* actIdx;
+};
+__host__ __device__ inline BndHalf bound_half(const DevState& v) {
+    return BndHalf{v.cand, v.active, v.corr, v.corrPos, v.actIdx};
+}
+
+// All passes of a step by one workgroup: list, records, dependent pass and
+// apply of every pass with barriers between them instead of launches.  On a
+// small mesh a pass has a few hundred candidates at most and its four launches
+// are launch and memory latency (about 25 us a pass with the gaps between
+// them); one workgroup has no look-back, no polling and no idle launches after
+// the last cell is in bounds.  A's halves of the double buffers are those of
+// even passes, B those of odd ones.  Only the candidate bitmap
+// changes by atomics here; its words are read past the L1.
+//
+// 10 passes of about 200 candidates (33^3 perturbed, the default dictionary):
+// 151 us, against 250 us of kernels in 40 launches and the gaps between them; 3
+// passes of 1 to 20 (16^3): 34 us against 61.
+constexpr int SMALL_THREADS = 512;
+
+template <int MF>
+__device__ __attribute__((always_inline)) inline void k_bnd_small_body(const DevMesh& m, const DevState& A,
+                                                                       const BndHalf& B, int nPasses, double dt,
+                                                                       const double* Sp, const double* Su,
+                                                                       int epoch) {
+    constexpr int T = SMALL_THREADS, NS = T * MF, NW = T / 64;
+    __shared__ unsigned long long sVal[NS + 1];   // corrections of the chunk's cells; the last one 0.0
+    __shared__ int sFid[NS];
+    __shared__ int sItem[T * (MF + 1)];            // (candidate, face slot) pairs of the apply
+    __shared__ int sWave[NW];
+    __shared__ int sOob, sAct, sOpen, sItems;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int nWords = (m.nC + 63) / 64, per = (nWords + T - 1) / T;
+    const double rDeltaT = 1.0 / dt;
+    const BndStore<MF> recs(A.bndRec, m.nC);
+    int* bcount = A.bcount;
+    if (t < 64) {
+        int n = A.oobCount[OOB_STRIDE * t];
+        static_assert(OOB_SLOTS == 64, "one counter per lane");
+        for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+        if (t == 0) sOob = n;
+    }
+    int nPrev = bcount[BND_PREV_COUNT];
+    for (int pass = 0; pass < nPasses; ++pass) {
+        const bool odd = (pass & 1) != 0;
+        DevState st = A;   // this pass's half; `other` the one before it left
+        st.cand = odd ? B.cand : A.cand;
+        st.active = odd ? B.active : A.active;
+        st.corr = odd ? B.corr : A.corr;
+        st.corrPos = odd ? B.corrPos : A.corrPos;
+        st.actIdx = odd ? B.actIdx : A.actIdx;
+        const BndPrev other{odd ? A.cand : B.cand, odd ? A.active : B.active, odd ? A.corr : B.corr,
+                            odd ? A.corrPos : B.corrPos, odd ? A.actIdx : B.actIdx};
+        __syncthreads();
+        if (sOob == 0) {
+            bound_clear(m, other, nPrev, t, T);
+            nPrev = 0;
+            break;
+        }
+        // ascending candidates: every thread its run of words
+        int cnt = 0;
+        for (int w = t * per; w < min(nWords, (t + 1) * per); ++w)
+            cnt += __popcll(__hip_atomic_load(&st.candBits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        int x = cnt;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) sWave[wave] = x;
+        __syncthreads();
+        int off = x - cnt, nCand = 0;
+        for (int w = 0; w < NW; ++w) {
+            off += w < wave ? sWave[w] : 0;
+            nCand += sWave[w];
+        }
+        if (cnt)
+            for (int w = t * per; w < min(nWords, (t + 1) * per); ++w) {
+                unsigned long long bits =
+                    __hip_atomic_load(&st.candBits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                while (bits) {
+                    st.cand[off++] = w * 64 + __ffsll((long long)bits) - 1;
+                    bits &= bits - 1;
+                }
+            }
+        if (t == 0) sAct = sOpen = sItems = 0;
+        __syncthreads();
+        int nOpen = 0;
+        for (int i = t; i < nCand; i += T) nOpen += bound_prepare<MF>(m, st, recs, i, dt, Sp, Su);
+        if (nOpen) atomicAdd(&sOpen, nOpen);
+        // the dependent part, chunk after chunk: an earlier chunk's
+        // corrections are final, so only the chunk's own are waited for
+        for (int base = 0; base < nCand; base += T) {
+            __syncthreads();
+            const int i = base + t;
+            const bool active = i < nCand && st.active[i] != 0;
+            const unsigned long long act = __ballot(active);
+            if (lane == 0 && act) atomicAdd(&sAct, __popcll(act));
+            BndRec<MF> R;
+            recs.get(active ? i : base, R);
+            if (active && nCand <= T) {
+                // the cell itself (slot MF) and its first-loop faces
+                int at = atomicAdd(&sItems, __popc(R.first) + 1);
+                sItem[at++] = t * 32 + MF;
+#pragma unroll
+                for (int k = 0; k < MF; ++k)
+                    if ((R.first >> k) & 1u) sItem[at++] = t * 32 + k;
+            }
+            auto bits = [&](int k) { return active ? R.flg[k >> 3] >> (4 * (k & 7)) : 0u; };
+            int wr[MF];
+#pragma unroll
+            for (int k = 0; k < MF; ++k) wr[k] = st.actIdx[(bits(k) & 8u) ? R.oth[k] : 0];
+#pragma unroll
+            for (int k = 0; k < MF; ++k) {
+                if (!(bits(k) & 8u)) wr[k] = -1;
+                sFid[t * MF + k] = ((bits(k) & 6u) == 6u) ? R.fid[k] : -1;
+                sVal[t * MF + k] = CORR_PENDING;
+            }
+            if (t == 0) sVal[NS] = 0ull;
+            __syncthreads();
+            int src[MF];
+            double early[MF];
+#pragma unroll
+            for (int k = 0; k < MF; ++k) {
+                src[k] = NS;
+                early[k] = 0.0;
+                const int p = wr[k];
+                if (p < 0) continue;
+                if (p >= base) {
+                    const int j = p - base;
+                    for (int q = 0; q < MF; ++q)
+                        if (sFid[j * MF + q] == R.fid[k]) src[k] = j * MF + q;
+                } else {
+                    early[k] = st.corr[R.fid[k]];
+                }
+            }
+            const BndDiv<MF> D = bound_divisors<MF>(R, rDeltaT);
+            auto out = [&](int k, int f, double v) {
+                __hip_atomic_store(&sVal[t * MF + k], (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                st.corr[f] = v;
+            };
+            BndSolve<MF> S;
+            bool pending = active;
+            int iter = 0, idle = 0;
+            while (__any(pending)) {
+                if (pending && iter > 0) {
+                    S.share(R, D);
+                    iter++;
+                } else if (pending) {
+                    unsigned long long u[MF];
+#pragma unroll
+                    for (int k = 0; k < MF; ++k)
+                        u[k] = __hip_atomic_load(&sVal[src[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    bool ready = true;
+#pragma unroll
+                    for (int k = 0; k < MF; ++k) ready &= u[k] != CORR_PENDING;
+                    if (ready) {
+                        double cin[MF];
+#pragma unroll
+                        for (int k = 0; k < MF; ++k) cin[k] = early[k] + __longlong_as_double((long long)u[k]);
+                        S.start(R, D, cin);
+                        iter = 1;
+                    }
+                }
+                const bool moved = pending && iter > 0;
+                if (moved) {
+                    S.settle(R, D);
+                    if (iter >= BOUND_ITERATIONS || S.settled()) {
+                        S.publish(R, D, out);
+                        pending = false;
+                    }
+                }
+                // the lowest unfinished candidate is always ready, so a wave
+                // waits for a few levels at most
+                if (__any(moved)) {
+                    __builtin_amdgcn_s_setprio(3);
+                    idle = 0;
+                } else {
+                    __builtin_amdgcn_s_setprio(0);
+                    __builtin_amdgcn_s_sleep(1);
+                    if (++idle > FLOW_STALL_CHECKS * 64) {
+                        if (lane == 0) atomicOr(A.errFlag, ERR_BOUND_STALL);
+                        break;
+                    }
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        __syncthreads();
+        if (t == 0 && nCand > 0) {
+            A.boundStats[4 * pass + 0] = nCand;
+            A.boundStats[4 * pass + 1] = sAct;
+            A.boundStats[4 * pass + 2] = 0;
+            A.boundStats[4 * pass + 3] = sOpen;
+            A.boundTotals[0] += (unsigned long long)nCand;
+            A.boundTotals[1] += (unsigned long long)sAct;
+            A.boundTotals[3] += (unsigned long long)sOpen;
+            A.boundTotals[4] += 1ull;
+            *A.candCount = nCand;
+        }
+        // the listed pairs, or all of more candidates than the list is for;
+        // then what the pass before left
+        const bool listed = nCand <= T;
+        const int nPad = (nCand + 63) / 64 * 64, nWork = listed ? sItems : nPad * (MF + 1);
+        int d = 0;
+        for (int idx = t; idx < nWork; idx += T)
+            d += bound_apply_item<MF>(m, st, recs, listed ? sItem[idx] & 31 : idx / nPad,
+                                      listed ? sItem[idx] >> 5 : idx % nPad, nCand, epoch);
+        if (d) atomicAdd(&sOob, d);
+        bound_clear(m, other, nPrev, T - 1 - t, T);
+        nPrev = nCand;
+    }
+    if (t == 0) bcount[BND_PREV_COUNT] = nPrev;
+}
+
+template <int MF>
+__global__ void __launch_bounds__(SMALL_THREADS) k_bnd_small(DevMesh m, DevState A, BndHalf B, int nPasses,
+                                                                   double dt, const double* Sp, const double* Su) {
+    k_bnd_small_body<MF>(m, A, B, nPasses, dt, Sp, Su, A.epoch);
 }
 
 template <int MF>
@@ -2578,19 +2827,42 @@ size_t bound_record_bytes(int maxCellFaces) {
     }
 }
 
+// Meshes whose passes one workgroup takes (knob SVP_BND_SMALL; results do not
+// depend on it): few enough cells that a pass seldom has more candidates than
+// its threads.  Not for cells of more than 8 faces, whose records do not fit
+// the registers next to the other phases' (refined 20^3: 228 us a step against
+// 150 for the separate launches).
+bool bound_small(const DevMesh& m, const DevState& st) {
+    return st.bndFlow && st.maxCellFaces <= NS_CELL_FACES && m.nC <= st.bndSmall;
+}
+
+template <int MF>
+void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
+                        const double* Su, int* passSeq, hipStream_t s) {
+    if constexpr (MF <= NS_CELL_FACES) {
+        if (nPasses > 0 && bound_small(m, st)) {
+            k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
+                                                         bound_half(bound_pass_view(m, st, *passSeq + 1)), nPasses, dt,
+                                                         Sp, Su);
+            *passSeq += nPasses;
+            return;
+        }
+    }
+    for (int pass = 0; pass < nPasses; ++pass) {
+        const int seq = (*passSeq)++;
+        launch_bound_pass<MF>(m, bound_pass_view(m, st, seq), pass, dt, Sp, Su,
+                              bound_prev(bound_pass_view(m, st, seq + 1)), s);
+    }
+}
+
 void launch_bound(const DevMesh& m, const DevState& st, const Params& p, double dt, const double* Sp,
                   const double* Su, int* passSeq, hipStream_t s) {
     const int nPasses = std::min(p.nAlphaBounds, MAX_BOUND_PASSES);
-    for (int pass = 0; pass < nPasses; ++pass) {
-        const int seq = (*passSeq)++;
-        const DevState sp = bound_pass_view(m, st, seq);
-        const BndPrev prev = bound_prev(bound_pass_view(m, st, seq + 1));
-        switch (bound_faces(st.maxCellFaces)) {
-            case 4: launch_bound_pass<4>(m, sp, pass, dt, Sp, Su, prev, s); break;
-            case 6: launch_bound_pass<6>(m, sp, pass, dt, Sp, Su, prev, s); break;
-            case NS_CELL_FACES: launch_bound_pass<NS_CELL_FACES>(m, sp, pass, dt, Sp, Su, prev, s); break;
-            default: launch_bound_pass<MAX_CELL_FACES>(m, sp, pass, dt, Sp, Su, prev, s); break;
-        }
+    switch (bound_faces(st.maxCellFaces)) {
+        case 4: launch_bound_faces<4>(m, st, nPasses, dt, Sp, Su, passSeq, s); break;
+        case 6: launch_bound_faces<6>(m, st, nPasses, dt, Sp, Su, passSeq, s); break;
+        case NS_CELL_FACES: launch_bound_faces<NS_CELL_FACES>(m, st, nPasses, dt, Sp, Su, passSeq, s); break;
+        default: launch_bound_faces<MAX_CELL_FACES>(m, st, nPasses, dt, Sp, Su, passSeq, s); break;
     }
 }
 
@@ -2765,11 +3037,28 @@ __global__ void kb_snap_clip(const BatchCase* __restrict__ bc, const BatchStepIn
     k_snap_clip_body(c.m.nC, st.alpha, snapTol, clip, st);
 }
 
+template <int MF>
+__global__ void __launch_bounds__(SMALL_THREADS) kb_bnd_small(const BatchCase* __restrict__ bc,
+                                                                    const BatchStepInfo* __restrict__ info,
+                                                                    int nPasses) {
+    const BatchCase& c = bc[blockIdx.y];
+    const BatchStepInfo si = info[blockIdx.y];
+    if (!(si.dt > 0.0)) return;
+    k_bnd_small_body<MF>(c.m, batch_view(c, si, 1, 0), bound_half(batch_view(c, si, 1, 1)), nPasses, si.dt, nullptr,
+                         nullptr, si.epoch);
+}
+
 // pass = the pass of the step: its candidate-list half is the case's hPar
 // flipped per pass, and it indexes the pass statistics
 template <int MF>
 static void launch_batch_bound(const BatchCase* bc, const BatchStepInfo* info, int n, int maxListBlocks,
-                               const BatchDims& d, int nPasses, hipStream_t s) {
+                               const BatchDims& d, int nPasses, bool small, hipStream_t s) {
+    if constexpr (MF <= NS_CELL_FACES) {
+        if (small && nPasses > 0) {
+            kb_bnd_small<MF><<<dim3(1, n), SMALL_THREADS, 0, s>>>(bc, info, nPasses);
+            return;
+        }
+    }
     for (int pass = 0; pass < nPasses; ++pass) {
         kb_bnd_list<<<dim3(maxListBlocks, n), 256, 0, s>>>(bc, info, pass);
         kb_bnd_prep<MF><<<dim3(d.prep, n), 256, 0, s>>>(bc, info, pass);
@@ -2780,7 +3069,7 @@ static void launch_batch_bound(const BatchCase* bc, const BatchStepInfo* info, i
 
 void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* info, int n, int maxC, int maxF,
                         int maxDetBlocks, int maxListBlocks, const BatchDims& d, const Params& p, int G, int MF,
-                        int fluxKind, bool fluxListed, hipStream_t s) {
+                        int fluxKind, bool fluxListed, bool bndSmall, hipStream_t s) {
     switch (stage) {
         case STAGE_DETECT:
             kb_detect_list<<<dim3(maxDetBlocks, n), DETECT_LIST_THREADS, 0, s>>>(bc, info, p.mixedCellTol);
@@ -2808,10 +3097,10 @@ void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* inf
         case STAGE_BOUND: {
             const int nPasses = std::min(p.nAlphaBounds, MAX_BOUND_PASSES);
             switch (MF) {
-                case 4: launch_batch_bound<4>(bc, info, n, maxListBlocks, d, nPasses, s); break;
-                case 6: launch_batch_bound<6>(bc, info, n, maxListBlocks, d, nPasses, s); break;
-                case NS_CELL_FACES: launch_batch_bound<NS_CELL_FACES>(bc, info, n, maxListBlocks, d, nPasses, s); break;
-                default: launch_batch_bound<MAX_CELL_FACES>(bc, info, n, maxListBlocks, d, nPasses, s); break;
+                case 4: launch_batch_bound<4>(bc, info, n, maxListBlocks, d, nPasses, bndSmall, s); break;
+                case 6: launch_batch_bound<6>(bc, info, n, maxListBlocks, d, nPasses, bndSmall, s); break;
+                case NS_CELL_FACES: launch_batch_bound<NS_CELL_FACES>(bc, info, n, maxListBlocks, d, nPasses, bndSmall, s); break;
+                default: launch_batch_bound<MAX_CELL_FACES>(bc, info, n, maxListBlocks, d, nPasses, bndSmall, s); break;
             }
             break;
         }

@@ -97,6 +97,7 @@ struct DevState {
     int gridRounds;     // bounding rounds run as grid-wide kernels before the one-workgroup tail
     int bndGrid;        // workgroups of the grid-stride bounding kernels
     int bndFlow;        // workgroups of the one-launch dataflow pass, 0 = rounds and tail
+    int bndSmall;       // cells up to which one workgroup takes all passes
     int bndListWords;   // bitmap words per block of the candidate list (64..4096)
     void* bndRec;       // BndStore<MF> of the active bounding candidates, capacity nC
     int maxCellFaces;
@@ -137,6 +138,10 @@ constexpr int MAX_BOUND_PASSES = 64;
 constexpr int MAX_GRID_ROUNDS = 8;
 constexpr int OOB_SLOTS = 64;   // counters of the out-of-bounds count, one per 64-byte line
 constexpr int OOB_STRIDE = 16;
+
+// meshes whose bounding passes one workgroup takes: on its own, and as a case of
+// a batch (where the other cases fill the chip meanwhile)
+constexpr int BOUND_SMALL_CELLS = 49152, BOUND_SMALL_BATCH_CELLS = 131072;
 
 constexpr int DETECT_BLOCK = 256;
 
@@ -335,6 +340,8 @@ int detect_list_blocks(int nC);   // blocks of the one-launch detection
 int bound_faces(int maxCellFaces);
 size_t bound_record_bytes(int maxCellFaces);
 void launch_count_warped(const DevMesh& m, int* count, hipStream_t s);  // faces below flatness 1 - tSmall
+// whether one workgroup takes all bounding passes of this mesh
+bool bound_small(const DevMesh& m, const DevState& st);
 // the state of bounding pass number seq of a handle: the half (seq & 1) of
 // the double-buffered bounding arrays
 DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
@@ -343,7 +350,7 @@ DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
 // size shared by all cases
 void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC, int maxF,
                         int maxDetBlocks, int maxListBlocks, const BatchDims& d, const Params& p, int G, int MF,
-                        int fluxKind, bool fluxListed, hipStream_t s);
+                        int fluxKind, bool fluxListed, bool bndSmall, hipStream_t s);
 void launch_batch_courant(const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC,
                           unsigned long long* out, hipStream_t s);
 void launch_batch_scale_flow(const BatchCase* bc, const BatchStepInfo* info, const double* factors, int nCases,

@@ -2,7 +2,7 @@
 that leave many cells out of bounds (a random alpha advected with a large
 step), so that a pass has fewer candidates than a workgroup takes, exactly
 about as many, and several workgroups' worth that read one another's
-corrections; with and without sources, under both schedules."""
+corrections; with and without sources, under every schedule."""
 import numpy as np
 import pytest
 
@@ -24,10 +24,12 @@ def case_mesh(kind, N):
                                                    ("hexp", 14, 10, False), ("hex", 20, 3, False), ("tet", 4, 3, True),
                                                    ("tet", 10, 4, False), ("refined", 8, 3, False),
                                                    ("refined", 12, 3, True)])
-@pytest.mark.parametrize("schedule", ["flow", "rounds"])
+@pytest.mark.parametrize("schedule", ["one", "flow", "rounds"])
 def test_bound_every_count(oracle_lib, monkeypatch, kind, N, passes, sources, schedule):
     import geometricvofext_amd as g
     print("bound", kind, N, passes, sources, schedule, flush=True)
+    if schedule != "one":       # "one": a workgroup takes all passes, as on every mesh of these sizes
+        monkeypatch.setenv("SVP_BND_SMALL", "0")
     if schedule == "rounds":
         monkeypatch.setenv("SVP_BND_FLOW", "0")
     mesh = case_mesh(kind, N)
