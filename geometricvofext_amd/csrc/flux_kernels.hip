@@ -174,8 +174,8 @@ __device__ __attribute__((always_inline)) inline double face_flux(const DevMesh&
                                                                   int f, double phi, V3 normal, double distance,
                                                                   double Un0, double dt, bool& ok) {
     const int base = t - c;
-    const int fs = m.facePoints ? f * m.facePoints : m.fOff[f];
-    const int n = m.facePoints ? m.facePoints : m.fOff[f + 1] - fs;
+    int n;
+    const int fs = face_points(m, f, n);
     const double magSf = m.magSf[f];
     const bool moving = fabs(Un0 * dt) > SVP_TSMALL;
     auto swept = [&](int from, int number, int points, const double (&dots)[FP], double full, double mg) {
@@ -270,8 +270,9 @@ __device__ __attribute__((always_inline)) inline void interface_flux_pairs(const
             // the pair's cell and face loaded once, before the needBounding
             // stores (after which reloads of them would wait)
             const int cell = st.mixed[i];
-            const int fb = m.cOff[cell];
-            if (k >= m.cOff[cell + 1] - fb) continue;
+            int nf;
+            const int fb = cell_faces(m, cell, nf);
+            if (k >= nf) continue;
             f = m.cFaces[fb + k];
             ph = st.phi[f];
             const int status = st.status[i];

@@ -319,8 +319,8 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
     for (int wi = blockIdx.x * cells + slot; wi < nWork; wi += gridDim.x * cells) {
         const int i = wl ? wl[wi] : wi;
         const int c = st.mixed[i];
-        const int fb = m.cOff[c], nF = m.cOff[c + 1] - fb;
-        const int pb = m.cpOff[c], np = m.cpOff[c + 1] - pb;
+        int nF, np;
+        const int fb = cell_faces(m, c, nF), pb = cell_points(m, c, np);
         const V3 normalI = ld3(st.ifN, i);
         const double alphaI = st.alpha[c];
         const V3 Cc = ld3(m.C, c);
@@ -348,7 +348,8 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
         int cp[PPL];
 #pragma unroll
         for (int k = 0; k < PPL; ++k) cp[k] = m.cPts[pb + min(l + k * G, np - 1)];
-        const int s0 = m.fOff[fL], fsz = m.fOff[fL + 1] - s0;
+        int fsz;
+        const int s0 = face_points(m, fL, fsz);
         int pl[FP];
 #pragma unroll
         for (int k = 0; k < FP; ++k) pl[k] = m.fPts[s0 + min(k, fsz - 1)];
@@ -567,9 +568,10 @@ __global__ void __launch_bounds__(64, 1) k_un0_group(DevMesh m, DevState st) {
         double un0 = 0.0;
         if (st.status[i] == 0) {
             const int c = st.mixed[i];
-            const int fb = m.cOff[c], nF = m.cOff[c + 1] - fb;
+            int nF, fsz;
+            const int fb = cell_faces(m, c, nF);
             const int fL = m.cFaces[fb + min(l, nF - 1)];
-            const int s0 = m.fOff[fL], fsz = m.fOff[fL + 1] - s0;
+            const int s0 = face_points(m, fL, fsz);
             int pl[FP];
 #pragma unroll
             for (int k = 0; k < FP; ++k) pl[k] = m.fPts[s0 + min(k, fsz - 1)];

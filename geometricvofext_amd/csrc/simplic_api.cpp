@@ -896,6 +896,12 @@ private:
         m_.facePoints = fOff[1];
         for (int f = 0; f < nF; ++f)
             if (fOff[f + 1] - fOff[f] != m_.facePoints) m_.facePoints = 0;
+        m_.cellFaces = cOff[1];
+        m_.cellPoints = cpOff[1];
+        for (int c = 0; c < nC; ++c) {
+            if (cOff[c + 1] - cOff[c] != m_.cellFaces) m_.cellFaces = 0;
+            if (cpOff[c + 1] - cpOff[c] != m_.cellPoints) m_.cellPoints = 0;
+        }
         // point interpolation sources: boundary points -> their non-empty
         // boundary faces (ascending); other points -> their cells (ascending)
         std::vector<std::vector<int>> bFaces(nP);

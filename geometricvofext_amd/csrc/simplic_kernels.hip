@@ -500,7 +500,8 @@ __global__ void __launch_bounds__(64, 1) k_grad_normal(DevMesh m, DevState st) {
         const double ac = st.alpha[c];
         const double Vc = m.V[c];
         V3 g = VZERO;
-        const int b = m.cOff[c], e = m.cOff[c + 1];
+        int nf;
+        const int b = cell_faces(m, c, nf), e = b + nf;
         for (int k0 = b; k0 < e; k0 += FB) {
             int ev[FB];
 #pragma unroll
@@ -1344,7 +1345,8 @@ __device__ __attribute__((always_inline)) inline void k_flux_list_body(const Dev
             const int i = (int)(w / slots), k = (int)(w % slots);
             const int c = st.mixed[i];
             const int status = st.status[i];
-            const int fb = m.cOff[c], nf = m.cOff[c + 1] - fb;
+            int nf;
+            const int fb = cell_faces(m, c, nf);
             if (k < nf) {
                 const int f = m.cFaces[fb + k];
                 entry = make_int2(i, f);
@@ -1402,7 +1404,8 @@ constexpr int UPDATE_BLOCK = 256;
 // per face; larger cells take the face-by-face loop.
 template <int MF>
 __device__ __attribute__((always_inline)) inline double cell_face_sum(const DevMesh& m, const DevState& st, int c) {
-    const int b = m.cOff[c], nf = m.cOff[c + 1] - b;
+    int nf;
+    const int b = cell_faces(m, c, nf);
     double sI = 0.0;
     if (MF > 0 && nf <= MF) {
         constexpr int N = MF > 0 ? MF : 1;
@@ -1572,7 +1575,8 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
     const double Vi = m.V[c];
     const double aOld = st.alphaOld[c];
     const double suC = Su ? Su[c] : 0.0, spC = Sp ? Sp[c] : 0.0;
-    const int b = m.cOff[c], nf = m.cOff[c + 1] - b;
+    int nf;
+    const int b = cell_faces(m, c, nf);
     const double alphaOvershoot = pos0(ac - 1.0) * (ac - 1.0) + neg0(ac) * ac;
     if (fabs(alphaOvershoot) < aTol) return 0;
     const double fluidToPassOn = alphaOvershoot * Vi;
@@ -1850,7 +1854,8 @@ __device__ __attribute__((always_inline)) inline void bound_clear(const DevMesh&
     for (int i = t; i < nPrev; i += nt) {
         if (!prev.active[i]) continue;
         const int c = prev.cand[i];
-        const int fb = m.cOff[c], nf = m.cOff[c + 1] - fb;
+        int nf;
+        const int fb = cell_faces(m, c, nf);
         if (nf <= 8) {
             // the face labels loaded together, then the stores
             int fs[8];
@@ -2397,7 +2402,8 @@ template <int MF>
 __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevMesh& m, const DevState& st, int c,
                                                                       int face, int epoch) {
     const double aTol = 100.0 * SVP_SMALL;
-    const int b = m.cOff[c], nf = m.cOff[c + 1] - b;
+    int nf;
+    const int b = cell_faces(m, c, nf);
     // every load unconditional (slots past nf repeat the last face), in
     // batches: labels; keys; corrections, owners, empty flags, alpha
     int fid[MF], kpos[MF], kon[MF];

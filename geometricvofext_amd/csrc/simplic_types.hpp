@@ -27,7 +27,9 @@ struct DevMesh {
     const int* cPts;
     int maxCellPoints;
     int triQuadFaces;       // 1 when every face has 3 or 4 points
-    int facePoints;         // points of every face when all have the same number, else 0
+    // points of every face, faces and points of every cell when all have the
+    // same number, else 0
+    int facePoints, cellFaces, cellPoints;
     // cell-point-cell stencil: the cell first, then the other cells ascending
     const int* stOff;
     const int* st;
