@@ -1,11 +1,8 @@
 // Harness kernels of the deformation benchmark (plicVofAdvectionFoam) and
 // input checks.
-#include "simplic_device.hpp"
-#include "simplic_types.hpp"
+#include "mesh_device.hpp"
 
 namespace svp {
-
-static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
 // updateU.H:117-127: phi *= uFactor; U *= uFactor
 __device__ inline void scale_flow_at(int i, int nC, int nF, int nB, const double* U0, const double* phi0,
@@ -42,31 +39,59 @@ void launch_scale_flow(int nC, int nF, int nB, const double* U0, const double* p
 
 // fvc::surfaceSum(mag(phi)) in ascending face order, then max of sum/V and of
 // (pos0(alpha-0.01)*pos0(0.99-alpha)*sum)/V.  All values are >= 0, so the max
-// is an integer max over the IEEE bit patterns.  Grid-stride blocks reduce in
-// LDS and issue one atomic pair per block.
-__device__ inline void courant_cell(const DevMesh& m, const double* phi, const double* alpha, int c, double& r,
-                                    double& ra) {
+// is an integer max over the IEEE bit patterns.  A cell of at most MF faces has
+// its labels, then its fluxes, loaded together; larger ones go face by face.
+template <int MF>
+__device__ __attribute__((always_inline)) inline void courant_cell(const DevMesh& m, const double* phi,
+                                                                   const double* alpha, int c, double& r, double& ra) {
+    int nf;
+    const int b = cell_faces(m, c, nf);
+    const double a = alpha[c], V = m.V[c];
     double s = 0.0;
-    for (int k = m.cOff[c]; k < m.cOff[c + 1]; ++k) {
-        const int e = m.cFacesAsc[k];
-        const int f = e >= 0 ? e : ~e;
-        if (f >= m.nIF && m.fEmpty[f]) continue;
-        s += fabs(phi[f]);
+    if (nf <= MF) {
+        int e[MF];
+        double v[MF];
+        unsigned char em[MF];
+#pragma unroll
+        for (int k = 0; k < MF; ++k) e[k] = m.cFacesAsc[b + min(k, nf - 1)];
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            const int f = e[k] >= 0 ? e[k] : ~e[k];
+            v[k] = phi[f];
+            em[k] = m.fEmpty[empty_slot(m, f)];
+            e[k] = f;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < MF; ++k)
+            if (k < nf && !(e[k] >= m.nIF && em[k])) s += fabs(v[k]);
+    } else {
+        for (int k = b; k < b + nf; ++k) {
+            const int e = m.cFacesAsc[k];
+            const int f = e >= 0 ? e : ~e;
+            if (f >= m.nIF && m.fEmpty[f]) continue;
+            s += fabs(phi[f]);
+        }
     }
-    const double a = alpha[c];
-    r = s / m.V[c];
-    ra = (pos0(a - 0.01) * pos0(0.99 - a) * s) / m.V[c];
+    r = s / V;
+    ra = (pos0(a - 0.01) * pos0(0.99 - a) * s) / V;
 }
 
 __device__ inline unsigned long long umax64(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
 
+// The block's two maxima into its own place of out, a host buffer the GPU can
+// reach; the host takes the maximum over the blocks.  Bound by the mesh it
+// streams (133 MB at 128^3 cells, a 26 us copy): 36 us there, 5.4 on 132k
+// tetrahedra.  Two atomic maxima per block on one address took 83 and 17 us,
+// with a launch to clear them (3.7) and a copy back (3) beside; the blocks'
+// atomics queued.
 __device__ __attribute__((always_inline)) inline void k_courant_body(const DevMesh& m, const double* phi,
-                                                                    const double* alpha, unsigned long long* out) {
+                                                                    const double* alpha, ulonglong2* out) {
     __shared__ unsigned long long lr[4], lra[4];
     unsigned long long br = 0ull, bra = 0ull;
     for (int c = blockIdx.x * 256 + threadIdx.x; c < m.nC; c += gridDim.x * 256) {
         double r, ra;
-        courant_cell(m, phi, alpha, c, r, ra);
+        courant_cell<6>(m, phi, alpha, c, r, ra);
         br = umax64(br, (unsigned long long)__double_as_longlong(r));
         bra = umax64(bra, (unsigned long long)__double_as_longlong(ra));
     }
@@ -80,40 +105,39 @@ __device__ __attribute__((always_inline)) inline void k_courant_body(const DevMe
         lra[w] = bra;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        atomicMax(out, umax64(umax64(lr[0], lr[1]), umax64(lr[2], lr[3])));
-        atomicMax(out + 1, umax64(umax64(lra[0], lra[1]), umax64(lra[2], lra[3])));
-    }
+    if (threadIdx.x == 0)
+        out[blockIdx.x] = make_ulonglong2(umax64(umax64(lr[0], lr[1]), umax64(lr[2], lr[3])),
+                                          umax64(umax64(lra[0], lra[1]), umax64(lra[2], lra[3])));
 }
 
-__global__ void __launch_bounds__(256) k_courant(DevMesh m, const double* phi, const double* alpha,
-                                                 unsigned long long* out) {
+__global__ void __launch_bounds__(256) k_courant(DevMesh m, const double* phi, const double* alpha, ulonglong2* out) {
     k_courant_body(m, phi, alpha, out);
 }
 
-// batch: the Courant sums of case blockIdx.y into out[2 y], out[2 y + 1],
-// from its current alpha (view aPar)
+// batch: the blocks' maxima of case blockIdx.y into out[y gridDim.x ...], from
+// its current alpha (view aPar)
 __global__ void __launch_bounds__(256) kb_courant(const BatchCase* __restrict__ bc,
-                                                  const BatchStepInfo* __restrict__ info, unsigned long long* out) {
+                                                  const BatchStepInfo* __restrict__ info, ulonglong2* out) {
     const BatchCase& c = bc[blockIdx.y];
     const DevState& st = c.st[info[blockIdx.y].aPar << 1];
-    k_courant_body(c.m, st.phi, st.alpha, out + 2 * blockIdx.y);
+    k_courant_body(c.m, st.phi, st.alpha, out + (size_t)blockIdx.y * gridDim.x);
 }
 
 __global__ void k_zero_one_int(int* p) {
     if (threadIdx.x == 0) *p = 0;
 }
 
-__global__ void k_zero_u64(unsigned long long* p, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
+// blocks per case: enough to fill the chip; more would only lengthen the list
+// that the host goes through
+constexpr int COURANT_BLOCKS = 1024;
+int courant_blocks(int nCases, int maxC) {
+    return std::min(cdiv(maxC, 256), std::max(COURANT_BLOCKS / nCases, 32));
 }
 
 void launch_courant(const DevMesh& m, const double* phi, const double* alpha, unsigned long long* out,
                     hipStream_t s) {
-    k_zero_u64<<<1, 64, 0, s>>>(out, 2);
-    k_courant<<<std::min(2048, cdiv(m.nC, 256)), 256, 0, s>>>(m, phi, alpha, out);
+    k_courant<<<courant_blocks(1, m.nC), 256, 0, s>>>(m, phi, alpha, (ulonglong2*)out);
 }
-
 
 // ---------------------------------------------------------------------------
 // Initial alpha of a union of spheres / ellipsoids by adaptive tetrahedral
@@ -508,8 +532,7 @@ void launch_count_nonfinite(const double* x, long n, int* count, hipStream_t s) 
 
 void launch_batch_courant(const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC,
                           unsigned long long* out, hipStream_t s) {
-    k_zero_u64<<<cdiv(2L * nCases, 256), 256, 0, s>>>(out, 2 * nCases);
-    kb_courant<<<dim3(std::min(2048, cdiv(maxC, 256)), nCases), 256, 0, s>>>(bc, info, out);
+    kb_courant<<<dim3(courant_blocks(nCases, maxC), nCases), 256, 0, s>>>(bc, info, (ulonglong2*)out);
 }
 
 }  // namespace svp

@@ -29,6 +29,7 @@
 namespace svp {
 void launch_scale_flow(int nC, int nF, int nB, const double* U0, const double* phi0, const double* U0b,
                        double factor, double* U, double* phi, double* Ub, hipStream_t s);
+int courant_blocks(int nCases, int maxC);
 void launch_courant(const DevMesh& m, const double* phi, const double* alpha, unsigned long long* out,
                     hipStream_t s);
 void launch_count_nonfinite(const double* x, long n, int* count, hipStream_t s);
@@ -88,6 +89,31 @@ namespace gve {
 namespace SimPLIC {
 
 using namespace svp;
+
+// Where the Courant kernels leave their blocks' maxima (two bit patterns each):
+// host memory that the GPU writes, one buffer per handle, made by the first call.
+struct CourantMax {
+    unsigned long long* p = nullptr;
+    int blocks = 0;   // per case
+    CourantMax() = default;
+    CourantMax(const CourantMax&) = delete;
+    CourantMax& operator=(const CourantMax&) = delete;
+    ~CourantMax() {
+        if (p) (void)hipHostFree(p);
+    }
+    unsigned long long* need(int nCases, int maxC) {
+        blocks = courant_blocks(nCases, maxC);
+        if (!p) HIPCHECK(hipHostMalloc((void**)&p, 2 * sizeof(unsigned long long) * (size_t)blocks * nCases, 0));
+        return p;
+    }
+    // case k's two maxima, once the stream has been waited for
+    void read(int k, double v[2]) const {
+        unsigned long long r[2] = {0, 0};
+        const unsigned long long* q = p + 2 * (size_t)blocks * k;
+        for (int i = 0; i < 2 * blocks; ++i) r[i & 1] = std::max(r[i & 1], q[i]);
+        std::memcpy(v, r, sizeof r);
+    }
+};
 
 // Host mirror of the reference's solveVofEqu: owns the device mesh, the
 // per-step state and the stream all kernels of this alpha field run on.
@@ -654,7 +680,7 @@ public:
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
     double* U0b_ = nullptr;
-    unsigned long long* courant_ = nullptr;
+    CourantMax courant_;
     int* nonfinite_ = nullptr;
     std::vector<double> hostC_, hostCf_, hostSf_;
     // learned orientation method
@@ -1036,7 +1062,6 @@ private:
         st_.minmax = dalloc<double>(4);
         st_.errFlag = dalloc<int>(1);
         st_.nIcTotal = dalloc<unsigned long long>(1);
-        courant_ = dalloc<unsigned long long>(2);
         nonfinite_ = dalloc<int>(1);
     }
 };
@@ -1138,7 +1163,6 @@ public:
         bc_.upload(host);
         info_.alloc<BatchStepInfo>(n);
         factors_.alloc<double>(n);
-        courant_.alloc<unsigned long long>(2L * n);
         for (int r = 0; r < RING; ++r) {
             HIPCHECK(hipHostMalloc((void**)&ring_[r], sizeof(BatchStepInfo) * n + sizeof(double) * n, 0));
             HIPCHECK(hipEventCreateWithFlags(&ringEv_[r], hipEventDisableTiming));
@@ -1232,15 +1256,12 @@ public:
         const int n = size();
         upload(nullptr, nullptr);
         launch_batch_courant((const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, n, maxC_,
-                             (unsigned long long*)courant_.p, stream_);
+                             courant_.need(n, maxC_), stream_);
         HIPCHECK(hipGetLastError());
-        std::vector<unsigned long long> r(2L * n);
-        HIPCHECK(hipMemcpyAsync(r.data(), courant_.p, sizeof(unsigned long long) * r.size(), hipMemcpyDeviceToHost,
-                                stream_));
         HIPCHECK(hipStreamSynchronize(stream_));
         for (int k = 0; k < n; ++k) {
             double v[2];
-            std::memcpy(v, &r[2L * k], sizeof v);
+            courant_.read(k, v);
             if (co) co[k] = v[0];
             if (aco) aco[k] = v[1];
         }
@@ -1394,7 +1415,8 @@ private:
     // one); rebuilt after the launch shapes change
     bool useGraph_ = true;
     hipGraphExec_t graph_ = nullptr;
-    DBuf bc_, info_, factors_, courant_;
+    DBuf bc_, info_, factors_;
+    gve::SimPLIC::CourantMax courant_;
     char* ring_[RING] = {};
     hipEvent_t ringEv_[RING] = {};
     int ringPos_ = 0;
@@ -2001,12 +2023,12 @@ int svp_harness_init_alpha(svp_handle* h, const double* shapes, int nShapes, int
 int svp_harness_courant(svp_handle* h, double* co, double* aco) {
     return guarded([&] {
         solveVofEqu& s = H(h);
-        svp::launch_courant(s.m_, s.st_.phi, s.st_.alpha, s.courant_, s.stream_);
-        unsigned long long r[2];
-        HIPCHECK(hipMemcpyAsync(r, s.courant_, sizeof r, hipMemcpyDeviceToHost, s.stream_));
+        unsigned long long* out = s.courant_.need(1, s.m_.nC);
+        svp::launch_courant(s.m_, s.st_.phi, s.st_.alpha, out, s.stream_);
+        HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(s.stream_));
         double v[2];
-        std::memcpy(v, r, sizeof v);
+        s.courant_.read(0, v);
         if (co) *co = v[0];
         if (aco) *aco = v[1];
     });
