@@ -182,6 +182,22 @@ struct FaceWalk {
         return ok;
     }
 
+    // the plane's crossings of the cut face alone; false as for subFace
+    __device__ __attribute__((always_inline)) inline bool crossings() {
+        if (FP == 4 || n <= 4) {
+            const CutWalk w = walks[(n == 3 ? 16u : 0u) + mask];
+            nIf = (int)((w.info >> 4) & 15u);
+            listCrossing(w, 0);
+            listCrossing(w, 1);
+            if (nIf > 2) {
+                listCrossing(w, 2);
+                listCrossing(w, 3);
+            }
+            return true;
+        }
+        return walkPoints([](V3) {}, true);
+    }
+
     // centre and area of the cut face (calcSubFaceCentreAndArea,
     // cutFace.C:37-96); false when the plane crosses it more than
     // MAX_IF_POINTS times

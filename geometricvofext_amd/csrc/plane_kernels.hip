@@ -610,4 +610,211 @@ void launch_batch_fsd_group(const BatchCase* bc, const BatchStepInfo* info, int 
     else kb_fsd_group<8, 4><<<dim3(x, n), 64, 0, s>>>(bc, info);
 }
 
+// ---------------------------------------------------------------------------
+// PLIC surface: reconstruction::interface (reconstruction.C:787-835) with
+// cutCell::interfacePoints (cutCell.C:545-608)
+// ---------------------------------------------------------------------------
+// Vector::normalise of OpenFOAM: zero below ROOTVSMALL, else divided by its
+// magnitude component by component
+__device__ inline V3 normalised(V3 v) {
+    const double s = mag(v);
+    return s < SVP_ROOTVSMALL ? VZERO : v / s;
+}
+
+// One wave's LDS: per lane of a wave (a cell face) its points, crossings and
+// interface segments, per group the angles of all its crossings.
+template <int G, int FP>
+struct PlicLds {
+    static constexpr int NG = 64 / G;
+    static constexpr int NX = MAX_IF_POINTS * G;
+    double ps[FP + MAX_IF_POINTS][3][64];
+    double sn[MAX_IF_POINTS - 1][3][64], sc[MAX_IF_POINTS - 1][3][64], sa[MAX_IF_POINTS - 1][64];
+    double ang[NG][NX], sorted[NG][NX];   // crossing order, angle order
+    unsigned char drop[NG][NX];           // angle order: the crossing repeats the one before it
+    CutWalk walk[24];
+};
+
+// The polygon of every mixed cell, its plane cut through the mesh faces again
+// (no warped-face split), as the reference does: the crossings of the cut
+// faces (face order, crossing order) sorted by their angle about the interface
+// centre, in a frame with z along the interface area vector and x towards the
+// first crossing; a crossing whose angle lies within 1e-8 of the previous one
+// in that order is dropped.  The sort is stable, like sortedOrder.
+// Count mode (pts == nullptr): ptOff[i] = polygon size of mixed cell i,
+// faceIdx[i] = 1 if it has a polygon.  Write mode: ptOff and faceIdx hold the
+// exclusive scans of those; the polygon goes to pts[ptOff[i]..], its cell and
+// first point to faceCells / faceOff at faceIdx[i].
+//
+// A lane per cell face, G lanes per cell, as for the plane placement: a lane
+// takes its face's crossings, their angles and their places in the order;
+// neither the cut faces' areas nor the volume are needed.  Bound by its chain
+// of divisions, roots and sums (3.5k hexahedra are 350 waves): 136 -> 10.4 us
+// a launch at 64^3 against one lane per cell with its records in scratch.
+template <int G, int FP>
+__global__ void __launch_bounds__(64, 1) k_plic_group(DevMesh m, DevState st, int nMixed, int* ptOff, int* faceIdx,
+                                                      double* pts, int* faceCells, int* faceOff) {
+    using Lds = PlicLds<G, FP>;
+    constexpr int NG = Lds::NG;
+    constexpr unsigned long long GM = (1ull << G) - 1ull;
+    __shared__ Lds L;
+    const int t = threadIdx.x;
+    if (t < 24) L.walk[t] = kCutWalks.w[t];
+    __syncthreads();
+    const int g = t / G, l = t % G, gb = g * G;
+    if (g >= NG) return;
+    for (int i = blockIdx.x * NG + g; i < nMixed; i += gridDim.x * NG) {
+        const int c = st.mixed[i];
+        int nF, n;
+        const int fb = cell_faces(m, c, nF);
+        const V3 normalI = ld3(st.ifN, i);
+        const double dist = st.ifD[i];
+        const int fL = m.cFaces[fb + min(l, nF - 1)];
+        const int s0 = face_points(m, fL, n);
+        int pl[FP];
+#pragma unroll
+        for (int k = 0; k < FP; ++k) pl[k] = m.fPts[s0 + min(k, n - 1)];
+        V3 q[FP];
+#pragma unroll
+        for (int k = 0; k < FP; ++k) q[k] = ld3(m.pts, pl[k]);
+        double dots[FP];
+#pragma unroll
+        for (int k = 0; k < FP; ++k) {
+            lds3_put(L.ps[k], t, q[k]);
+            dots[k] = dot(q[k], normalI);
+        }
+        int status = 1, nIf = 0;
+        bool ok = true;
+        if (l < nF) {
+            FaceWalk<FP> w(L.ps, L.walk, t, n, dots, dist);
+            status = w.status();
+            if (status == 0) {
+                ok = w.crossings();
+                nIf = w.nIf;
+            }
+        }
+        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
+        const V3 NEG = v3(-0.0, -0.0, -0.0);   // changes no sum
+        if (nIf == 0) {
+            lds3_put(L.ps[FP], t, NEG);
+            lds3_put(L.ps[FP + 1], t, NEG);
+        }
+        const unsigned cut = (unsigned)((__ballot(nIf > 0) >> gb) & GM);
+        const unsigned sub = (unsigned)((__ballot(l < nF && status == -1) >> gb) & GM);
+        const unsigned long long fourAll = __ballot(nIf > 2);
+        const unsigned four = (unsigned)((fourAll >> gb) & GM);
+        const int nX = 2 * (__popc(cut) + __popc(four));
+        __builtin_amdgcn_wave_barrier();
+        // calcInterfaceCentreAndArea (cutCell.C:37-100)
+        V3 fC = VZERO;
+        for (int f = 0; f < nF; ++f) {
+            fC = fC + lds3(L.ps[FP], gb + f) + lds3(L.ps[FP + 1], gb + f);
+            if ((four >> f) & 1u) fC = fC + lds3(L.ps[FP + 2], gb + f) + lds3(L.ps[FP + 3], gb + f);
+        }
+        if (nX > 0) fC = fC / (double)nX;
+        if (nIf == 0) {
+            lds3_put(L.sn[0], t, NEG);
+            lds3_put(L.sc[0], t, NEG);
+            L.sa[0][t] = -0.0;
+        }
+        for (int k = 0; k + 1 < nIf; ++k) {
+            const V3 a = lds3(L.ps[FP + k], t), b = lds3(L.ps[FP + k + 1], t);
+            const V3 nn = cross(b - a, fC - a);
+            const double ar = mag(nn);
+            lds3_put(L.sn[k], t, nn);
+            lds3_put(L.sc[k], t, ar * (a + b + fC));
+            L.sa[k][t] = ar;
+        }
+        __builtin_amdgcn_wave_barrier();
+        V3 sumN = VZERO, sumAc = VZERO;
+        double sumA = 0.0;
+        for (int f = 0; f < nF; ++f) {
+            const int nSeg = ((four >> f) & 1u) ? MAX_IF_POINTS - 1 : 1;
+            for (int k = 0; k < nSeg; ++k) {
+                const V3 nn = lds3(L.sn[k], gb + f);
+                sumN = sumN + flip_if_neg(nn, dot(nn, sumN));
+                sumA += L.sa[k][gb + f];
+                sumAc = sumAc + lds3(L.sc[k], gb + f);
+            }
+        }
+        const bool small = sumA < SVP_ROOTVSMALL;
+        const V3 quot = (1.0 / 3.0) * sumAc / sumA;
+        V3 C = vsel(small, fC, quot), S = vsel(small, VZERO, 0.5 * sumN);
+        if (dot(S, C) < 0.0) S = (-1.0) * S;
+        const double magS = mag(S);
+        const unsigned all = nF >= 32 ? ~0u : ((1u << nF) - 1u);
+        const bool isCut = (cut | sub) != 0u && sub != all && !(magS < SVP_TSMALL) && nX > 0;
+        int out = 0;   // polygon size
+        if (isCut) {
+            const V3 zhat = S / magS;
+            V3 xhat = lds3(L.ps[FP], gb + __ffs((int)cut) - 1) - C;
+            xhat = xhat - dot(xhat, zhat) * zhat;
+            xhat = normalised(xhat);
+            const V3 yhat = normalised(cross(zhat, xhat));
+            const unsigned before = (1u << l) - 1u;
+            const int first = 2 * (__popc(cut & before) + __popc(four & before));   // place of the lane's crossings
+            for (int k = 0; k < nIf; ++k) {
+                const V3 r = lds3(L.ps[FP + k], t) - C;
+                L.ang[g][first + k] = atan2(dot(r, yhat), dot(r, xhat));
+            }
+            __builtin_amdgcn_wave_barrier();
+            int rank[MAX_IF_POINTS];
+#pragma unroll
+            for (int k = 0; k < MAX_IF_POINTS; ++k) {
+                if (k >= nIf) break;
+                const double a = L.ang[g][first + k];
+                int r = 0;
+                for (int j = 0; j < nX; ++j) {
+                    const double b = L.ang[g][j];
+                    r += j < first + k ? !(b > a) : (a > b);
+                }
+                rank[k] = r;
+                L.sorted[g][r] = a;
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < MAX_IF_POINTS; ++k) {
+                if (k >= nIf) break;
+                const int r = rank[k];
+                L.drop[g][r] = r > 0 && !(fabs(L.sorted[g][r] - L.sorted[g][r - 1]) > 1e-8);
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int j = 0; j < nX; ++j) out += !L.drop[g][j];
+            if (pts) {
+                const int o = ptOff[i];
+#pragma unroll
+                for (int k = 0; k < MAX_IF_POINTS; ++k) {
+                    if (k >= nIf || L.drop[g][rank[k]]) continue;
+                    int at = 0;
+                    for (int j = 0; j < rank[k]; ++j) at += !L.drop[g][j];
+                    st3(pts, o + at, lds3(L.ps[FP + k], t));
+                }
+            }
+        }
+        if (l == 0) {
+            if (!pts) {
+                ptOff[i] = out;
+                faceIdx[i] = out > 0 ? 1 : 0;
+            } else if (out > 0) {
+                faceCells[faceIdx[i]] = c;
+                faceOff[faceIdx[i]] = ptOff[i];
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// lanes per cell as for the plane placement of unsplit cells
+void launch_plic_polygons(const DevMesh& m, const DevState& st, int nMixed, int* ptOff, int* faceIdx, double* pts,
+                          int* faceCells, int* faceOff, hipStream_t s) {
+    const int grid = std::min(4 * PLACE_WAVES, cdiv(nMixed, 64 / st.plicGroup));
+    switch (st.plicGroup) {
+        case 4: k_plic_group<4, 4><<<grid, 64, 0, s>>>(m, st, nMixed, ptOff, faceIdx, pts, faceCells, faceOff); break;
+        case 6: k_plic_group<6, 4><<<grid, 64, 0, s>>>(m, st, nMixed, ptOff, faceIdx, pts, faceCells, faceOff); break;
+        case 8: k_plic_group<8, 4><<<grid, 64, 0, s>>>(m, st, nMixed, ptOff, faceIdx, pts, faceCells, faceOff); break;
+        default:
+            k_plic_group<32, MAX_FACE_POINTS><<<grid, 64, 0, s>>>(m, st, nMixed, ptOff, faceIdx, pts, faceCells,
+                                                                  faceOff);
+    }
+}
+
 }  // namespace svp

@@ -1055,9 +1055,9 @@ private:
         st_.bndSmall = BOUND_SMALL_CELLS;
         if (const char* e = std::getenv("SVP_BND_SMALL")) st_.bndSmall = std::atoi(e);
         st_.bndRec = (void*)dalloc<unsigned char>(bound_record_bytes(maxCellFaces_) * (size_t)nC);
-        st_.un0Fused = (!dict_.split_warped_face && maxCellFaces_ <= 8 && m_.maxCellPoints <= NS_CELL_POINTS &&
-                        m_.triQuadFaces) ? 1 : 0;
-        st_.placeGroup = dict_.split_warped_face ? 0 : (st_.un0Fused ? batchGroup() : 32);
+        st_.plicGroup = maxCellFaces_ <= 8 && m_.maxCellPoints <= NS_CELL_POINTS && m_.triQuadFaces ? batchGroup() : 32;
+        st_.placeGroup = dict_.split_warped_face ? 0 : st_.plicGroup;
+        st_.un0Fused = st_.placeGroup > 0 && st_.placeGroup <= 8 ? 1 : 0;
         st_.fsdKeep = rdfNormal_ ? 1 : 0;
         st_.minmax = dalloc<double>(4);
         st_.errFlag = dalloc<int>(1);

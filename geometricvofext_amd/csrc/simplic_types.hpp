@@ -93,6 +93,7 @@ struct DevState {
     unsigned long long* detTicket;  // detection block tickets (grows by the block count per launch)
     unsigned long long* bndTicket;  // candidate-list block tickets (the same)
     int placeGroup;     // lanes per cell of the plane placement: 4, 6, 8 or 32 (0: one lane per cell, split warped faces)
+    int plicGroup;      // lanes per cell of the PLIC polygons: as placeGroup of the unsplit cells
     int un0Fused;       // the plane placement also computes Un0 (groups of 4, 6 and 8)
     int fluxFan;        // face flux with lanes for four fan triangles per face (most faces warped)
     int fsdKeep;        // 1: where findSignedDistance writes no d/C/S they keep their values (isoRDF)
@@ -353,6 +354,9 @@ DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
 void launch_batch_stage(int stage, const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC, int maxF,
                         int maxDetBlocks, int maxListBlocks, const BatchDims& d, const Params& p, int G, int MF,
                         int fluxKind, bool fluxListed, bool bndSmall, hipStream_t s);
+// PLIC polygons of the mixed cells: sizes (pts null) or points
+void launch_plic_polygons(const DevMesh& m, const DevState& st, int nMixed, int* ptOff, int* faceIdx, double* pts,
+                          int* faceCells, int* faceOff, hipStream_t s);
 void launch_batch_courant(const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC,
                           unsigned long long* out, hipStream_t s);
 void launch_batch_scale_flow(const BatchCase* bc, const BatchStepInfo* info, const double* factors, int nCases,
