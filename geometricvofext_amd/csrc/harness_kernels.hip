@@ -519,15 +519,50 @@ void launch_init_alpha_surface(const DevMesh& m, const double* tris, int nT, int
     k_surface_apply<<<cdiv(m.nC, 256), 256, 0, s>>>(m.nC, frac, mode, alpha);
 }
 
-__global__ void k_count_nonfinite(const double* x, long n, int* count) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool bad = (i < n) && !isfinite(x[i]);
-    const unsigned long long b = __ballot(bad);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(count, __popcll(b));
+// Non-finite values of x and of y (empty: ny = 0): every block's two counts
+// into its own place of a host buffer the GPU can reach, as the Courant maxima.
+// One launch and one wait per call, for both arrays: a cleared counter, the
+// count, a copy back and a wait for each took 64 us more on a 64^3 call that
+// sets alpha and the flow (490 -> 427 us with two steps of it).
+__global__ void __launch_bounds__(256) k_count_nonfinite(const double* x, long nx, const double* y, long ny,
+                                                         ulonglong2* out) {
+    __shared__ int lx[4], ly[4];
+    int bx = 0, by = 0;
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < nx; i += gridDim.x * 256L) bx += !isfinite(x[i]);
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < ny; i += gridDim.x * 256L) by += !isfinite(y[i]);
+    for (int o = 32; o > 0; o >>= 1) {
+        bx += __shfl_xor(bx, o);
+        by += __shfl_xor(by, o);
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        lx[w] = bx;
+        ly[w] = by;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        out[blockIdx.x] = make_ulonglong2((unsigned)(lx[0] + lx[1] + lx[2] + lx[3]),
+                                          (unsigned)(ly[0] + ly[1] + ly[2] + ly[3]));
 }
 
-void launch_count_nonfinite(const double* x, long n, int* count, hipStream_t s) {
-    if (n > 0) k_count_nonfinite<<<cdiv(n, 256), 256, 0, s>>>(x, n, count);
+int count_blocks(long n) { return (int)std::min<long>(COURANT_BLOCKS, (n + 255) / 256); }
+
+void launch_count_nonfinite(const double* x, long nx, const double* y, long ny, unsigned long long* out,
+                            hipStream_t s) {
+    k_count_nonfinite<<<count_blocks(std::max(nx, ny)), 256, 0, s>>>(x, nx, y, ny, (ulonglong2*)out);
+}
+
+// the words of a handle's state that host decisions take, to host memory in one go
+__global__ void k_status(const int* err, const int* nMixed, const int* totals, int* out) {
+    if (threadIdx.x != 0) return;
+    out[0] = *err;
+    out[1] = *nMixed;
+    out[2] = totals ? totals[0] : 0;
+    out[3] = totals ? totals[1] : 0;
+}
+
+void launch_status(const DevState& st, const int* totals, int* out, hipStream_t s) {
+    k_status<<<1, 64, 0, s>>>(st.errFlag, st.nMixed, totals, out);
 }
 
 void launch_batch_courant(const BatchCase* bc, const BatchStepInfo* info, int nCases, int maxC,

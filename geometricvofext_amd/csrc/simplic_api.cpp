@@ -32,7 +32,10 @@ void launch_scale_flow(int nC, int nF, int nB, const double* U0, const double* p
 int courant_blocks(int nCases, int maxC);
 void launch_courant(const DevMesh& m, const double* phi, const double* alpha, unsigned long long* out,
                     hipStream_t s);
-void launch_count_nonfinite(const double* x, long n, int* count, hipStream_t s);
+int count_blocks(long n);
+void launch_count_nonfinite(const double* x, long nx, const double* y, long ny, unsigned long long* out,
+                            hipStream_t s);
+void launch_status(const DevState& st, const int* totals, int* out, hipStream_t s);
 void launch_init_alpha(const DevMesh& m, const void* shapes, int nShapes, int maxDepth, double* alpha,
                        hipStream_t s);
 void launch_init_alpha_surface(const DevMesh& m, const double* tris, int nT, int mode, double* frac, int* cutList,
@@ -90,28 +93,29 @@ namespace SimPLIC {
 
 using namespace svp;
 
-// Where the Courant kernels leave their blocks' maxima (two bit patterns each):
-// host memory that the GPU writes, one buffer per handle, made by the first call.
-struct CourantMax {
+// Host memory that kernels write and the host reads after waiting for the
+// stream: two words per block of a reduction, one buffer per handle.
+struct HostOut {
     unsigned long long* p = nullptr;
-    int blocks = 0;   // per case
-    CourantMax() = default;
-    CourantMax(const CourantMax&) = delete;
-    CourantMax& operator=(const CourantMax&) = delete;
-    ~CourantMax() {
+    HostOut() = default;
+    HostOut(const HostOut&) = delete;
+    HostOut& operator=(const HostOut&) = delete;
+    ~HostOut() {
         if (p) (void)hipHostFree(p);
     }
-    unsigned long long* need(int nCases, int maxC) {
-        blocks = courant_blocks(nCases, maxC);
-        if (!p) HIPCHECK(hipHostMalloc((void**)&p, 2 * sizeof(unsigned long long) * (size_t)blocks * nCases, 0));
+    unsigned long long* alloc(size_t blocks) {
+        if (!p) HIPCHECK(hipHostMalloc((void**)&p, 2 * sizeof(unsigned long long) * blocks, 0));
         return p;
     }
-    // case k's two maxima, once the stream has been waited for
-    void read(int k, double v[2]) const {
+    // maxima (of doubles >= 0, as bit patterns) over `blocks` blocks from block `first`
+    void maxima(size_t first, int blocks, double v[2]) const {
         unsigned long long r[2] = {0, 0};
-        const unsigned long long* q = p + 2 * (size_t)blocks * k;
-        for (int i = 0; i < 2 * blocks; ++i) r[i & 1] = std::max(r[i & 1], q[i]);
+        for (size_t i = 2 * first; i < 2 * (first + blocks); ++i) r[i & 1] = std::max(r[i & 1], p[i]);
         std::memcpy(v, r, sizeof r);
+    }
+    void sums(int blocks, unsigned long long v[2]) const {
+        v[0] = v[1] = 0;
+        for (int i = 0; i < 2 * blocks; ++i) v[i & 1] += p[i];
     }
 };
 
@@ -299,10 +303,22 @@ public:
         for (int i = 0; i < N_STAGES; ++i) { profSec_[i] = 0.0; profCnt_[i] = 0; }
     }
 
-    void checkDeviceErrors() {
-        int err = 0;
-        HIPCHECK(hipMemcpyAsync(&err, st_.errFlag, sizeof(int), hipMemcpyDeviceToHost, stream_));
+    // error bits, mixed cells and two totals, as the stream's work so far
+    // leaves them: one launch and one wait
+    struct Status {
+        int err, nMixed, totals[2];
+    };
+    Status readStatus(const int* totals = nullptr) {
+        int* w = (int*)status_.p;
+        launch_status(st_, totals, w, stream_);
+        HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
+        return Status{w[0], w[1], {w[2], w[3]}};
+    }
+    // the same, refused when an error bit is set
+    Status checkDeviceErrors(const int* totals = nullptr) {
+        const Status status = readStatus(totals);
+        const int err = status.err;
         if (err) {
             HIPCHECK(hipMemsetAsync(st_.errFlag, 0, sizeof(int), stream_));
             char buf[256];
@@ -314,11 +330,12 @@ public:
                           err, MAX_IF_POINTS);
             throw SvpError(SVP_E_DEVICE, buf);
         }
+        return status;
     }
 
     void setAlpha(const double* a, int where) {
         copyIn(st_.alpha, a, m_.nC, where);
-        checkFinite(st_.alpha, m_.nC, "alpha");
+        checkFinite(st_.alpha, m_.nC, "alpha", nullptr, 0, nullptr);
         reconstructed_ = false;
     }
     void setFlow(const double* phi, const double* U, const double* Ub, int where) {
@@ -326,8 +343,7 @@ public:
         copyIn(st_.U, U, 3L * m_.nC, where);
         if (Ub) copyIn(st_.Ub, Ub, 3L * nB_, where);
         else HIPCHECK(hipMemsetAsync(st_.Ub, 0, sizeof(double) * 3 * std::max(nB_, 1), stream_));
-        checkFinite(st_.phi, m_.nF, "phi");
-        checkFinite(st_.U, 3L * m_.nC, "U");
+        checkFinite(st_.phi, m_.nF, "phi", st_.U, 3L * m_.nC, "U");
     }
 
     // Host outputs wait for the stream anyway, so their calls also report
@@ -434,8 +450,7 @@ public:
         const bool want = cells || offs || pts;
         if (want && !(cells && offs && pts))
             throw SvpError(SVP_E_ARG, "svp_get_plic_surface: give face_cells, face_offsets and points, or none");
-        checkDeviceErrors();
-        const int k = nMixed();
+        const int k = checkDeviceErrors().nMixed;
         int tot[2] = {0, 0};
         if (k > 0) {
             if (plicIdx_.bytes < sizeof(int) * (2L * k + 2)) plicIdx_.alloc<int>(2L * k + 2);
@@ -444,9 +459,9 @@ public:
             int* totals = faceIdx + k;
             launch_plic_surface(m_, st_, k, 0, ptOff, faceIdx, totals, nullptr, nullptr, nullptr, stream_);
             HIPCHECK(hipGetLastError());
-            HIPCHECK(hipMemcpyAsync(tot, totals, sizeof(tot), hipMemcpyDeviceToHost, stream_));
-            HIPCHECK(hipStreamSynchronize(stream_));
-            checkDeviceErrors();
+            const Status status = checkDeviceErrors(totals);
+            tot[0] = status.totals[0];
+            tot[1] = status.totals[1];
         }
         *nPts = tot[0];
         *nFaces = tot[1];
@@ -467,8 +482,8 @@ public:
             HIPCHECK(hipGetLastError());
         }
         // the closing offset: face_offsets[n_faces] = n_points
-        HIPCHECK(hipMemcpyAsync(dOffs + tot[1], &tot[0], sizeof(int), hipMemcpyHostToDevice, stream_));
-        HIPCHECK(hipStreamSynchronize(stream_));
+        launch_plic_close(dOffs, k > 0 ? (int*)plicIdx_.p + 2L * k : nullptr, stream_);
+        HIPCHECK(hipGetLastError());
         checkDeviceErrors();
         if (where != SVP_DEVICE) {
             copyOut(pts, dPts, 3L * tot[0], SVP_HOST);
@@ -488,8 +503,7 @@ public:
             throw SvpError(SVP_E_ARG,
                            "svp_get_plic_surface_device: give face_cells, face_offsets and points, or none");
         int* ptOff = scratch_address(device_);
-        checkDeviceErrors();
-        const int k = nMixed();
+        const int k = checkDeviceErrors().nMixed;
         if (k > SVP_PLIC_NOALLOC_MAX_CELLS)
             throw SvpError(SVP_E_ARG, "svp_get_plic_surface_device: " + std::to_string(k) +
                                           " mixed cells exceed the scratch of " +
@@ -501,9 +515,9 @@ public:
         if (k > 0) {
             launch_plic_surface(m_, st_, k, 0, ptOff, faceIdx, totals, nullptr, nullptr, nullptr, stream_);
             HIPCHECK(hipGetLastError());
-            HIPCHECK(hipMemcpyAsync(tot, totals, sizeof(tot), hipMemcpyDeviceToHost, stream_));
-            HIPCHECK(hipStreamSynchronize(stream_));
-            checkDeviceErrors();
+            const Status status = checkDeviceErrors(totals);
+            tot[0] = status.totals[0];
+            tot[1] = status.totals[1];
         }
         *nPts = tot[0];
         *nFaces = tot[1];
@@ -511,7 +525,6 @@ public:
         if (k > 0) launch_plic_surface(m_, st_, k, 1, ptOff, faceIdx, nullptr, pts, cells, offs, stream_);
         launch_plic_close(offs, k > 0 ? totals : nullptr, stream_);
         HIPCHECK(hipGetLastError());
-        HIPCHECK(hipStreamSynchronize(stream_));
         checkDeviceErrors();
     }
 
@@ -603,12 +616,7 @@ public:
         }
     }
 
-    int nMixed() {
-        int n = 0;
-        HIPCHECK(hipMemcpyAsync(&n, st_.nMixed, sizeof(int), hipMemcpyDeviceToHost, stream_));
-        HIPCHECK(hipStreamSynchronize(stream_));
-        return n;
-    }
+    int nMixed() { return readStatus().nMixed; }
 
     void timers(double& rec, double& adv, uint64_t& nic) {
         HIPCHECK(hipStreamSynchronize(stream_));
@@ -680,8 +688,8 @@ public:
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
     double* U0b_ = nullptr;
-    CourantMax courant_;
-    int* nonfinite_ = nullptr;
+    HostOut courant_, finite_, status_;   // apart, so that a getter on another thread disturbs none
+    int* nonfinite_ = nullptr;   // count of warped faces
     std::vector<double> hostC_, hostCf_, hostSf_;
     // learned orientation method
     struct {
@@ -719,13 +727,18 @@ public:
                                 stream_));
         if (where != SVP_DEVICE) HIPCHECK(hipStreamSynchronize(stream_));
     }
-    void checkFinite(const double* x, long n, const char* what) {
-        HIPCHECK(hipMemsetAsync(nonfinite_, 0, sizeof(int), stream_));
-        launch_count_nonfinite(x, n, nonfinite_, stream_);
-        int bad = 0;
-        HIPCHECK(hipMemcpyAsync(&bad, nonfinite_, sizeof(int), hipMemcpyDeviceToHost, stream_));
+    // refuses non-finite values of x, then of y
+    void checkFinite(const double* x, long nx, const char* whatX, const double* y, long ny, const char* whatY) {
+        if (nx <= 0 && ny <= 0) return;
+        launch_count_nonfinite(x, nx, y, ny, finite_.p, stream_);
+        HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
-        if (bad) throw SvpError(SVP_E_NAN, std::string(what) + ": " + std::to_string(bad) + " non-finite values");
+        unsigned long long bad[2];
+        finite_.sums(count_blocks(std::max(nx, ny)), bad);
+        for (int k = 0; k < 2; ++k)
+            if (bad[k])
+                throw SvpError(SVP_E_NAN, std::string(k ? whatY : whatX) + ": " + std::to_string(bad[k]) +
+                                              " non-finite values");
     }
     void ensureHostGeometry() {
         if (!hostC_.empty()) return;
@@ -1063,6 +1076,9 @@ private:
         st_.errFlag = dalloc<int>(1);
         st_.nIcTotal = dalloc<unsigned long long>(1);
         nonfinite_ = dalloc<int>(1);
+        courant_.alloc(courant_blocks(1, m_.nC));
+        finite_.alloc(count_blocks(std::max<long>(m_.nF, 3L * m_.nC)));
+        status_.alloc(1);
     }
 };
 
@@ -1255,13 +1271,14 @@ public:
     void courant(double* co, double* aco) {
         const int n = size();
         upload(nullptr, nullptr);
+        const int blocks = courant_blocks(n, maxC_);
         launch_batch_courant((const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, n, maxC_,
-                             courant_.need(n, maxC_), stream_);
+                             courant_.alloc((size_t)blocks * n), stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
         for (int k = 0; k < n; ++k) {
             double v[2];
-            courant_.read(k, v);
+            courant_.maxima((size_t)blocks * k, blocks, v);
             if (co) co[k] = v[0];
             if (aco) aco[k] = v[1];
         }
@@ -1416,7 +1433,7 @@ private:
     bool useGraph_ = true;
     hipGraphExec_t graph_ = nullptr;
     DBuf bc_, info_, factors_;
-    gve::SimPLIC::CourantMax courant_;
+    gve::SimPLIC::HostOut courant_;
     char* ring_[RING] = {};
     hipEvent_t ringEv_[RING] = {};
     int ringPos_ = 0;
@@ -1715,8 +1732,7 @@ int svp_n_mixed(svp_handle* h, int32_t* n) {
     return guarded([&] {
         if (!n) throw SvpError(SVP_E_ARG, "null output");
         solveVofEqu& s = H(h);
-        s.checkDeviceErrors();
-        *n = s.nMixed();
+        *n = s.checkDeviceErrors().nMixed;
     });
 }
 
@@ -1724,8 +1740,7 @@ int svp_get_interface(svp_handle* h, int32_t* cells, int32_t* status, double* n,
                       double* S, int where) {
     return guarded([&] {
         solveVofEqu& s = H(h);
-        s.checkDeviceErrors();
-        const int k = s.nMixed();
+        const int k = s.checkDeviceErrors().nMixed;
         s.copyOutT(cells, s.st_.mixed, k, where);
         s.copyOutT(status, s.st_.status, k, where);
         s.copyOut(n, s.st_.ifN, 3L * k, where);
@@ -1836,7 +1851,6 @@ int svp_profile_get(svp_handle* h, double* seconds, int64_t* counts, int reset) 
 int svp_synchronize(svp_handle* h) {
     return guarded([&] {
         solveVofEqu& s = H(h);
-        HIPCHECK(hipStreamSynchronize(s.stream_));
         s.checkDeviceErrors();
     });
 }
@@ -2023,12 +2037,11 @@ int svp_harness_init_alpha(svp_handle* h, const double* shapes, int nShapes, int
 int svp_harness_courant(svp_handle* h, double* co, double* aco) {
     return guarded([&] {
         solveVofEqu& s = H(h);
-        unsigned long long* out = s.courant_.need(1, s.m_.nC);
-        svp::launch_courant(s.m_, s.st_.phi, s.st_.alpha, out, s.stream_);
+        svp::launch_courant(s.m_, s.st_.phi, s.st_.alpha, s.courant_.p, s.stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(s.stream_));
         double v[2];
-        s.courant_.read(0, v);
+        s.courant_.maxima(0, svp::courant_blocks(1, s.m_.nC), v);
         if (co) *co = v[0];
         if (aco) *aco = v[1];
     });
