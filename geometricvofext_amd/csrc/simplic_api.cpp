@@ -333,9 +333,15 @@ public:
         return status;
     }
 
+    // few candidates seen before a new alpha or flow say nothing about the next step
+    void fieldChanged() {
+        if (*st_.bndHint <= SMALL_CANDS) *st_.bndHint = -1;
+    }
+
     void setAlpha(const double* a, int where) {
         copyIn(st_.alpha, a, m_.nC, where);
         checkFinite(st_.alpha, m_.nC, "alpha", nullptr, 0, nullptr);
+        fieldChanged();
         reconstructed_ = false;
     }
     void setFlow(const double* phi, const double* U, const double* Ub, int where) {
@@ -344,6 +350,7 @@ public:
         if (Ub) copyIn(st_.Ub, Ub, 3L * nB_, where);
         else HIPCHECK(hipMemsetAsync(st_.Ub, 0, sizeof(double) * 3 * std::max(nB_, 1), stream_));
         checkFinite(st_.phi, m_.nF, "phi", st_.U, 3L * m_.nC, "U");
+        fieldChanged();
     }
 
     // Host outputs wait for the stream anyway, so their calls also report
@@ -564,6 +571,7 @@ public:
         freeEvents_.push_back(a);
         freeEvents_.push_back(b);
         checkDeviceErrors();
+        fieldChanged();
         reconstructed_ = false;
     }
 
@@ -1066,7 +1074,7 @@ private:
         // all passes in one workgroup up to this many cells (knob
         // SVP_BND_SMALL; results do not depend on it)
         st_.bndSmall = BOUND_SMALL_CELLS;
-        if (const char* e = std::getenv("SVP_BND_SMALL")) st_.bndSmall = std::atoi(e);
+        if (const char* e = std::getenv("SVP_BND_SMALL")) st_.bndSmall = std::min(std::atoi(e), BOUND_SMALL_CELLS);
         st_.bndRec = (void*)dalloc<unsigned char>(bound_record_bytes(maxCellFaces_) * (size_t)nC);
         st_.plicGroup = maxCellFaces_ <= 8 && m_.maxCellPoints <= NS_CELL_POINTS && m_.triQuadFaces ? batchGroup() : 32;
         st_.placeGroup = dict_.split_warped_face ? 0 : st_.plicGroup;
@@ -1078,7 +1086,10 @@ private:
         nonfinite_ = dalloc<int>(1);
         courant_.alloc(courant_blocks(1, m_.nC));
         finite_.alloc(count_blocks(std::max<long>(m_.nF, 3L * m_.nC)));
-        status_.alloc(1);
+        status_.alloc(2);
+        st_.bndHint = (int*)(status_.p + 2);
+        *st_.bndHint = 0;
+        fieldChanged();
     }
 };
 

@@ -1740,6 +1740,9 @@ __device__ __attribute__((always_inline)) inline void bound_finish(const BndRec<
 // the per-pass counters.
 // candidates of the previous pass, whose leftovers the next list clears
 constexpr int BND_PREV_COUNT = 16;
+// whether one workgroup has taken the step's passes (k_bnd_small), so that the
+// launches queued behind it have nothing to do
+constexpr int BND_HANDLED = 17;
 // any cell out of bounds: sum of the spread counters (each slot is one cache
 // line, so the update kernel's blocks do not queue on a single address)
 __device__ inline bool oob_any(const DevState& st) {
@@ -1851,7 +1854,9 @@ __device__ __attribute__((always_inline)) inline void k_bnd_list_body(const DevM
     }
 }
 
-__global__ void __launch_bounds__(256) k_bnd_list(DevMesh m, DevState st, int nWords, int nBlocks, BndPrev prev) {
+__global__ void __launch_bounds__(256) k_bnd_list(DevMesh m, DevState st, int nWords, int nBlocks, BndPrev prev,
+                                                  int behind) {
+    if (behind && st.bcount[BND_HANDLED]) return;
     k_bnd_list_body(m, st, nWords, nBlocks, prev);
 }
 
@@ -1899,7 +1904,9 @@ __device__ __attribute__((always_inline)) inline void k_bnd_prep_body(const DevM
 }
 
 template <int MF>
-__global__ void __launch_bounds__(256) k_bnd_prep(DevMesh m, DevState st, double dt, const double* Sp, const double* Su) {
+__global__ void __launch_bounds__(256) k_bnd_prep(DevMesh m, DevState st, double dt, const double* Sp, const double* Su,
+                                                  int behind) {
+    if (behind && st.bcount[BND_HANDLED]) return;
     k_bnd_prep_body<MF>(m, st, dt, Sp, Su);
 }
 
@@ -2291,19 +2298,48 @@ __device__ __attribute__((always_inline)) inline void k_bnd_flow_body(const DevM
 }
 
 template <int MF>
-__global__ void __launch_bounds__(flow_threads<MF>()) k_bnd_flow(DevMesh m, DevState st, double dt) {
+__global__ void __launch_bounds__(flow_threads<MF>()) k_bnd_flow(DevMesh m, DevState st, double dt, int behind) {
+    if (behind && st.bcount[BND_HANDLED]) return;
     k_bnd_flow_body<MF>(m, st, dt);
 }
 
+
+// The candidate bitmap: the words of global memory, or one workgroup's copy in
+// LDS.  There a thread's run of 2^sh words lies at a stride of T words, so that the
+// threads' reads of their runs do not meet in a bank.
+struct BndBits {
+    unsigned long long* w;
+    __device__ inline bool get(int c) const {
+        // (an atomic load: the word changes by atomics, past the L1)
+        return (__hip_atomic_load(&w[c >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (c & 63)) & 1ull;
+    }
+    __device__ inline void set(int c, bool on) const {
+        if (on) atomicOr(&w[c >> 6], 1ull << (c & 63));
+        else atomicAnd(&w[c >> 6], ~(1ull << (c & 63)));
+    }
+};
+template <int T>
+struct BndLdsBits {
+    unsigned long long* w;
+    int sh;
+    __device__ inline int at(int word) const { return (word & ((1 << sh) - 1)) * T + (word >> sh); }
+    __device__ inline bool get(int c) const {
+        return (__hip_atomic_load(&w[at(c >> 6)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> (c & 63)) & 1ull;
+    }
+    __device__ inline void set(int c, bool on) const {
+        if (on) atomicOr(&w[at(c >> 6)], 1ull << (c & 63));
+        else atomicAnd(&w[at(c >> 6)], ~(1ull << (c & 63)));
+    }
+};
 
 // alpha of a cell with corrected faces, in correctedFaces order
 // (advectionTemplates.C:164-192), and its candidate bit; returns the change of
 // the out-of-bounds count.  face >= 0: only
 // if that face is the first of the cell's corrected faces in that order, so
 // that of all faces that lead to a cell one applies it.
-template <int MF>
-__device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevMesh& m, const DevState& st, int c,
-                                                                      int face, int epoch) {
+template <int MF, class Bits>
+__device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevMesh& m, const DevState& st,
+                                                                      const Bits& cands, int c, int face, int epoch) {
     const double aTol = 100.0 * SVP_SMALL;
     int nf;
     const int b = cell_faces(m, c, nf);
@@ -2369,22 +2405,15 @@ __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevM
     }
     st.alpha[c] = a;
     const bool candNew = cell_oob(a, aTol) && need_bounding(st, c, epoch);
-    const unsigned long long bit = 1ull << (c & 63);
-    // (an atomic load: the word changes by atomics, past the L1 that a kernel
-    // of several passes would read)
-    const bool candOld = (__hip_atomic_load(&st.candBits[c >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) != 0ull;
-    if (candNew != candOld) {
-        if (candNew) atomicOr(&st.candBits[c >> 6], bit);
-        else atomicAnd(&st.candBits[c >> 6], ~bit);
-    }
+    if (candNew != cands.get(c)) cands.set(c, candNew);
     return (int)loop_oob(a, aTol) - (int)loop_oob(before, aTol);
 }
 
 // slot k of candidate i (k = MF: the candidate's own cell)
-template <int MF>
+template <int MF, class Bits>
 __device__ __attribute__((always_inline)) inline int bound_apply_item(const DevMesh& m, const DevState& st,
-                                                                      const BndStore<MF>& recs, int k, int i,
-                                                                      int nCand, int epoch) {
+                                                                      const Bits& cands, const BndStore<MF>& recs,
+                                                                      int k, int i, int nCand, int epoch) {
     int c = -1, face = -1;
     if (i < nCand && st.active[i]) {
         if (k == MF) {
@@ -2400,7 +2429,7 @@ __device__ __attribute__((always_inline)) inline int bound_apply_item(const DevM
             face = f;
         }
     }
-    return c >= 0 ? bound_apply_cell<MF>(m, st, c, face, epoch) : 0;
+    return c >= 0 ? bound_apply_cell<MF>(m, st, cands, c, face, epoch) : 0;
 }
 
 // The corrections applied: one thread per (candidate, face slot) and one per
@@ -2418,6 +2447,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
     // pass statistics, and the candidate count for the next list's clearing
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st.bcount[BND_PREV_COUNT] = nCand;
+        if (pass == 0) *st.bndHint = nCand;
         if (pass < MAX_BOUND_PASSES && nCand > 0) {
             int nAct = 0;
             for (int r = 0; r <= st.gridRounds; ++r) nAct += st.bcount[3 + r];
@@ -2440,7 +2470,8 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
     // is a multiple of 64, so a wave's lanes leave the loop together
     const long nPad = ((long)nCand + 63) / 64 * 64, total = nPad * (MF + 1);
     for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-        const int dOob = bound_apply_item<MF>(m, st, recs, (int)(idx / nPad), (int)(idx % nPad), nCand, epoch);
+        const int dOob =
+            bound_apply_item<MF>(m, st, BndBits{st.candBits}, recs, (int)(idx / nPad), (int)(idx % nPad), nCand, epoch);
         // one add per wave (a wave's cells lie together)
         const int d = __popcll(__ballot(dOob > 0)) - __popcll(__ballot(dOob < 0));
         if (d && (threadIdx.x & 63) == 0)
@@ -2449,7 +2480,8 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
 }
 
 template <int MF>
-__global__ void __launch_bounds__(256) k_bnd_apply(DevMesh m, DevState st, int pass) {
+__global__ void __launch_bounds__(256) k_bnd_apply(DevMesh m, DevState st, int pass, int behind) {
+    if (behind && st.bcount[BND_HANDLED]) return;
     k_bnd_apply_body<MF>(m, st, pass, st.epoch);
 }
 
@@ -2471,19 +2503,20 @@ __host__ __device__ inline BndHalf bound_half(const DevState& v) {
 // are launch and memory latency (about 25 us a pass with the gaps between
 // them); one workgroup has no look-back, no polling and no idle launches after
 // the last cell is in bounds.  A's halves of the double buffers are those of
-// even passes, B those of odd ones.  Only the candidate bitmap
-// changes by atomics here; its words are read past the L1.
+// even passes, B those of odd ones.  The candidate bitmap is kept in LDS (the
+// update writes all of it anew).
 //
 // 10 passes of about 200 candidates (33^3 perturbed, the default dictionary):
 // 151 us, against 250 us of kernels in 40 launches and the gaps between them; 3
 // passes of 1 to 20 (16^3): 34 us against 61.
 constexpr int SMALL_THREADS = 512;
+constexpr int SMALL_WORDS = BOUND_SMALL_CELLS / 64;
 
 template <int MF>
 __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const DevMesh& m, const DevState& A,
                                                                        const BndHalf& B, int nPasses, double dt,
                                                                        const double* Sp, const double* Su,
-                                                                       int epoch) {
+                                                                       int epoch, bool mayDecline) {
     constexpr int T = SMALL_THREADS, NS = T * MF, NW = T / 64;
     __shared__ unsigned long long sVal[NS + 1];   // corrections of the chunk's cells; the last one 0.0
     __shared__ int sFid[NS];
@@ -2491,10 +2524,15 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
     __shared__ int sWave[NW];
     __shared__ int sOob, sAct, sOpen, sItems;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nWords = (m.nC + 63) / 64, per = (nWords + T - 1) / T;
+    __shared__ unsigned long long sBits[SMALL_WORDS];   // the candidate bitmap
+    const int nWords = (m.nC + 63) / 64;
+    int sh = 0;   // a thread's run of 2^sh words
+    while ((T << sh) < nWords) ++sh;
+    const BndLdsBits<T> cands{sBits, sh};
     const double rDeltaT = 1.0 / dt;
     const BndStore<MF> recs(A.bndRec, m.nC);
     int* bcount = A.bcount;
+    for (int w = t; w < (T << sh); w += T) sBits[cands.at(w)] = w < nWords ? A.candBits[w] : 0ull;
     if (t < 64) {
         int n = A.oobCount[OOB_STRIDE * t];
         static_assert(OOB_SLOTS == 64, "one counter per lane");
@@ -2514,14 +2552,17 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
                             odd ? A.corrPos : B.corrPos, odd ? A.actIdx : B.actIdx};
         __syncthreads();
         if (sOob == 0) {
+            if (t == 0 && pass == 0) {
+                *A.bndHint = 0;
+                bcount[BND_HANDLED] = 1;
+            }
             bound_clear(m, other, nPrev, t, T);
             nPrev = 0;
             break;
         }
         // ascending candidates: every thread its run of words
         int cnt = 0;
-        for (int w = t * per; w < min(nWords, (t + 1) * per); ++w)
-            cnt += __popcll(__hip_atomic_load(&st.candBits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        for (int j = 0; j < (1 << sh); ++j) cnt += __popcll(sBits[j * T + t]);
         int x = cnt;
         for (int o = 1; o < 64; o <<= 1) {
             const int y = __shfl_up(x, o);
@@ -2534,12 +2575,18 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
             off += w < wave ? sWave[w] : 0;
             nCand += sWave[w];
         }
+        if (pass == 0) {
+            if (t == 0) {
+                *A.bndHint = nCand;
+                bcount[BND_HANDLED] = mayDecline && nCand > SMALL_CANDS ? 0 : 1;
+            }
+            if (mayDecline && nCand > SMALL_CANDS) return;
+        }
         if (cnt)
-            for (int w = t * per; w < min(nWords, (t + 1) * per); ++w) {
-                unsigned long long bits =
-                    __hip_atomic_load(&st.candBits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int j = 0; j < (1 << sh); ++j) {
+                unsigned long long bits = sBits[j * T + t];
                 while (bits) {
-                    st.cand[off++] = w * 64 + __ffsll((long long)bits) - 1;
+                    st.cand[off++] = ((t << sh) + j) * 64 + __ffsll((long long)bits) - 1;
                     bits &= bits - 1;
                 }
             }
@@ -2665,7 +2712,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
         const int nPad = (nCand + 63) / 64 * 64, nWork = listed ? sItems : nPad * (MF + 1);
         int d = 0;
         for (int idx = t; idx < nWork; idx += T)
-            d += bound_apply_item<MF>(m, st, recs, listed ? sItem[idx] & 31 : idx / nPad,
+            d += bound_apply_item<MF>(m, st, cands, recs, listed ? sItem[idx] & 31 : idx / nPad,
                                       listed ? sItem[idx] >> 5 : idx % nPad, nCand, epoch);
         if (d) atomicAdd(&sOob, d);
         bound_clear(m, other, nPrev, T - 1 - t, T);
@@ -2676,29 +2723,31 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
 
 template <int MF>
 __global__ void __launch_bounds__(SMALL_THREADS) k_bnd_small(DevMesh m, DevState A, BndHalf B, int nPasses,
-                                                                   double dt, const double* Sp, const double* Su) {
-    k_bnd_small_body<MF>(m, A, B, nPasses, dt, Sp, Su, A.epoch);
+                                                                   double dt, const double* Sp, const double* Su,
+                                                                   int mayDecline) {
+    k_bnd_small_body<MF>(m, A, B, nPasses, dt, Sp, Su, A.epoch, mayDecline != 0);
 }
 
 template <int MF>
 void launch_bound_pass(const DevMesh& m, const DevState& st, int pass, double dt, const double* Sp,
-                       const double* Su, const BndPrev& prev, hipStream_t s) {
+                       const double* Su, const BndPrev& prev, int behind, hipStream_t s) {
     const int nWords = (m.nC + 63) / 64;
     // candidate-sized work: a modest grid-stride grid launches faster than
     // one thread per cell of the mesh
     const int grid = std::max(1, std::min(st.bndGrid, cdiv(m.nC, 256)));
     const int nbw = cdiv(nWords, st.bndListWords);
-    k_bnd_list<<<nbw, 256, 0, s>>>(m, st, nWords, nbw, prev);
-    k_bnd_prep<MF><<<grid, 256, 0, s>>>(m, st, dt, Sp, Su);
+    k_bnd_list<<<nbw, 256, 0, s>>>(m, st, nWords, nbw, prev, behind);
+    k_bnd_prep<MF><<<grid, 256, 0, s>>>(m, st, dt, Sp, Su, behind);
     if (st.bndFlow) {
         k_bnd_flow<MF><<<std::max(1, std::min(st.bndFlow, cdiv(m.nC, flow_chunk<MF>()))), flow_threads<MF>(), 0,
-                         s>>>(m, st, dt);
+                         s>>>(m, st, dt, behind);
     } else {
         k_bnd_scatter<MF><<<grid, 256, 0, s>>>(m, st);
         for (int r = 0; r < st.gridRounds; ++r) k_bnd_round<MF><<<grid, 256, 0, s>>>(m, st, r, dt);
         k_bnd_tail<MF><<<1, TAIL_THREADS, 0, s>>>(m, st, dt);
     }
-    k_bnd_apply<MF><<<std::max(1, std::min(4 * st.bndGrid, cdiv((long)m.nC * (MF + 1), 256))), 256, 0, s>>>(m, st, pass);
+    k_bnd_apply<MF><<<std::max(1, std::min(4 * st.bndGrid, cdiv((long)m.nC * (MF + 1), 256))), 256, 0, s>>>(m, st, pass,
+                                                                                                     behind);
 }
 
 // The state of bounding pass number seq of a handle: its candidate list,
@@ -2736,31 +2785,47 @@ size_t bound_record_bytes(int maxCellFaces) {
     }
 }
 
-// Meshes whose passes one workgroup takes (knob SVP_BND_SMALL; results do not
-// depend on it): few enough cells that a pass seldom has more candidates than
-// its threads.  Not for cells of more than 8 faces, whose records do not fit
-// the registers next to the other phases' (refined 20^3: 228 us a step against
-// 150 for the separate launches).
+// Meshes whose passes one workgroup may take (knob SVP_BND_SMALL; results do
+// not depend on it): those whose candidate bitmap fits its LDS.  Not for cells
+// of more than 8 faces, whose records do not fit the registers next to the
+// other phases' (refined 20^3: 228 us a step against 150 for the separate
+// launches).
 bool bound_small(const DevMesh& m, const DevState& st) {
     return st.bndFlow && st.maxCellFaces <= NS_CELL_FACES && m.nC <= st.bndSmall;
 }
 
+// One workgroup takes a step's passes where they have few candidates.  Three
+// passes of 221, 16 and 3 (64^3): 82 us in one launch, 102 and the gaps between
+// them in twelve (a step 206 us against 228); with the first of them by the
+// separate launches 36 + 42, and the step slower by their gaps (217).  900 (48^3
+// perturbed, 341 us a step against 134) are left to the separate launches.
+// Meshes of up to BOUND_ALWAYS_SMALL_CELLS are not looked at: the launches to
+// fall back on would cost their steps more than a pass of many candidates does.
+// The host goes by the first pass's count that the GPU last reported, which may
+// be a few steps old; only the time depends on it.  Where it was few and may not be
+// any more (a new alpha or flow) the workgroup looks itself, and where it declines the separate launches,
+// queued behind it in any case, do the work.
 template <int MF>
 void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
                         const double* Su, int* passSeq, hipStream_t s) {
+    int behind = 0;
     if constexpr (MF <= NS_CELL_FACES) {
-        if (nPasses > 0 && bound_small(m, st)) {
+        const int last = m.nC <= BOUND_ALWAYS_SMALL_CELLS ? 0 : *(const volatile int*)st.bndHint;
+        if (nPasses > 0 && bound_small(m, st) && last <= SMALL_CANDS) {
+            behind = last < 0;
             k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
                                                          bound_half(bound_pass_view(m, st, *passSeq + 1)), nPasses, dt,
-                                                         Sp, Su);
-            *passSeq += nPasses;
-            return;
+                                                         Sp, Su, behind);
+            if (!behind) {
+                *passSeq += nPasses;
+                return;
+            }
         }
     }
     for (int pass = 0; pass < nPasses; ++pass) {
         const int seq = (*passSeq)++;
         launch_bound_pass<MF>(m, bound_pass_view(m, st, seq), pass, dt, Sp, Su,
-                              bound_prev(bound_pass_view(m, st, seq + 1)), s);
+                              bound_prev(bound_pass_view(m, st, seq + 1)), behind, s);
     }
 }
 
@@ -2954,7 +3019,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) kb_bnd_small(const BatchCase* _
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
     k_bnd_small_body<MF>(c.m, batch_view(c, si, 1, 0), bound_half(batch_view(c, si, 1, 1)), nPasses, si.dt, nullptr,
-                         nullptr, si.epoch);
+                         nullptr, si.epoch, false);
 }
 
 // pass = the pass of the step: its candidate-list half is the case's hPar

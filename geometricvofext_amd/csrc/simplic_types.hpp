@@ -101,6 +101,7 @@ struct DevState {
     int bndGrid;        // workgroups of the grid-stride bounding kernels
     int bndFlow;        // workgroups of the one-launch dataflow pass, 0 = rounds and tail
     int bndSmall;       // cells up to which one workgroup takes all passes
+    int* bndHint;       // host memory: candidates of the last step's first bounding pass, -1 not known
     int bndListWords;   // bitmap words per block of the candidate list (64..4096)
     void* bndRec;       // BndStore<MF> of the active bounding candidates, capacity nC
     int maxCellFaces;
@@ -142,9 +143,11 @@ constexpr int MAX_GRID_ROUNDS = 8;
 constexpr int OOB_SLOTS = 64;   // counters of the out-of-bounds count, one per 64-byte line
 constexpr int OOB_STRIDE = 16;
 
-// meshes whose bounding passes one workgroup takes: on its own, and as a case of
-// a batch (where the other cases fill the chip meanwhile)
-constexpr int BOUND_SMALL_CELLS = 49152, BOUND_SMALL_BATCH_CELLS = 131072;
+// meshes whose bounding passes one workgroup takes: always, where the last step
+// had few candidates, and as a case of a batch (where the other cases fill the
+// chip meanwhile)
+constexpr int BOUND_ALWAYS_SMALL_CELLS = 49152, BOUND_SMALL_CELLS = 524288, BOUND_SMALL_BATCH_CELLS = 131072;
+constexpr int SMALL_CANDS = 512;   // more candidates are left to the separate launches
 
 constexpr int DETECT_BLOCK = 256;
 

@@ -59,3 +59,40 @@ def test_bound_every_count(oracle_lib, monkeypatch, kind, N, passes, sources, sc
         assert bits_equal(gpu.alpha_phi(), ors.alpha_phi()), step
     print("candidates", gpu.bound_stats()[:, 0].tolist(), flush=True)
     gpu.synchronize()
+
+
+@pytest.mark.parametrize("kind,N", [("hexp", 38), ("tet", 21)])
+def test_bound_few_then_many(oracle_lib, kind, N):
+    """A mesh whose passes one workgroup takes or leaves by the candidate count
+    last seen: few, many (unforeseen), few again (unforeseen), and the same
+    after a new alpha or flow, when the workgroup decides itself."""
+    import geometricvofext_amd as g
+    print("bound few then many", kind, N, flush=True)
+    mesh = case_mesh(kind, N)
+    om = oracle_lib.OracleMesh(mesh)
+    rng = np.random.default_rng(N)
+    r = np.linalg.norm(om.C - 0.5, axis=1) * N
+    ball = np.clip(3.5 - r, 0.0, 1.0)      # a few cells' radius
+    noisy = np.clip(ball + (rng.random(mesh.n_cells) < 0.08) * rng.normal(0.0, 0.5, mesh.n_cells), 0.0, 1.0)
+    V = np.array([0.5, -0.4, 0.7])
+    U, phi = np.tile(V, (mesh.n_cells, 1)), om.Sf @ V
+    h = float(np.min(om.V)) ** (1.0 / 3.0)
+    opts = dict(nAlphaBounds=3, clip=False)
+    gpu = g.SolveVofEqu(mesh, dict(orientationMethod="LS", **opts))
+    ors = oracle_lib.OracleSolver(om, threads=8, **opts)
+    seen = []
+    # (a step of 1e-16 moves no cell out of bounds)
+    for k, (alpha, dts) in enumerate([(noisy, (1e-16, 1e-16, 0.9, 0.9, 1e-16, 0.9)), (ball, (0.5, 0.5, 0.2)),
+                                      (noisy, (0.9, 0.9)), (ball, (0.5,))]):
+        for s in (gpu, ors):
+            s.set_alpha(alpha)
+            s.set_flow(phi, U)
+        for j, f in enumerate(dts):
+            for s in (gpu, ors):
+                s.reconstruct()
+                s.advect(f * h)
+            assert bits_equal(gpu.alpha(), ors.alpha()), (k, j)
+            assert bits_equal(gpu.alpha_phi(), ors.alpha_phi()), (k, j)
+            seen.append(int(gpu.bound_stats()[:1, 0].sum()))
+    print("candidates", seen, flush=True)
+    assert min(seen) <= 512 < max(seen)
