@@ -74,4 +74,42 @@ __device__ inline const DevState& batch_view(const BatchCase& c, const BatchStep
     return c.st[((si.aPar ^ swapped) << 1) | (si.hPar ^ (pass & 1))];
 }
 
+// The GPU times of reconstruct and advect, taken by their own kernels: an event
+// record before and after each (four commands that the kernels of a step
+// queue behind) took 14 us of a 125 us step at 16^3 cells, 12 at 64^3 (four
+// steps 888 -> 838 us).  The first kernel of a stage adds up what has
+// ended before it and notes its start; the waves of kernels that may be the
+// last note their end, each in one of CLOCK_SLOTS words, by a maximum that
+// nothing waits for.
+// adds the finished stages to their sums (one wave)
+__device__ inline void stage_fold(const DevState& st, int lane) {
+    for (int k = 0; k < 2; ++k) {
+        unsigned long long end = st.clock[CLOCK_STRIDE + (k * CLOCK_SLOTS + lane) * CLOCK_STRIDE];
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long x = __shfl_xor(end, o);
+            end = x > end ? x : end;
+        }
+        if (lane == 0) {
+            const unsigned long long start = st.clock[k];
+            if (start != 0ull && end > start) st.clock[2 + k] += end - start;
+            st.clock[k] = 0ull;
+        }
+    }
+}
+__device__ inline void stage_start(const DevState& st, int stage, int lane) {
+    const unsigned long long now = wall_clock64();
+    stage_fold(st, lane);
+    if (lane == 0) st.clock[stage] = now;
+}
+// (one lane per wave)
+__device__ inline void stage_stop(const DevState& st, int stage) {
+    const int slot = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (CLOCK_SLOTS - 1);
+    atomicMax(&st.clock[CLOCK_STRIDE + (stage * CLOCK_SLOTS + slot) * CLOCK_STRIDE],
+              (unsigned long long)wall_clock64());
+}
+// the same for a kernel whose workgroups all do the same work: those started last
+__device__ inline void stage_stop_tail(const DevState& st, int stage) {
+    if ((threadIdx.x & 63) == 0 && blockIdx.x + 16 >= gridDim.x) stage_stop(st, stage);
+}
+
 }  // namespace svp

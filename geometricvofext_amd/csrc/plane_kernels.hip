@@ -546,6 +546,7 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
 template <int G, int FP>
 __global__ void __launch_bounds__(64, SVP_FSD_WAVES) k_fsd_group(DevMesh m, DevState st, const int* wl, const int* wn) {
     k_fsd_group_body<G, FP>(m, st, wl, wn);
+    if (threadIdx.x == 0) stage_stop(st, 0);
 }
 
 template <int G, int FP>

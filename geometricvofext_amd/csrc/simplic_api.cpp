@@ -170,8 +170,6 @@ public:
 
     // reconstruction::reconstruct (reconstruction.C:680-722)
     void reconstruct() {
-        hipEvent_t a = event(), b = event();
-        HIPCHECK(hipEventRecord(a, stream_));
         st_.epoch = nextEpoch();
         stage(STAGE_DETECT, [&] { launch_detect(m_, st_, params_, stream_); });
         if (learned_.active) {
@@ -184,9 +182,7 @@ public:
             });
             stage(STAGE_FSD, [&] { placePlanes(); });
         }
-        HIPCHECK(hipEventRecord(b, stream_));
         HIPCHECK(hipGetLastError());
-        pendingRecon_.push_back({a, b});
         reconstructed_ = true;
     }
 
@@ -195,14 +191,10 @@ public:
     void advect(double dt, const double* Sp, const double* Su) {
         if (!(dt > 0.0) || !std::isfinite(dt)) throw SvpError(SVP_E_ARG, "advect: dt must be positive");
         if (!reconstructed_) reconstruct();
-        hipEvent_t a = event(), b = event();
-        HIPCHECK(hipEventRecord(a, stream_));
         std::swap(st_.alpha, st_.alphaOld);
         for (int sg = STAGE_UPWIND; sg <= STAGE_SNAPCLIP; ++sg)
             stage(sg, [&] { launch_advect_stage(sg, m_, st_, params_, dt, Sp, Su, &bndPassSeq_, stream_); });
-        HIPCHECK(hipEventRecord(b, stream_));
         HIPCHECK(hipGetLastError());
-        pendingAdvect_.push_back({a, b});
         lastDt_ = dt;
         alphaPhiValid_ = false;
         reconstructed_ = false;
@@ -627,21 +619,16 @@ public:
     int nMixed() { return readStatus().nMixed; }
 
     void timers(double& rec, double& adv, uint64_t& nic) {
+        // what the kernels of the stages noted (in ticks of the GPU's clock)
+        launch_stage_fold(st_, stream_);
+        HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
-        auto drain = [&](std::vector<std::pair<hipEvent_t, hipEvent_t>>& v, double& acc) {
-            for (auto& e : v) {
-                float ms = 0.f;
-                HIPCHECK(hipEventElapsedTime(&ms, e.first, e.second));
-                acc += 1e-3 * ms;
-                freeEvents_.push_back(e.first);
-                freeEvents_.push_back(e.second);
-            }
-            v.clear();
-        };
-        drain(pendingRecon_, reconTime_);
-        drain(pendingAdvect_, advectTime_);
-        rec = reconTime_;
-        adv = advectTime_;
+        unsigned long long sum[2];
+        HIPCHECK(hipMemcpy(sum, st_.clock + 2, sizeof sum, hipMemcpyDeviceToHost));
+        int rate = 0;   // kHz
+        HIPCHECK(hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, device_));
+        rec = 1e-3 * (double)sum[0] / rate;
+        adv = 1e-3 * (double)sum[1] / rate;
         unsigned long long n = 0;
         HIPCHECK(hipMemcpy(&n, st_.nIcTotal, sizeof(n), hipMemcpyDeviceToHost));
         nic = n;
@@ -764,10 +751,9 @@ public:
 
 private:
     std::vector<std::unique_ptr<DBuf>> bufs_;
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pendingRecon_, pendingAdvect_;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events_;
     std::vector<hipEvent_t> freeEvents_;
-    double reconTime_ = 0.0, advectTime_ = 0.0, mapTime_ = 0.0;
+    double mapTime_ = 0.0;
     bool reconstructed_ = false;
     bool gaussNormal_ = false;  // orientationMethod alphaGrad
     bool pointLinear_ = false;  // alphaGrad with grad(alpha1) Gauss pointLinear
@@ -1082,6 +1068,7 @@ private:
         st_.fsdKeep = rdfNormal_ ? 1 : 0;
         st_.minmax = dalloc<double>(4);
         st_.errFlag = dalloc<int>(1);
+        st_.clock = dalloc<unsigned long long>(STAGE_CLOCK_WORDS);
         st_.nIcTotal = dalloc<unsigned long long>(1);
         nonfinite_ = dalloc<int>(1);
         courant_.alloc(courant_blocks(1, m_.nC));

@@ -317,12 +317,19 @@ __device__ __attribute__((always_inline)) inline void k_detect_list_body(const D
 }
 
 __global__ void __launch_bounds__(DETECT_LIST_THREADS) k_detect_list(DevMesh m, DevState st, double tol, int nBlocks) {
+    if (blockIdx.x == 0) {   // (the body's blocks go by tickets)
+        if (threadIdx.x < 64) stage_start(st, 0, threadIdx.x);
+        return;
+    }
     k_detect_list_body(m, st, tol, nBlocks);
 }
 
+__global__ void __launch_bounds__(64) k_stage_fold(DevState st) { stage_fold(st, threadIdx.x); }
+void launch_stage_fold(const DevState& st, hipStream_t s) { k_stage_fold<<<1, 64, 0, s>>>(st); }
+
 void launch_detect(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s) {
     const int nb = cdiv(m.nC, DETECT_LIST_CELLS);
-    k_detect_list<<<nb, DETECT_LIST_THREADS, 0, s>>>(m, st, p.mixedCellTol, nb);
+    k_detect_list<<<nb + 1, DETECT_LIST_THREADS, 0, s>>>(m, st, p.mixedCellTol, nb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1014,6 +1021,7 @@ __global__ void __launch_bounds__(64) k_find_signed_distance(DevMesh m, DevState
             st3(st.ifS, i, o.wrote ? o.S : VZERO);
         }
     }
+    if (threadIdx.x == 0) stage_stop(st, 0);
 }
 
 // cells whose warped faces are split keep one lane per cell; all others take
@@ -1114,14 +1122,15 @@ void launch_plic_close(int* faceOff, const int* totals, hipStream_t s) {
 // dVf = upwind(phi).flux(alpha)*dt (advectionTemplates.C:371): face value
 // lambda*(aP - aN) + aN with lambda = pos0(phi); zeroGradient boundary value
 // is the owner value; empty patches carry nothing.
-__device__ __attribute__((always_inline)) inline void k_upwind_body(const DevMesh& m, const DevState& st, double dtStep) {
+__device__ __attribute__((always_inline)) inline void k_upwind_body(const DevMesh& m, const DevState& st, double dtStep,
+                                                                   int block) {
     // the out-of-bounds counters of the update and the flux work-list count
     // of the interface flux that follow start at zero
-    if (blockIdx.x == 0) {
+    if (block == 0) {
         for (int k = threadIdx.x; k < OOB_SLOTS * OOB_STRIDE; k += blockDim.x) st.oobCount[k] = 0;
         if (threadIdx.x == 0) *st.fluxCount = 0;
     }
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    const int f = block * blockDim.x + threadIdx.x;
     if (f >= m.nF) return;
     const double dt = dtStep;
     const double ph = st.phi[f];
@@ -1139,7 +1148,11 @@ __device__ __attribute__((always_inline)) inline void k_upwind_body(const DevMes
 }
 
 __global__ void __launch_bounds__(256) k_upwind(DevMesh m, DevState st, double dtStep) {
-    k_upwind_body(m, st, dtStep);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 64) stage_start(st, 1, threadIdx.x);
+        return;
+    }
+    k_upwind_body(m, st, dtStep, blockIdx.x - 1);
 }
 
 
@@ -1385,6 +1398,7 @@ __device__ __attribute__((always_inline)) inline void k_update_body(const DevMes
 template <int MF>
 __global__ void __launch_bounds__(UPDATE_BLOCK) k_update(DevMesh m, DevState st, double dtStep, const double* Sp, const double* Su) {
     k_update_body<MF>(m, st, dtStep, Sp, Su, st.epoch);
+    stage_stop_tail(st, 1);
 }
 
 // face slots of the update's gathered form: the mesh's largest cell when it
@@ -2483,6 +2497,7 @@ template <int MF>
 __global__ void __launch_bounds__(256) k_bnd_apply(DevMesh m, DevState st, int pass, int behind) {
     if (behind && st.bcount[BND_HANDLED]) return;
     k_bnd_apply_body<MF>(m, st, pass, st.epoch);
+    if ((threadIdx.x & 63) == 0) stage_stop(st, 1);
 }
 
 // one half of the bounding double buffers
@@ -2726,6 +2741,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_bnd_small(DevMesh m, DevState
                                                                    double dt, const double* Sp, const double* Su,
                                                                    int mayDecline) {
     k_bnd_small_body<MF>(m, A, B, nPasses, dt, Sp, Su, A.epoch, mayDecline != 0);
+    if (threadIdx.x == 0) stage_stop(A, 1);
 }
 
 template <int MF>
@@ -2852,6 +2868,7 @@ __device__ __attribute__((always_inline)) inline void k_snap_clip_body(int nC, d
 
 __global__ void k_snap_clip(int nC, double* alpha, double snapTol, int clip, DevState st) {
     k_snap_clip_body(nC, alpha, snapTol, clip, st);
+    stage_stop_tail(st, 1);
 }
 
 __global__ void k_zero_int(int* p, int n) {
@@ -2862,7 +2879,7 @@ void launch_advect_stage(int stage, const DevMesh& m, const DevState& st, const 
                          const double* Sp, const double* Su, int* passSeq, hipStream_t s) {
     switch (stage) {
         case STAGE_UPWIND:
-            k_upwind<<<cdiv(m.nF, 256), 256, 0, s>>>(m, st, dt);
+            k_upwind<<<cdiv(m.nF, 256) + 1, 256, 0, s>>>(m, st, dt);
             break;
         case STAGE_IFLUX:
             if (!st.placeGroup) k_un0<<<512, 64, 0, s>>>(m, st);
@@ -2944,7 +2961,7 @@ __global__ void __launch_bounds__(256) kb_upwind(const BatchCase* __restrict__ b
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_upwind_body(c.m, batch_view(c, si, 1, 0), si.dt);
+    k_upwind_body(c.m, batch_view(c, si, 1, 0), si.dt, blockIdx.x);
 }
 
 __global__ void __launch_bounds__(256) kb_flux_list(const BatchCase* __restrict__ bc,

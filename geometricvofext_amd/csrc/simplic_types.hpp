@@ -107,6 +107,7 @@ struct DevState {
     int maxCellFaces;
     double* minmax;     // [4]: min, max before bounding, min, max after
     int* errFlag;       // [1] device error bits
+    unsigned long long* clock;  // [STAGE_CLOCK_WORDS] GPU times of reconstruct and advect (stage_start, stage_stop)
     unsigned long long* nIcTotal;  // [1] running sum of mixed-cell counts
 };
 
@@ -142,6 +143,10 @@ constexpr int MAX_BOUND_PASSES = 64;
 constexpr int MAX_GRID_ROUNDS = 8;
 constexpr int OOB_SLOTS = 64;   // counters of the out-of-bounds count, one per 64-byte line
 constexpr int OOB_STRIDE = 16;
+// GPU clock of reconstruct (0) and advect (1): starts, sums, then per stage
+// CLOCK_SLOTS end times, one per 64-byte line
+constexpr int CLOCK_SLOTS = 64, CLOCK_STRIDE = 8;
+constexpr int STAGE_CLOCK_WORDS = CLOCK_STRIDE + 2 * CLOCK_SLOTS * CLOCK_STRIDE;
 
 // meshes whose bounding passes one workgroup takes: always, where the last step
 // had few candidates, and as a case of a batch (where the other cases fill the
@@ -263,6 +268,7 @@ struct BatchDims {
 
 // launchers (simplic_kernels.hip)
 void launch_geometry(const DevMesh& m, hipStream_t s);
+void launch_stage_fold(const DevState& st, hipStream_t s);
 void launch_detect(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s);
 // wl/wn: optional device list of mixed-cell positions and its length
 void launch_ls_normal(const DevMesh& m, const DevState& st, hipStream_t s, const int* wl = nullptr,
