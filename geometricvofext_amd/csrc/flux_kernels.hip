@@ -278,7 +278,7 @@ __device__ __attribute__((always_inline)) inline void interface_flux_pairs(const
             const int status = st.status[i];
             const int fo = m.own[f];
             const int fn = f < m.nIF ? m.nbr[f] : -1;
-            const unsigned char em = m.fEmpty[empty_slot(m, f)];
+            const unsigned char em = empty_flag(m, f);
             if (c == 0) {
                 if (k == 0) st.nbTag[cell] = epoch;
                 if (f < m.nIF) st.nbTag[fo == cell ? fn : fo] = epoch;
@@ -333,8 +333,9 @@ __global__ void __launch_bounds__(64, FP > 4 ? 2 : SVP_FLUX_WAVES) kb_interface_
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    const DevState& st = batch_view(c, si, 1, 0);
-    k_interface_flux_body<FG, FP, LISTED>(c.m, st, si.dt, st.maxCellFaces, si.epoch);
+    const DevMesh m = c.m;
+    const DevState st = batch_view(c, si, 1, 0);
+    k_interface_flux_body<FG, FP, LISTED>(m, st, si.dt, st.maxCellFaces, si.epoch);
 }
 
 // lanes per face, by the mesh: triangles only (and cells of at most 4 faces,

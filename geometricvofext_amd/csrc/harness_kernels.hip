@@ -20,8 +20,9 @@ __global__ void k_scale_flow(int nC, int nF, int nB, const double* U0, const dou
 // batch: every case's base flow scaled by its own factor (blockIdx.y = case)
 __global__ void kb_scale_flow(const BatchCase* __restrict__ bc, const double* __restrict__ factors) {
     const BatchCase& c = bc[blockIdx.y];
+    const DevMesh m = c.m;
     const DevState& st = c.st[0];
-    scale_flow_at(blockIdx.x * blockDim.x + threadIdx.x, c.m.nC, c.m.nF, c.nB, c.U0, c.phi0, c.U0b,
+    scale_flow_at(blockIdx.x * blockDim.x + threadIdx.x, m.nC, m.nF, c.nB, c.U0, c.phi0, c.U0b,
                   factors[blockIdx.y], st.U, st.phi, st.Ub);
 }
 
@@ -58,9 +59,9 @@ __device__ __attribute__((always_inline)) inline void courant_cell(const DevMesh
         for (int k = 0; k < MF; ++k) {
             const int f = e[k] >= 0 ? e[k] : ~e[k];
             v[k] = phi[f];
-            em[k] = m.fEmpty[empty_slot(m, f)];
             e[k] = f;
         }
+        empty_flags(m, e, em);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < MF; ++k)
@@ -81,7 +82,7 @@ __device__ inline unsigned long long umax64(unsigned long long a, unsigned long 
 
 // The block's two maxima into its own place of out, a host buffer the GPU can
 // reach; the host takes the maximum over the blocks.  Bound by the mesh it
-// streams (133 MB at 128^3 cells, a 26 us copy): 36 us there, 5.4 on 132k
+// streams (133 MB at 128^3 cells, a 26 us copy): 31 us there, 5.0 on 132k
 // tetrahedra.  Two atomic maxima per block on one address took 83 and 17 us,
 // with a launch to clear them (3.7) and a copy back (3) beside; the blocks'
 // atomics queued.
@@ -119,8 +120,9 @@ __global__ void __launch_bounds__(256) k_courant(DevMesh m, const double* phi, c
 __global__ void __launch_bounds__(256) kb_courant(const BatchCase* __restrict__ bc,
                                                   const BatchStepInfo* __restrict__ info, ulonglong2* out) {
     const BatchCase& c = bc[blockIdx.y];
+    const DevMesh m = c.m;
     const DevState& st = c.st[info[blockIdx.y].aPar << 1];
-    k_courant_body(c.m, st.phi, st.alpha, out + (size_t)blockIdx.y * gridDim.x);
+    k_courant_body(m, st.phi, st.alpha, out + (size_t)blockIdx.y * gridDim.x);
 }
 
 __global__ void k_zero_one_int(int* p) {

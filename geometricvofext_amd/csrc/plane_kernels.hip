@@ -555,7 +555,8 @@ __global__ void __launch_bounds__(64, SVP_FSD_WAVES) kb_fsd_group(const BatchCas
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_fsd_group_body<G, FP>(c.m, batch_view(c, si, 0, 0), nullptr, nullptr);
+    const DevMesh m = c.m;
+    k_fsd_group_body<G, FP>(m, batch_view(c, si, 0, 0), nullptr, nullptr);
 }
 
 // Un0 of every mixed cell by the same lane groups, where the plane placement

@@ -963,9 +963,14 @@ private:
         m_.own = dupload(own);
         m_.nbr = dupload(nbr);
         m_.fEmpty = dupload(fEmpty);
+        m_.hasEmpty = std::count(fEmpty.begin(), fEmpty.end(), 0) < (long)nF ? 1 : 0;
         m_.cOff = dupload(cOff);
         m_.cFaces = dupload(cFaces);
         m_.cFacesAsc = dupload(cFacesAsc);
+        std::vector<int> cFacesSgn(cFaces.size());
+        for (int c = 0; c < nC; ++c)
+            for (int k = cOff[c]; k < cOff[c + 1]; ++k) cFacesSgn[k] = own[cFaces[k]] == c ? cFaces[k] : ~cFaces[k];
+        m_.cFacesSgn = dupload(cFacesSgn);
         m_.stOff = dupload(stOff);
         m_.st = dupload(st);
         m_.psOff = dupload(psOff);

@@ -1254,18 +1254,19 @@ __device__ __attribute__((always_inline)) inline void k_flux_list_body(const Dev
             int nf;
             const int fb = cell_faces(m, c, nf);
             if (k < nf) {
-                const int f = m.cFaces[fb + k];
+                const int e = m.cFacesSgn[fb + k];
+                const bool own = e >= 0;
+                const int f = own ? e : ~e;
                 entry = make_int2(i, f);
-                const int fo = m.own[f];
-                const int fn = f < m.nIF ? m.nbr[f] : -1;
+                const int other = (own ? m.nbr : m.own)[f];
                 const double ph = st.phi[f];
-                const unsigned char em = m.fEmpty[empty_slot(m, f)];
+                const unsigned char em = empty_flag(m, f);
                 // needBounding: the cell (slot 0) and its neighbour across
                 // each internal face
                 if (k == 0) st.nbTag[c] = epoch;
-                if (f < m.nIF) st.nbTag[fo == c ? fn : fo] = epoch;
+                if (f < m.nIF) st.nbTag[other] = epoch;
                 if (status == 0) {
-                    if (f < m.nIF) take = (fo == c) ? (ph >= 0.0) : (ph < 0.0);
+                    if (f < m.nIF) take = own ? (ph >= 0.0) : (ph < 0.0);
                     else take = !em && (ph >= 0.0);
                 }
             }
@@ -1325,7 +1326,7 @@ __device__ __attribute__((always_inline)) inline double cell_face_sum(const DevM
     double sI = 0.0;
     if (MF > 0 && nf <= MF) {
         constexpr int N = MF > 0 ? MF : 1;
-        int e[N];
+        int e[N], f[N];
         double v[N];
         unsigned char em[N];
 #pragma unroll
@@ -1336,10 +1337,10 @@ __device__ __attribute__((always_inline)) inline double cell_face_sum(const DevM
         // that every thread shares, instead of a line per face.
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            const int f = e[k] >= 0 ? e[k] : ~e[k];
-            v[k] = st.dVf[f];
-            em[k] = m.fEmpty[empty_slot(m, f)];
+            f[k] = e[k] >= 0 ? e[k] : ~e[k];
+            v[k] = st.dVf[f[k]];
         }
+        empty_flags(m, f, em);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
@@ -1506,20 +1507,21 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
     for (int w = 0; w < (MF + 7) / 8; ++w) flg[w] = 0u;
     // all face loads first, unconditional (slots past nf repeat the last
     // face), so they are in flight together instead of one face at a time
-    int fo[MF], fn[MF];
+    int fo[MF];   // across the face
+    bool own[MF];
     double fph[MF], fdv[MF];
     unsigned char fem[MF];
 #pragma unroll
-    for (int k = 0; k < MF; ++k) fid[k] = m.cFaces[b + min(k, nf - 1)];
+    for (int k = 0; k < MF; ++k) fid[k] = m.cFacesSgn[b + min(k, nf - 1)];
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
-        const int f = fid[k];
-        fo[k] = m.own[f];
-        fn[k] = m.nbr[f];
-        fph[k] = st.phi[f];
-        fdv[k] = st.dVf[f];
-        fem[k] = m.fEmpty[empty_slot(m, f)];
+        own[k] = fid[k] >= 0;
+        fid[k] = own[k] ? fid[k] : ~fid[k];
+        fo[k] = (own[k] ? m.nbr : m.own)[fid[k]];
+        fph[k] = st.phi[fid[k]];
+        fdv[k] = st.dVf[fid[k]];
     }
+    empty_flags(m, fid, fem);
     __builtin_amdgcn_sched_barrier(0);
     const OverTol tol = over_tol(Vi, aTol);
     bool near = false;
@@ -1531,18 +1533,17 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
         smax[k] = 0.0;
         if (k < nf) {
             const int f = fid[k];
-            const bool own = (fo[k] == c);
-            if (f < m.nIF) oth[k] = own ? fn[k] : fo[k];
+            if (f < m.nIF) oth[k] = fo[k];
             // face_value: empty-patch faces carry nothing
             const bool live = (f < m.nIF) || !fem[k];
             const double ph = live ? fph[k] : 0.0;
             const double dv = live ? fdv[k] : 0.0;
             phdt[k] = ph * dt + 0.0;   // (never -0: its sign bit is sgn(phi))
             dvf[k] = dv;
-            const bool down = own ? (ph >= 0) : (ph < 0);
+            const bool down = own[k] ? (ph >= 0) : (ph < 0);
             const bool writable = live;
             const bool lowerWriter = oth[k] >= 0 && !down && oth[k] < c;
-            flg[k >> 3] |= ((own ? 1u : 0u) | (down ? 2u : 0u) | (writable ? 4u : 0u) | (lowerWriter ? 8u : 0u))
+            flg[k >> 3] |= ((own[k] ? 1u : 0u) | (down ? 2u : 0u) | (writable ? 4u : 0u) | (lowerWriter ? 8u : 0u))
                            << (4 * (k & 7));
             if (down) {
                 const double dVff = dv + 0.0;
@@ -2358,14 +2359,19 @@ __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevM
     int nf;
     const int b = cell_faces(m, c, nf);
     // every load unconditional (slots past nf repeat the last face), in
-    // batches: labels; keys; corrections, owners, empty flags, alpha
-    int fid[MF], kpos[MF], kon[MF];
+    // batches: labels; keys; corrections, alpha
+    int fid[MF], kpos[MF];
     double kval[MF];
+    bool kown[MF];
     unsigned char kem[MF];
 #pragma unroll
-    for (int k = 0; k < MF; ++k) fid[k] = m.cFaces[b + min(k, nf - 1)];
+    for (int k = 0; k < MF; ++k) fid[k] = m.cFacesSgn[b + min(k, nf - 1)];
 #pragma unroll
-    for (int k = 0; k < MF; ++k) kpos[k] = st.corrPos[fid[k]];
+    for (int k = 0; k < MF; ++k) {
+        kown[k] = fid[k] >= 0;
+        fid[k] = kown[k] ? fid[k] : ~fid[k];
+        kpos[k] = st.corrPos[fid[k]];
+    }
     if (face >= 0) {
         int bpos = 0x7fffffff, bf = -1;
 #pragma unroll
@@ -2377,21 +2383,16 @@ __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevM
         if (bf != face) return 0;
     }
 #pragma unroll
-    for (int k = 0; k < MF; ++k) {
-        kval[k] = st.corr[fid[k]];
-        kon[k] = m.own[fid[k]];
-        kem[k] = m.fEmpty[empty_slot(m, fid[k])];
-    }
+    for (int k = 0; k < MF; ++k) kval[k] = st.corr[fid[k]];
+    empty_flags(m, fid, kem);
     const double before = st.alpha[c];
     const double Vc = m.V[c];
     __builtin_amdgcn_sched_barrier(0);
-    bool kown[MF];
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
         if (k >= nf) kpos[k] = -1;
         // face_value: empty-patch faces carry nothing
         kval[k] = (kpos[k] >= 0 && (fid[k] < m.nIF || !kem[k])) ? kval[k] : 0.0;
-        kown[k] = kpos[k] >= 0 && kon[k] == c;
     }
     double a = before;
     // corrections in ascending correctedFaces position (selection over
@@ -2436,7 +2437,7 @@ __device__ __attribute__((always_inline)) inline int bound_apply_item(const DevM
             const int f = recs.fid(k, i), o = recs.oth(k, i);
             // face_value of both: empty-patch faces keep theirs
             const double dv = st.dVf[f], cr = st.corr[f];
-            const unsigned char em = m.fEmpty[empty_slot(m, f)];
+            const unsigned char em = empty_flag(m, f);
             const bool other = o >= 0 && st.actIdx[max(o, 0)] < 0;
             if (f < m.nIF || !em) st.dVf[f] = dv + cr;
             c = other ? o : -1;
@@ -2949,7 +2950,8 @@ __global__ void __launch_bounds__(DETECT_LIST_THREADS) kb_detect_list(const Batc
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0) || (int)blockIdx.x >= c.detBlocks) return;
-    k_detect_list_body(c.m, batch_view(c, si, 0, 0), tol, c.detBlocks);
+    const DevMesh m = c.m;
+    k_detect_list_body(m, batch_view(c, si, 0, 0), tol, c.detBlocks);
 }
 
 __global__ void __launch_bounds__(64, 1) kb_ls_normal(const BatchCase* __restrict__ bc,
@@ -2957,7 +2959,8 @@ __global__ void __launch_bounds__(64, 1) kb_ls_normal(const BatchCase* __restric
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_ls_normal_body(c.m, batch_view(c, si, 0, 0), nullptr, nullptr);
+    const DevMesh m = c.m;
+    k_ls_normal_body(m, batch_view(c, si, 0, 0), nullptr, nullptr);
 }
 
 __global__ void __launch_bounds__(256) kb_upwind(const BatchCase* __restrict__ bc,
@@ -2965,9 +2968,10 @@ __global__ void __launch_bounds__(256) kb_upwind(const BatchCase* __restrict__ b
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    const DevState& st = batch_view(c, si, 1, 0);
+    const DevMesh m = c.m;
+    const DevState st = batch_view(c, si, 1, 0);
     if (blockIdx.x == 0 && threadIdx.x == 0) *st.fluxCount = 0;   // of the list kernel that follows
-    k_upwind_body(c.m, st, si.dt, blockIdx.x);
+    k_upwind_body(m, st, si.dt, blockIdx.x);
 }
 
 __global__ void __launch_bounds__(256) kb_flux_list(const BatchCase* __restrict__ bc,
@@ -2975,8 +2979,9 @@ __global__ void __launch_bounds__(256) kb_flux_list(const BatchCase* __restrict_
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    const DevState& st = batch_view(c, si, 1, 0);
-    k_flux_list_body(c.m, st, st.maxCellFaces, si.epoch, blockIdx.x, gridDim.x);
+    const DevMesh m = c.m;
+    const DevState st = batch_view(c, si, 1, 0);
+    k_flux_list_body(m, st, st.maxCellFaces, si.epoch, blockIdx.x, gridDim.x);
 }
 
 template <int MF>
@@ -2985,7 +2990,8 @@ __global__ void __launch_bounds__(UPDATE_BLOCK) kb_update(const BatchCase* __res
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_update_body<MF>(c.m, batch_view(c, si, 1, 0), si.dt, nullptr, nullptr, si.epoch);
+    const DevMesh m = c.m;
+    k_update_body<MF>(m, batch_view(c, si, 1, 0), si.dt, nullptr, nullptr, si.epoch);
 }
 
 __global__ void __launch_bounds__(256) kb_bnd_list(const BatchCase* __restrict__ bc,
@@ -2993,9 +2999,10 @@ __global__ void __launch_bounds__(256) kb_bnd_list(const BatchCase* __restrict__
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0) || (int)blockIdx.x >= c.listBlocks) return;
-    const DevState& o = batch_view(c, si, 1, pass + 1);
+    const DevMesh m = c.m;
+    const DevState o = batch_view(c, si, 1, pass + 1);
     const BndPrev prev{o.cand, o.active, o.corr, o.corrPos, o.actIdx};
-    k_bnd_list_body(c.m, batch_view(c, si, 1, pass), c.listWords, c.listBlocks, prev);
+    k_bnd_list_body(m, batch_view(c, si, 1, pass), c.listWords, c.listBlocks, prev);
 }
 
 template <int MF>
@@ -3004,7 +3011,8 @@ __global__ void __launch_bounds__(256) kb_bnd_prep(const BatchCase* __restrict__
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_bnd_prep_body<MF>(c.m, batch_view(c, si, 1, pass), si.dt, nullptr, nullptr);
+    const DevMesh m = c.m;
+    k_bnd_prep_body<MF>(m, batch_view(c, si, 1, pass), si.dt, nullptr, nullptr);
 }
 
 template <int MF>
@@ -3013,7 +3021,8 @@ __global__ void __launch_bounds__(flow_threads<MF>()) kb_bnd_flow(const BatchCas
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_bnd_flow_body<MF>(c.m, batch_view(c, si, 1, pass), si.dt);
+    const DevMesh m = c.m;
+    k_bnd_flow_body<MF>(m, batch_view(c, si, 1, pass), si.dt);
 }
 
 template <int MF>
@@ -3022,7 +3031,8 @@ __global__ void __launch_bounds__(256) kb_bnd_apply(const BatchCase* __restrict_
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_bnd_apply_body<MF>(c.m, batch_view(c, si, 1, pass), pass, si.epoch);
+    const DevMesh m = c.m;
+    k_bnd_apply_body<MF>(m, batch_view(c, si, 1, pass), pass, si.epoch);
 }
 
 __global__ void kb_snap_clip(const BatchCase* __restrict__ bc, const BatchStepInfo* __restrict__ info,
@@ -3030,8 +3040,9 @@ __global__ void kb_snap_clip(const BatchCase* __restrict__ bc, const BatchStepIn
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    const DevState& st = batch_view(c, si, 1, 0);
-    k_snap_clip_body(c.m.nC, st.alpha, snapTol, clip, st);
+    const DevMesh m = c.m;
+    const DevState st = batch_view(c, si, 1, 0);
+    k_snap_clip_body(m.nC, st.alpha, snapTol, clip, st);
 }
 
 template <int MF>
@@ -3041,7 +3052,8 @@ __global__ void __launch_bounds__(SMALL_THREADS) kb_bnd_small(const BatchCase* _
     const BatchCase& c = bc[blockIdx.y];
     const BatchStepInfo si = info[blockIdx.y];
     if (!(si.dt > 0.0)) return;
-    k_bnd_small_body<MF>(c.m, batch_view(c, si, 1, 0), bound_half(batch_view(c, si, 1, 1)), nPasses, si.dt, nullptr,
+    const DevMesh m = c.m;
+    k_bnd_small_body<MF>(m, batch_view(c, si, 1, 0), bound_half(batch_view(c, si, 1, 1)), nPasses, si.dt, nullptr,
                          nullptr, si.epoch, false);
 }
 

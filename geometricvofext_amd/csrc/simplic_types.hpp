@@ -22,6 +22,8 @@ struct DevMesh {
     // same cells, faces in ascending face order (fvc::surfaceIntegrate order),
     // neighbour faces stored as ~f
     const int* cFacesAsc;
+    const int* cFacesSgn;    // cFaces, with ~face where the cell is the face's neighbour
+    int hasEmpty;            // 1 when any face lies on an empty patch
     // cell -> point CSR (unique points, ascending labels)
     const int* cpOff;
     const int* cPts;
