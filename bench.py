@@ -3,7 +3,7 @@
 
 Metric: interface-cell updates/s = sum over steps of the mixed
 cell count N_ic / sum over steps of (t_reconstruct + t_advect), both times
-measured with HIP events on the library's stream.  A step is one
+measured on the GPU by the library (svp_timers).  A step is one
 reconstruct() + advect() of the deformation test (applications/test/
 plicVofAdvectionFoam) on the workload below; the unscaled velocity and flux
 are resident in HBM, and each step rescales them on the GPU by the harness's
