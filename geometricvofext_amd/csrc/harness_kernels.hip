@@ -49,7 +49,7 @@ __device__ __attribute__((always_inline)) inline void courant_cell(const DevMesh
     const int b = cell_faces(m, c, nf);
     const double a = alpha[c], V = m.V[c];
     double s = 0.0;
-    if (nf <= MF) {
+    if (nf > 0 && nf <= MF) {
         int e[MF];
         double v[MF];
         unsigned char em[MF];

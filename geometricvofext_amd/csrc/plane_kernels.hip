@@ -325,7 +325,8 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
         const double alphaI = st.alpha[c];
         const V3 Cc = ld3(m.C, c);
         const double Vc = m.V[c];
-        if (mag(normalI) < SVP_TSMALL) {
+        // (a cell without faces has no loads to make and no plane)
+        if (nF == 0 || mag(normalI) < SVP_TSMALL) {
             if (l == 0 && s == 0) {
                 st.status[i] = (int)sgn(0.5 - alphaI);
                 st.nCutPts[i] = 0;
@@ -668,6 +669,10 @@ __global__ void __launch_bounds__(64, 1) k_plic_group(DevMesh m, DevState st, in
         const int c = st.mixed[i];
         int nF, n;
         const int fb = cell_faces(m, c, nF);
+        if (nF == 0) {   // no face to load, no polygon
+            if (l == 0 && !pts) ptOff[i] = faceIdx[i] = 0;
+            continue;
+        }
         const V3 normalI = ld3(st.ifN, i);
         const double dist = st.ifD[i];
         const int fL = m.cFaces[fb + min(l, nF - 1)];

@@ -1324,7 +1324,7 @@ __device__ __attribute__((always_inline)) inline double cell_face_sum(const DevM
     int nf;
     const int b = cell_faces(m, c, nf);
     double sI = 0.0;
-    if (MF > 0 && nf <= MF) {
+    if (MF > 0 && nf > 0 && nf <= MF) {
         constexpr int N = MF > 0 ? MF : 1;
         int e[N], f[N];
         double v[N];
