@@ -518,6 +518,9 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
             }
             __builtin_amdgcn_wave_barrier();
         }
+        // (every group's: a group without the final cut may have cut the last
+        // bracket at two thirds)
+        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
         if (s != owner) continue;
         if (l == 0) {
             unsigned long long fcls = 0ull;
@@ -532,7 +535,6 @@ __device__ __attribute__((always_inline)) inline void k_fsd_group_body(const Dev
             st3(st.ifC, i, cc.C);
             st3(st.ifS, i, cc.S);
         }
-        if (!ok) atomicOr(st.errFlag, ERR_TOO_MANY_CROSSINGS);
         // (a large group's Un0 waits for the advect, k_un0_group)
         if constexpr (G <= 8) {
             double un0 = 0.0;

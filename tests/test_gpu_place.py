@@ -87,3 +87,18 @@ def test_place_every_split(oracle_lib, kind, N, mixed):
         assert bits_equal(gi[k], oi[k]), k
     assert bits_equal(gpu.un0(), oi["un0"])
     gpu.synchronize()
+
+
+# strongly warped faces of 8 points, one of which its cell's plane crosses six
+# times, with two groups per cell (up to 1024 mixed cells) and with one
+@pytest.mark.parametrize("N", [5, 13])
+def test_place_refuses_many_crossings(N):
+    import geometricvofext_amd as g
+    print("crossings", N, flush=True)
+    mesh = g.brick_box(N, seed=N, perturb=0.3)
+    s = g.SolveVofEqu(mesh, dict(orientationMethod="LS"))
+    s.set_alpha(np.random.default_rng(N).uniform(0.02, 0.98, mesh.n_cells))
+    s.reconstruct()
+    with pytest.raises(g.SvpError, match="0x2 "):
+        s.synchronize()
+    s.synchronize()     # (reported once)
