@@ -554,13 +554,17 @@ void launch_count_nonfinite(const double* x, long nx, const double* y, long ny, 
     k_count_nonfinite<<<count_blocks(std::max(nx, ny)), 256, 0, s>>>(x, nx, y, ny, (ulonglong2*)out);
 }
 
-// the words of a handle's state that host decisions take, to host memory in one go
+// the words of a handle's state that host decisions take, to host memory in one
+// go; the totals' words only for a call that asks for them, so that a getter on
+// another thread does not clear those of an export that has still to read them
 __global__ void k_status(const int* err, const int* nMixed, const int* totals, int* out) {
     if (threadIdx.x != 0) return;
     out[0] = *err;
     out[1] = *nMixed;
-    out[2] = totals ? totals[0] : 0;
-    out[3] = totals ? totals[1] : 0;
+    if (totals) {
+        out[2] = totals[0];
+        out[3] = totals[1];
+    }
 }
 
 void launch_status(const DevState& st, const int* totals, int* out, hipStream_t s) {

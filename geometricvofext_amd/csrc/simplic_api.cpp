@@ -295,8 +295,8 @@ public:
         for (int i = 0; i < N_STAGES; ++i) { profSec_[i] = 0.0; profCnt_[i] = 0; }
     }
 
-    // error bits, mixed cells and two totals, as the stream's work so far
-    // leaves them: one launch and one wait
+    // error bits, mixed cells and (asked for) two totals, as the stream's work
+    // so far leaves them: one launch and one wait
     struct Status {
         int err, nMixed, totals[2];
     };
@@ -305,7 +305,9 @@ public:
         launch_status(st_, totals, w, stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
-        return Status{w[0], w[1], {w[2], w[3]}};
+        Status r{w[0], w[1], {0, 0}};
+        if (totals) std::memcpy(r.totals, w + 2, sizeof r.totals);
+        return r;
     }
     // the same, refused when an error bit is set
     Status checkDeviceErrors(const int* totals = nullptr) {
@@ -683,7 +685,7 @@ public:
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
     double* U0b_ = nullptr;
-    HostOut courant_, finite_, status_;   // apart, so that a getter on another thread disturbs none
+    HostOut courant_, finite_, status_;   // apart: one call's words are not another's
     int* nonfinite_ = nullptr;   // count of warped faces
     std::vector<double> hostC_, hostCf_, hostSf_;
     // learned orientation method
