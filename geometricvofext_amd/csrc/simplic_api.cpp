@@ -327,10 +327,8 @@ public:
         return status;
     }
 
-    // few candidates seen before a new alpha or flow say nothing about the next step
-    void fieldChanged() {
-        if (*st_.bndHint <= SMALL_CANDS) *st_.bndHint = -1;
-    }
+    // the bounding candidates of the steps so far say nothing about the next one
+    void fieldChanged() { st_.bndSince = st_.epoch; }
 
     void setAlpha(const double* a, int where) {
         copyIn(st_.alpha, a, m_.nC, where);
@@ -659,6 +657,7 @@ public:
         if (st_.epoch == 0x7ffffffe) {
             HIPCHECK(hipMemsetAsync(st_.nbTag, 0, sizeof(int) * m_.nC, stream_));
             st_.epoch = 0;
+            st_.bndSince = 0;
         }
         return st_.epoch + 1;
     }
@@ -1081,8 +1080,8 @@ private:
         courant_.alloc(courant_blocks(1, m_.nC));
         finite_.alloc(count_blocks(std::max<long>(m_.nF, 3L * m_.nC)));
         status_.alloc(2);
-        st_.bndHint = (int*)(status_.p + 2);
-        *st_.bndHint = 0;
+        st_.bndReport = status_.p + 2;
+        *st_.bndReport = 0;
         fieldChanged();
     }
 };
@@ -1226,27 +1225,29 @@ public:
         for (int k = 0; k < n; ++k)
             if (!std::isfinite(dt[k])) throw SvpError(SVP_E_ARG, "svp_batch_step: non-finite dt");
         upload(dt, nullptr);
+        const bool small = oneWorkgroup();
         hipEvent_t a = event(), b = event();
         HIPCHECK(hipEventRecord(a, stream_));
         if (profMask_ || !useGraph_) {
             for (int sg = STAGE_DETECT; sg <= STAGE_SNAPCLIP; ++sg)
-                profiled(sg, [&] { launchStage(sg); });
+                profiled(sg, [&] { launchStage(sg, small); });
         } else {
             // the step's launches do not depend on dt or the buffer
             // parities (both are read from info_ on the device), so one
             // captured graph replays every step
-            if (!graph_) {
+            hipGraphExec_t& exec = graph_[small];
+            if (!exec) {
                 hipGraph_t g = nullptr;
                 HIPCHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-                for (int sg = STAGE_DETECT; sg <= STAGE_SNAPCLIP; ++sg) launchStage(sg);
+                for (int sg = STAGE_DETECT; sg <= STAGE_SNAPCLIP; ++sg) launchStage(sg, small);
                 const hipError_t launched = hipGetLastError();
                 HIPCHECK(hipStreamEndCapture(stream_, &g));
                 HIPCHECK(launched);
-                const hipError_t made = hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0);
+                const hipError_t made = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
                 HIPCHECK(made);
             }
-            HIPCHECK(hipGraphLaunch(graph_, stream_));
+            HIPCHECK(hipGraphLaunch(exec, stream_));
         }
         HIPCHECK(hipEventRecord(b, stream_));
         HIPCHECK(hipGetLastError());
@@ -1261,14 +1262,30 @@ public:
         steps_++;
     }
 
-    void launchStage(int sg) {
+    void launchStage(int sg, bool small) {
         launch_batch_stage(sg, (const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, size(), maxC_, maxF_,
-                           maxDet_, maxList_, dims_, params_, G_, MF_, fluxKind_, fluxListed_, bndSmall_, stream_);
+                           maxDet_, maxList_, dims_, params_, G_, MF_, fluxKind_, fluxListed_, small, stream_);
     }
 
     void dropGraph() {
-        if (graph_) (void)hipGraphExecDestroy(graph_);
-        graph_ = nullptr;
+        for (hipGraphExec_t& exec : graph_) {
+            if (exec) (void)hipGraphExecDestroy(exec);
+            exec = nullptr;
+        }
+    }
+
+    // The bounding of the step by a workgroup per case, or by separate launches
+    // over all cases where one of them had many candidates in its last first
+    // pass: the step waits for that case's workgroup.  Whole steps, a workgroup
+    // per case against separate launches: 4 cases of 44^3 perturbed, 600 to 876
+    // candidates, 626 us and 500 (10 passes 1020 and 845); 4 of 50^3, 897 to
+    // 1303, 802 and 586; 4 of 36^3, 331 to 479, 417 and 407; 64 of 32^3, 152 to
+    // 570, 1055 and 1056; 12 of 32^3 plain, 19 to 101, 331 and 359.
+    bool oneWorkgroup() const {
+        if (!bndSmall_) return false;
+        for (const solveVofEqu* h : c_)
+            if (bound_last(h->st_) > SMALL_CANDS) return false;
+        return true;
     }
 
     // harness: max over each case's cells of sum|phi|/V and of the same for
@@ -1434,9 +1451,10 @@ private:
     bool haveFlow_ = true;
     BatchDims dims_{};
     // the step's launches as one graph (SVP_BATCH_GRAPH=0: launched one by
-    // one); rebuilt after the launch shapes change
+    // one), for either form of the bounding; rebuilt after the launch shapes
+    // change
     bool useGraph_ = true;
-    hipGraphExec_t graph_ = nullptr;
+    hipGraphExec_t graph_[2] = {};
     DBuf bc_, info_, factors_;
     gve::SimPLIC::HostOut courant_;
     char* ring_[RING] = {};

@@ -1758,6 +1758,10 @@ constexpr int BND_PREV_COUNT = 16;
 // whether one workgroup has taken the step's passes (k_bnd_small), so that the
 // launches queued behind it have nothing to do
 constexpr int BND_HANDLED = 17;
+// (one store: the host never sees one half without the other)
+__device__ inline void bound_report(const DevState& st, int epoch, int nCand) {
+    *st.bndReport = ((unsigned long long)(unsigned)epoch << 32) | (unsigned)nCand;
+}
 // any cell out of bounds: sum of the spread counters (each slot is one cache
 // line, so the update kernel's blocks do not queue on a single address)
 __device__ inline bool oob_any(const DevState& st) {
@@ -2462,7 +2466,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
     // pass statistics, and the candidate count for the next list's clearing
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st.bcount[BND_PREV_COUNT] = nCand;
-        if (pass == 0) *st.bndHint = nCand;
+        if (pass == 0) bound_report(st, epoch, nCand);
         if (pass < MAX_BOUND_PASSES && nCand > 0) {
             int nAct = 0;
             for (int r = 0; r <= st.gridRounds; ++r) nAct += st.bcount[3 + r];
@@ -2569,7 +2573,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
         __syncthreads();
         if (sOob == 0) {
             if (t == 0 && pass == 0) {
-                *A.bndHint = 0;
+                bound_report(A, epoch, 0);
                 bcount[BND_HANDLED] = 1;
             }
             bound_clear(m, other, nPrev, t, T);
@@ -2593,7 +2597,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
         }
         if (pass == 0) {
             if (t == 0) {
-                *A.bndHint = nCand;
+                bound_report(A, epoch, nCand);
                 bcount[BND_HANDLED] = mayDecline && nCand > SMALL_CANDS ? 0 : 1;
             }
             if (mayDecline && nCand > SMALL_CANDS) return;
@@ -2811,25 +2815,30 @@ bool bound_small(const DevMesh& m, const DevState& st) {
     return st.bndFlow && st.maxCellFaces <= NS_CELL_FACES && m.nC <= st.bndSmall;
 }
 
-// One workgroup takes a step's passes where they have few candidates.  Three
-// passes of 221, 16 and 3 (64^3): 82 us in one launch, 102 and the gaps between
-// them in twelve (a step 206 us against 228); with the first of them by the
-// separate launches 36 + 42, and the step slower by their gaps (217).  900 (48^3
-// perturbed, 341 us a step against 134) are left to the separate launches.
-// Meshes of up to BOUND_ALWAYS_SMALL_CELLS are not looked at: the launches to
-// fall back on would cost their steps more than a pass of many candidates does.
-// The host goes by the first pass's count that the GPU last reported, which may
-// be a few steps old; only the time depends on it.  Where it was few and may not be
-// any more (a new alpha or flow) the workgroup looks itself, and where it declines the separate launches,
+// One workgroup takes a step's passes where they have few candidates, by the
+// first pass's count that the GPU last reported; only the time depends on it.
+// Three passes of 221, 16 and 3 (64^3): 78 us in one launch, 102 and the gaps
+// between them in twelve.  Whole steps, one workgroup against separate launches:
+// 36^3 perturbed, 3 passes, 384 candidates 216 us and 211, 666: 243 and 226,
+// 1136: 290 and 247.  A pass more is 25 us of launches and, in the workgroup, a
+// short pass of few candidates, so on those meshes the line moves with the number
+// of passes (10 passes: 363 candidates 384 and 470, 1136: 438 and 471, 1400: 458
+// and 484).
+// The count may be a few steps old.  On meshes of up to BOUND_TRUST_CELLS a count
+// that grew meanwhile costs one step a fraction of what the measured ones show.
+// On larger ones, where it may have grown much (a new alpha or flow) since the
+// report, the workgroup looks itself, and where it declines the separate launches,
 // queued behind it in any case, do the work.
 template <int MF>
 void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
                         const double* Su, int* passSeq, hipStream_t s) {
     int behind = 0;
     if constexpr (MF <= NS_CELL_FACES) {
-        const int last = m.nC <= BOUND_ALWAYS_SMALL_CELLS ? 0 : *(const volatile int*)st.bndHint;
-        if (nPasses > 0 && bound_small(m, st) && last <= SMALL_CANDS) {
-            behind = last < 0;
+        const bool trust = m.nC <= BOUND_TRUST_CELLS;
+        const int limit = trust ? std::max(SMALL_CANDS, SMALL_CANDS * nPasses / 3) : SMALL_CANDS;
+        const int reported = bound_last_epoch(st);
+        if (nPasses > 0 && bound_small(m, st) && bound_last(st) <= limit) {
+            behind = !trust && reported <= st.bndSince;
             k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
                                                          bound_half(bound_pass_view(m, st, *passSeq + 1)), nPasses, dt,
                                                          Sp, Su, behind);

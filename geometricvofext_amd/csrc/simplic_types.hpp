@@ -103,7 +103,10 @@ struct DevState {
     int bndGrid;        // workgroups of the grid-stride bounding kernels
     int bndFlow;        // workgroups of the one-launch dataflow pass, 0 = rounds and tail
     int bndSmall;       // cells up to which one workgroup takes all passes
-    int* bndHint;       // host memory: candidates of the last step's first bounding pass, -1 not known
+    // host memory: the last step's first bounding pass, number of its
+    // reconstruct (upper half) and candidates
+    unsigned long long* bndReport;
+    int bndSince;       // (host) reports of reconstructs up to this one are older than the field or the flow
     int bndListWords;   // bitmap words per block of the candidate list (64..4096)
     void* bndRec;       // BndStore<MF> of the active bounding candidates, capacity nC
     int maxCellFaces;
@@ -150,10 +153,10 @@ constexpr int OOB_STRIDE = 16;
 constexpr int CLOCK_SLOTS = 64, CLOCK_STRIDE = 8;
 constexpr int STAGE_CLOCK_WORDS = CLOCK_STRIDE + 2 * CLOCK_SLOTS * CLOCK_STRIDE;
 
-// meshes whose bounding passes one workgroup takes: always, where the last step
-// had few candidates, and as a case of a batch (where the other cases fill the
-// chip meanwhile)
-constexpr int BOUND_ALWAYS_SMALL_CELLS = 49152, BOUND_SMALL_CELLS = 524288, BOUND_SMALL_BATCH_CELLS = 131072;
+// meshes whose bounding passes one workgroup may take, alone and as a case of a
+// batch, and those where it takes them without a look at a count that may have
+// grown since the last report
+constexpr int BOUND_SMALL_CELLS = 524288, BOUND_SMALL_BATCH_CELLS = 131072, BOUND_TRUST_CELLS = 49152;
 constexpr int SMALL_CANDS = 512;   // more candidates are left to the separate launches
 
 constexpr int DETECT_BLOCK = 256;
@@ -354,8 +357,11 @@ int detect_list_blocks(int nC);   // blocks of the one-launch detection
 int bound_faces(int maxCellFaces);
 size_t bound_record_bytes(int maxCellFaces);
 void launch_count_warped(const DevMesh& m, int* count, hipStream_t s);  // faces below flatness 1 - tSmall
-// whether one workgroup takes all bounding passes of this mesh
+// whether one workgroup may take all bounding passes of this mesh
 bool bound_small(const DevMesh& m, const DevState& st);
+// what the GPU last reported of a first bounding pass
+inline int bound_last(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport & 0xffffffffull); }
+inline int bound_last_epoch(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport >> 32); }
 // the state of bounding pass number seq of a handle: the half (seq & 1) of
 // the double-buffered bounding arrays
 DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
