@@ -191,6 +191,7 @@ public:
     void advect(double dt, const double* Sp, const double* Su) {
         if (!(dt > 0.0) || !std::isfinite(dt)) throw SvpError(SVP_E_ARG, "advect: dt must be positive");
         if (!reconstructed_) reconstruct();
+        stepChanged(dt, Sp || Su);
         std::swap(st_.alpha, st_.alphaOld);
         for (int sg = STAGE_UPWIND; sg <= STAGE_SNAPCLIP; ++sg)
             stage(sg, [&] { launch_advect_stage(sg, m_, st_, params_, dt, Sp, Su, &bndPassSeq_, stream_); });
@@ -328,7 +329,17 @@ public:
     }
 
     // the bounding candidates of the steps so far say nothing about the next one
+    // (a new alpha or flow, more sources, a step or a flow of more than twice the
+    // size: with the candidates few before, there can be many)
     void fieldChanged() { st_.bndSince = st_.epoch; }
+    void stepChanged(double dt, bool sources) {
+        if (dt > 2.0 * lastDt_ || (sources && !hadSources_)) st_.bndSince = std::max(st_.bndSince, st_.epoch - 1);
+        hadSources_ = sources;
+    }
+    void flowScaled(double factor) {
+        if (!(factor * lastFactor_ > 0.0) || std::fabs(factor) > 2.0 * std::fabs(lastFactor_)) fieldChanged();
+        lastFactor_ = factor;
+    }
 
     void setAlpha(const double* a, int where) {
         copyIn(st_.alpha, a, m_.nC, where);
@@ -666,6 +677,7 @@ public:
         st_.epoch = nextEpoch();
         std::swap(st_.alpha, st_.alphaOld);
         bndPassSeq_ += nPasses;
+        stepChanged(dt, false);
         lastDt_ = dt;
         alphaPhiValid_ = false;
         reconstructed_ = false;
@@ -679,7 +691,8 @@ public:
     int device_ = 0;
     int nB_ = 0;
     hipStream_t stream_ = nullptr;
-    double lastDt_ = 0.0;
+    double lastDt_ = 0.0, lastFactor_ = 0.0;
+    bool hadSources_ = false;
     // harness base flow
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
@@ -1314,6 +1327,7 @@ public:
         launch_batch_scale_flow((const BatchCase*)bc_.p, (const BatchStepInfo*)info_.p, (const double*)factors_.p,
                                 size(), maxN_, stream_);
         HIPCHECK(hipGetLastError());
+        for (int k = 0; k < size(); ++k) c_[k]->flowScaled(factors[k]);
     }
 
     // GPU seconds of the batch steps so far and the summed mixed-cell counts
@@ -2010,6 +2024,7 @@ int svp_harness_upload_base_flow(svp_handle* h, const double* U0, const double* 
         s.copyIn(s.phi0_, phi0, s.m_.nF, SVP_HOST);
         if (U0b) s.copyIn(s.U0b_, U0b, 3L * s.nB_, SVP_HOST);
         else HIPCHECK(hipMemsetAsync(s.U0b_, 0, sizeof(double) * 3 * std::max(s.nB_, 1), s.stream_));
+        s.lastFactor_ = 0.0;   // the next scaled flow is a new one
     });
 }
 
@@ -2020,6 +2035,7 @@ int svp_harness_scale_flow(svp_handle* h, double factor) {
         svp::launch_scale_flow(s.m_.nC, s.m_.nF, s.nB_, s.U0_, s.phi0_, s.U0b_, factor, s.st_.U, s.st_.phi,
                                s.st_.Ub, s.stream_);
         HIPCHECK(hipGetLastError());
+        s.flowScaled(factor);
     });
 }
 
@@ -2040,6 +2056,7 @@ int svp_harness_init_alpha_surface(svp_handle* h, const double* tris, int32_t n_
         svp::launch_init_alpha_surface(s.m_, dtr, n_tris, mode, frac, cut, nCut, s.st_.alpha, s.stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(s.stream_));
+        s.fieldChanged();
     });
 }
 
@@ -2054,6 +2071,7 @@ int svp_harness_init_alpha(svp_handle* h, const double* shapes, int nShapes, int
         svp::launch_init_alpha(s.m_, ds, nShapes, maxDepth, s.st_.alpha, s.stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(s.stream_));
+        s.fieldChanged();
     });
 }
 

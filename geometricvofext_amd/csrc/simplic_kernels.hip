@@ -2826,9 +2826,9 @@ bool bound_small(const DevMesh& m, const DevState& st) {
 // and 484).
 // The count may be a few steps old.  On meshes of up to BOUND_TRUST_CELLS a count
 // that grew meanwhile costs one step a fraction of what the measured ones show.
-// On larger ones, where it may have grown much (a new alpha or flow) since the
-// report, the workgroup looks itself, and where it declines the separate launches,
-// queued behind it in any case, do the work.
+// On larger ones, where it may have grown much (a new alpha or flow, a longer
+// step) since the report, the workgroup looks itself, and where it declines the
+// separate launches, queued behind it in any case, do the work.
 template <int MF>
 void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
                         const double* Su, int* passSeq, hipStream_t s) {
