@@ -1390,6 +1390,12 @@ public:
                                         hipMemcpyDeviceToDevice, stream_));
         };
         const int oldMask = profMask_;
+        // the bounding shapes are those of its separate launches
+        struct Keep {
+            bool &v, old;
+            ~Keep() { v = old; }
+        } keep{bndSmall_, bndSmall_};
+        bndSmall_ = false;
         auto trial = [&](int stage) {
             profileSet(1 << stage);
             step(dt);

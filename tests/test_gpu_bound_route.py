@@ -93,3 +93,24 @@ def test_batch_few_and_many(oracle_lib, monkeypatch, kinds, graph):
         assert bits_equal(s.alpha(), o.alpha())
         s.synchronize()
 
+
+def test_batch_tune_keeps_the_route(oracle_lib):
+    """Launch shapes tuned on a batch whose passes one workgroup takes: the steps after are the oracle's."""
+    import geometricvofext_amd as g
+    print("batch tune", flush=True)
+    cases = [case(oracle_lib, "hexp", N, 0.05, N) for N in (9, 12)]
+    gpu = [g.SolveVofEqu(c[0], dict(orientationMethod="LS", **OPTS)) for c in cases]
+    ors = [oracle_lib.OracleSolver(c[1], threads=8, **OPTS) for c in cases]
+    for (_, _, alpha, U, phi, _), s, o in zip(cases, gpu, ors):
+        for x in (s, o):
+            x.set_alpha(alpha)
+            x.set_flow(phi, U)
+    b = g.CaseBatch(gpu)
+    dts = [0.5 * c[5] for c in cases]
+    b.tune(dts)
+    for _ in range(3):
+        b.step(dts)
+        for s, o, dt in zip(gpu, ors, dts):
+            o.reconstruct()
+            o.advect(dt)
+            assert bits_equal(s.alpha(), o.alpha())
