@@ -330,11 +330,13 @@ public:
 
     // the bounding candidates of the steps so far say nothing about the next one
     // (a new alpha or flow, more sources, a step or a flow of more than twice the
-    // size: with the candidates few before, there can be many)
+    // size, fields in the caller's hands: with the candidates few before, there
+    // can be many)
     void fieldChanged() { st_.bndSince = st_.epoch; }
     void stepChanged(double dt, bool sources) {
         if (dt > 2.0 * lastDt_ || (sources && !hadSources_)) st_.bndSince = std::max(st_.bndSince, st_.epoch - 1);
         hadSources_ = sources;
+        if (viewed_) fieldChanged();
     }
     void flowScaled(double factor) {
         if (!(factor * lastFactor_ > 0.0) || std::fabs(factor) > 2.0 * std::fabs(lastFactor_)) fieldChanged();
@@ -693,6 +695,7 @@ public:
     hipStream_t stream_ = nullptr;
     double lastDt_ = 0.0, lastFactor_ = 0.0;
     bool hadSources_ = false;
+    bool viewed_ = false;   // the caller holds device pointers: fields can change without a call
     // harness base flow
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
@@ -1858,6 +1861,7 @@ int svp_device_view_get(svp_handle* h, svp_device_view* out) {
         out->C = s.m_.C;
         out->V = s.m_.V;
         out->stream = (void*)s.stream_;
+        s.viewed_ = true;
     });
 }
 

@@ -114,3 +114,33 @@ def test_batch_tune_keeps_the_route(oracle_lib):
             o.reconstruct()
             o.advect(dt)
             assert bits_equal(s.alpha(), o.alpha())
+
+
+def test_flow_written_in_place(oracle_lib):
+    """phi written through the device view, with no call that tells of it: few candidates, many, few, many."""
+    import ctypes as C
+    import geometricvofext_amd as g
+    print("flow in place", flush=True)
+    mesh, om, alpha, U, phi, h = case(oracle_lib, "hexp", 38, 0.3, 38)
+    gpu = g.SolveVofEqu(mesh, dict(orientationMethod="LS", **OPTS))
+    ors = oracle_lib.OracleSolver(om, threads=8, **OPTS)
+    for s in (gpu, ors):
+        s.set_alpha(alpha)
+        s.set_flow(1e-16 * phi, U)
+    hip = C.CDLL("libamdhip64.so.7")    # the runtime the library runs on
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    at = gpu.device_view().phi
+    seen = []
+    for k, f in enumerate([1e-16, 1e-16, 1.0, 1.0, 1e-16, 1e-16, 0.5]):
+        gpu.synchronize()
+        now = np.ascontiguousarray(f * phi)
+        assert hip.hipMemcpy(at, now.ctypes.data, now.nbytes, 1) == 0
+        ors.set_flow(f * phi, U)
+        for s in (gpu, ors):
+            s.reconstruct()
+            s.advect(0.9 * h)
+        assert bits_equal(gpu.alpha(), ors.alpha()), k
+        seen.append(int(gpu.bound_stats()[:1, 0].sum()))
+    print("candidates", seen, flush=True)
+    assert min(seen) <= 512 < max(seen)
+    gpu.synchronize()
