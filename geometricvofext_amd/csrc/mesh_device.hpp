@@ -96,9 +96,12 @@ __device__ inline DevState batch_view(const BatchCase& c, const BatchStepInfo& s
 // record before and after each (four commands that the kernels of a step
 // queue behind) took 14 us of a 125 us step at 16^3 cells, 12 at 64^3 (four
 // steps 888 -> 838 us).  The first kernel of a stage adds up what has
-// ended before it and notes its start; the waves of kernels that may be the
-// last note their end, each in one of CLOCK_SLOTS words, by a maximum that
-// nothing waits for.
+// ended before it and notes its start; every block of the kernels that can be
+// the stage's last notes its end, in one of CLOCK_SLOTS words, by a maximum that
+// nothing waits for.  So a time runs from the first block of the first kernel
+// to the last block of the last one, without the command processor's work before and
+// after, which events around the call include: 331 us a step at 128^3 where they
+// give 342.
 // adds the finished stages to their sums (one wave)
 __device__ inline void stage_fold(const DevState& st, int lane) {
     for (int k = 0; k < 2; ++k) {
@@ -125,9 +128,10 @@ __device__ inline void stage_stop(const DevState& st, int stage) {
     atomicMax(&st.clock[CLOCK_STRIDE + (stage * CLOCK_SLOTS + slot) * CLOCK_STRIDE],
               (unsigned long long)wall_clock64());
 }
-// the same for a kernel whose workgroups all do the same work: those started last
-__device__ inline void stage_stop_tail(const DevState& st, int stage) {
-    if ((threadIdx.x & 63) == 0 && blockIdx.x + 16 >= gridDim.x) stage_stop(st, stage);
+// the same by one lane of every block, once all its waves are done
+__device__ inline void stage_stop_block(const DevState& st, int stage) {
+    __syncthreads();
+    if (threadIdx.x == 0) stage_stop(st, stage);
 }
 
 }  // namespace svp

@@ -1397,9 +1397,10 @@ __device__ __attribute__((always_inline)) inline void k_update_body(const DevMes
 }
 
 template <int MF>
-__global__ void __launch_bounds__(UPDATE_BLOCK) k_update(DevMesh m, DevState st, double dtStep, const double* Sp, const double* Su) {
+__global__ void __launch_bounds__(UPDATE_BLOCK) k_update(DevMesh m, DevState st, double dtStep, const double* Sp, const double* Su,
+                                                         int last) {
     k_update_body<MF>(m, st, dtStep, Sp, Su, st.epoch);
-    stage_stop_tail(st, 1);
+    if (last) stage_stop_block(st, 1);
 }
 
 // face slots of the update's gathered form: the mesh's largest cell when it
@@ -1408,14 +1409,15 @@ static int update_faces(int maxCellFaces) {
     return maxCellFaces <= 4 ? 4 : (maxCellFaces <= 6 ? 6 : (maxCellFaces <= 8 ? 8 : 0));
 }
 
+// last: no bounding pass and no snap or clip follows, to note the end of the advect
 static void launch_update(const DevMesh& m, const DevState& st, double dt, const double* Sp, const double* Su,
-                          hipStream_t s) {
+                          int last, hipStream_t s) {
     const dim3 grid(cdiv(m.nC, UPDATE_BLOCK));
     switch (update_faces(st.maxCellFaces)) {
-        case 4: k_update<4><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su); break;
-        case 6: k_update<6><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su); break;
-        case 8: k_update<8><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su); break;
-        default: k_update<0><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su); break;
+        case 4: k_update<4><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su, last); break;
+        case 6: k_update<6><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su, last); break;
+        case 8: k_update<8><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su, last); break;
+        default: k_update<0><<<grid, UPDATE_BLOCK, 0, s>>>(m, st, dt, Sp, Su, last); break;
     }
 }
 
@@ -2867,18 +2869,20 @@ void launch_bound(const DevMesh& m, const DevState& st, const Params& p, double 
 }
 
 // applyBruteForceBounding (advection.C:291-308)
+// (blocks that loop: each notes the end of the advect)
+constexpr int SNAP_BLOCKS = 2048;
 __device__ __attribute__((always_inline)) inline void k_snap_clip_body(int nC, double* alpha, double snapTol, int clip, const DevState& st) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nC) return;
-    double a = alpha[c];
-    if (snapTol > 0.0) a = a * pos0(a - snapTol) * neg0(a - (1.0 - snapTol)) + pos0(a - (1.0 - snapTol));
-    if (clip) a = fmin(1.0, fmax(0.0, a));
-    alpha[c] = a;
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
+        double a = alpha[c];
+        if (snapTol > 0.0) a = a * pos0(a - snapTol) * neg0(a - (1.0 - snapTol)) + pos0(a - (1.0 - snapTol));
+        if (clip) a = fmin(1.0, fmax(0.0, a));
+        alpha[c] = a;
+    }
 }
 
 __global__ void k_snap_clip(int nC, double* alpha, double snapTol, int clip, DevState st) {
     k_snap_clip_body(nC, alpha, snapTol, clip, st);
-    stage_stop_tail(st, 1);
+    stage_stop_block(st, 1);
 }
 
 __global__ void k_zero_int(int* p, int n) {
@@ -2902,14 +2906,14 @@ void launch_advect_stage(int stage, const DevMesh& m, const DevState& st, const 
             launch_interface_flux(m, st, dt, s);
             break;
         case STAGE_UPDATE:
-            launch_update(m, st, dt, Sp, Su, s);
+            launch_update(m, st, dt, Sp, Su, p.nAlphaBounds <= 0 && !(p.snapTol > 0.0 || p.clip), s);
             break;
         case STAGE_BOUND:
             launch_bound(m, st, p, dt, Sp, Su, passSeq, s);
             break;
         case STAGE_SNAPCLIP:
             if (p.snapTol > 0.0 || p.clip)
-                k_snap_clip<<<cdiv(m.nC, 256), 256, 0, s>>>(m.nC, st.alpha, p.snapTol, p.clip, st);
+                k_snap_clip<<<std::min(SNAP_BLOCKS, cdiv(m.nC, 256)), 256, 0, s>>>(m.nC, st.alpha, p.snapTol, p.clip, st);
             break;
         default:
             break;

@@ -186,7 +186,10 @@ int svp_get_geometry(svp_handle* h, double* Cf, double* Sf, double* magSf, doubl
                      double* C, double* V);
 /* Cumulative GPU seconds spent in reconstruct and advect (the reference's
  * reconstructionTime/advectionTime, solveVofEqu.H:195-211) and the running sum
- * of mixed-cell counts over all reconstruct calls. */
+ * of mixed-cell counts over all reconstruct calls.  Each call's span on the
+ * GPU's clock, first block of its first kernel to last block of its last one;
+ * steps of a batch are not in them (svp_batch_timers, which measures by HIP
+ * events around the step). */
 int svp_timers(svp_handle* h, double* reconstruction_s, double* advection_s, uint64_t* n_ic_total);
 /* solveVofEqu::alphaMappingTime (solveVofEqu.H:208-210 ->
  * reconstruction.H:396-399): cumulative GPU seconds of svp_map_alpha_field. */
