@@ -2748,7 +2748,7 @@ __global__ void __launch_bounds__(SMALL_THREADS) k_bnd_small(DevMesh m, DevState
                                                                    double dt, const double* Sp, const double* Su,
                                                                    int mayDecline) {
     k_bnd_small_body<MF>(m, A, B, nPasses, dt, Sp, Su, A.epoch, mayDecline != 0);
-    if (threadIdx.x == 0) stage_stop(A, 1);
+    stage_stop_block(A, 1);
 }
 
 template <int MF>
