@@ -248,191 +248,6 @@ __device__ inline bool calcSubFace(const V3* fPts, int n, V3 normal, double dist
     return ok;
 }
 
-// Element j of a register array of N values, as a select chain (keeps the
-// array in registers where a dynamic index would spill it to scratch).
-template <int N, class T>
-__device__ inline T pick(const T (&a)[N], int j) {
-    T r = a[0];
-#pragma unroll
-    for (int k = 1; k < N; ++k)
-        if (j == k) r = a[k];
-    return r;
-}
-
-// Rotate register arrays left by r (0 <= r < N): a[i] <- a[(i + r) % N], by
-// conditional moves with static indices only (binary stages of the shift),
-// so the arrays stay in registers.
-template <int N, class T>
-__device__ inline void rotate_left(T (&a)[N], int r) {
-#pragma unroll
-    for (int s = 1; s < N; s <<= 1) {
-        if (r & s) {
-            T t[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) t[i] = a[(i + s) % N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) a[i] = t[i];
-        }
-    }
-}
-
-// calcSubFace for a face of exactly N points held in registers; the same
-// operations in the same order as calcSubFace above.
-// IF: record the plane crossings in out.ifPts (the cell cut needs them; the
-// face-flux integrals only need the area).  out may live in LDS: it is then
-// written in place, which keeps a per-lane copy of the record out of scratch.
-// FULL: full holds face::centre and face::areaNormal of these points (6
-// values), which a fully submerged face takes as they are instead of
-// computing them again.  DOTS: dots holds dot(fPts[i], normal), so that a
-// cut adds only the distance (the same values, computed once).
-template <int N, bool IF = true, bool FULL = false, bool DOTS = FULL, class FC>
-__device__ inline bool calcSubFaceN(const V3 (&fPts)[N], V3 normal, double distance, FC& out,
-                                    const double* full = nullptr, const double* dots = nullptr) {
-    auto fullCentre = [&]() {
-        if constexpr (FULL) return v3(full[0], full[1], full[2]);
-        else return faceCentre(fPts, N);
-    };
-    auto fullArea = [&]() {
-        if constexpr (FULL) return v3(full[3], full[4], full[5]);
-        else return faceAreaNormal(fPts, N);
-    };
-    double dist[N];
-    int nSub = 0, first = -1;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        double di;
-        if constexpr (DOTS) di = dots[i] + distance;
-        else di = dot(fPts[i], normal) + distance;
-        if (fabs(di) < SVP_TSMALL) di += sgn(di) * SVP_TSMALL;
-        dist[i] = di;
-        if (di < 0.0) {
-            nSub++;
-            if (first == -1) first = i;
-        }
-    }
-    out.nIf = 0;
-    if (nSub == N || nSub == 0) {
-        if (nSub == N) {
-            out.status = -1;
-            out.centre = fullCentre();
-            out.area = fullArea();
-        } else {
-            out.status = 1;
-            out.centre = VZERO;
-            out.area = VZERO;
-        }
-        return true;
-    }
-    bool ok = true;
-    // the walk starts at the first submerged point: rotate it to slot 0
-    V3 rp[N];
-    double rd[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        rp[i] = fPts[i];
-        rd[i] = dist[i];
-    }
-    rotate_left(rp, first);
-    rotate_left(rd, first);
-    int nPts = 0;
-    V3 p0 = VZERO, p1 = VZERO, p2 = VZERO, fCentre = VZERO;
-    auto emit1 = [&](V3 q) {
-        fCentre = vsel(nPts == 0, q, fCentre + q);
-        p0 = vsel(nPts == 0, q, p0);
-        p1 = vsel(nPts == 1, q, p1);
-        p2 = vsel(nPts == 2, q, p2);
-        nPts++;
-    };
-    static_assert(MAX_IF_POINTS == 4, "four crossing registers");
-    V3 ip0 = VZERO, ip1 = VZERO, ip2 = VZERO, ip3 = VZERO;
-    int nIf = 0;
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const int nxt = (k + 1 == N) ? 0 : k + 1;
-        const double dc = rd[k], dn = rd[nxt];
-        const V3 pc = rp[k], pn = rp[nxt];
-        if (dc < 0) emit1(pc);
-        if ((dc * dn) < 0) {
-            const double w = dc / (dc - dn);
-            const V3 q = pc + w * (pn - pc);
-            emit1(q);
-            if constexpr (IF) {
-                ip0 = vsel(nIf == 0, q, ip0);
-                ip1 = vsel(nIf == 1, q, ip1);
-                ip2 = vsel(nIf == 2, q, ip2);
-                ip3 = vsel(nIf == 3, q, ip3);
-            }
-            if (nIf >= MAX_IF_POINTS) ok = false;
-            nIf++;
-        }
-    }
-    if constexpr (IF) {
-        out.ifPts[0] = ip0;
-        out.ifPts[1] = ip1;
-        out.ifPts[2] = ip2;
-        out.ifPts[3] = ip3;
-    }
-    out.nIf = nIf > MAX_IF_POINTS ? MAX_IF_POINTS : nIf;
-    if (nPts < 3) {
-        out.status = -1;
-        out.centre = fullCentre();
-        out.area = fullArea();
-        return ok;
-    }
-    out.status = 0;
-    if (nPts == 3) {
-        out.centre = (1.0 / 3.0) * (p0 + p1 + p2);
-        out.area = 0.5 * cross(p1 - p0, p2 - p0);
-        return ok;
-    }
-    fCentre = fCentre / (double)nPts;
-    V3 sumN = VZERO, sumAc = VZERO;
-    double sumA = 0.0;
-    V3 prev = VZERO, firstP = VZERO;
-    int kk = 0;
-    auto emit2 = [&](V3 q) {
-        const bool on = kk > 0;
-        firstP = vsel(on, firstP, q);
-        if (on) {
-            const V3 c = prev + q + fCentre;
-            const V3 nn = cross(q - prev, fCentre - prev);
-            const double ar = mag(nn);
-            sumN = sumN + nn;
-            sumA += ar;
-            sumAc = sumAc + ar * c;
-        }
-        prev = q;
-        kk++;
-    };
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const int nxt = (k + 1 == N) ? 0 : k + 1;
-        const double dc = rd[k], dn = rd[nxt];
-        const V3 pc = rp[k], pn = rp[nxt];
-        if (dc < 0) emit2(pc);
-        if ((dc * dn) < 0) {
-            const double w = dc / (dc - dn);
-            emit2(pc + w * (pn - pc));
-        }
-    }
-    {
-        const V3 c = prev + firstP + fCentre;
-        const V3 nn = cross(firstP - prev, fCentre - prev);
-        const double ar = mag(nn);
-        sumN = sumN + nn;
-        sumA += ar;
-        sumAc = sumAc + ar * c;
-    }
-    if (sumA < SVP_ROOTVSMALL) {
-        out.centre = fCentre;
-        out.area = VZERO;
-    } else {
-        out.centre = (1.0 / 3.0) * sumAc / sumA;
-        out.area = 0.5 * sumN;
-    }
-    return ok;
-}
-
 // Local description of one cell: its points and faces as point-index lists
 // (cutCell::getLocalPointFieldAndFaceList, cutCell.C:140-236).  Without
 // splitWarpedFace the faces are the mesh faces in their stored orientation.

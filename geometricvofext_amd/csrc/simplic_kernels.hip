@@ -1304,7 +1304,8 @@ __device__ inline bool loop_oob(double a, double aTol) { return (a - 1.0 > aTol)
 __device__ inline bool cell_oob(double a, double aTol) { return (a < -aTol) || (a > 1.0 + aTol); }
 
 // needBounding = mixed cells and their face neighbours (advection.C:54-82):
-// tagged with the reconstruct's number by the detection kernel
+// tagged with the reconstruct's number by the flux list, or by the unlisted
+// interface flux on tetrahedra
 __device__ inline bool need_bounding(const DevState& st, int c, int epoch) { return st.nbTag[c] == epoch; }
 
 // Conservative update (advectionTemplates.C:399-404) with fvc::surfaceIntegrate
@@ -1421,18 +1422,6 @@ static void launch_update(const DevMesh& m, const DevState& st, double dt, const
     }
 }
 
-__device__ inline double face_value(const DevMesh& m, const double* f, int facei) {
-    if (facei < m.nIF) return f[facei];
-    if (m.fEmpty[facei]) return 0.0;
-    return f[facei];
-}
-
-__device__ inline bool face_downwind_of(const DevMesh& m, const double* phi, int facei, int c) {
-    const double ph = face_value(m, phi, facei);
-    return (m.own[facei] == c) ? (ph >= 0) : (ph < 0);
-}
-
-
 // limitFlux (advectionTemplates.C:118-215), one pass = the kernels below.
 // The pass runs only while cells lie outside [-aTol, 1+aTol] (bound count of
 // the update kernel, kept current by the apply kernel):
@@ -1536,7 +1525,7 @@ __device__ inline int bound_record(const DevMesh& m, const DevState& st, int c, 
         if (k < nf) {
             const int f = fid[k];
             if (f < m.nIF) oth[k] = fo[k];
-            // face_value: empty-patch faces carry nothing
+            // empty-patch faces carry nothing (advectionTemplates.C:65-70)
             const bool live = (f < m.nIF) || !fem[k];
             const double ph = live ? fph[k] : 0.0;
             const double dv = live ? fdv[k] : 0.0;
@@ -2397,7 +2386,7 @@ __device__ __attribute__((always_inline)) inline int bound_apply_cell(const DevM
 #pragma unroll
     for (int k = 0; k < MF; ++k) {
         if (k >= nf) kpos[k] = -1;
-        // face_value: empty-patch faces carry nothing
+        // empty-patch faces carry nothing
         kval[k] = (kpos[k] >= 0 && (fid[k] < m.nIF || !kem[k])) ? kval[k] : 0.0;
     }
     double a = before;
@@ -2441,7 +2430,7 @@ __device__ __attribute__((always_inline)) inline int bound_apply_item(const DevM
             c = st.cand[i];
         } else if (((unsigned)recs.first(i) >> k) & 1u) {
             const int f = recs.fid(k, i), o = recs.oth(k, i);
-            // face_value of both: empty-patch faces keep theirs
+            // empty-patch faces keep theirs
             const double dv = st.dVf[f], cr = st.corr[f];
             const unsigned char em = empty_flag(m, f);
             const bool other = o >= 0 && st.actIdx[max(o, 0)] < 0;
@@ -2883,10 +2872,6 @@ __device__ __attribute__((always_inline)) inline void k_snap_clip_body(int nC, d
 __global__ void k_snap_clip(int nC, double* alpha, double snapTol, int clip, DevState st) {
     k_snap_clip_body(nC, alpha, snapTol, clip, st);
     stage_stop_block(st, 1);
-}
-
-__global__ void k_zero_int(int* p, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
 void launch_advect_stage(int stage, const DevMesh& m, const DevState& st, const Params& p, double dt,
