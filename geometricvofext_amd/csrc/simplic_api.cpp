@@ -1097,7 +1097,7 @@ private:
         finite_.alloc(count_blocks(std::max<long>(m_.nF, 3L * m_.nC)));
         status_.alloc(2);
         st_.bndReport = status_.p + 2;
-        *st_.bndReport = 0;
+        st_.bndReport[0] = st_.bndReport[1] = 0;
         fieldChanged();
     }
 };
@@ -1241,7 +1241,7 @@ public:
         for (int k = 0; k < n; ++k)
             if (!std::isfinite(dt[k])) throw SvpError(SVP_E_ARG, "svp_batch_step: non-finite dt");
         upload(dt, nullptr);
-        const bool small = oneWorkgroup();
+        const bool small = oneWorkgroup(dt);
         hipEvent_t a = event(), b = event();
         HIPCHECK(hipEventRecord(a, stream_));
         if (profMask_ || !useGraph_) {
@@ -1291,17 +1291,26 @@ public:
     }
 
     // The bounding of the step by a workgroup per case, or by separate launches
-    // over all cases where one of them had many candidates in its last first
-    // pass: the step waits for that case's workgroup.  Whole steps, a workgroup
-    // per case against separate launches: 4 cases of 44^3 perturbed, 600 to 876
-    // candidates, 626 us and 500 (10 passes 1020 and 845); 4 of 50^3, 897 to
-    // 1303, 802 and 586; 4 of 36^3, 331 to 479, 417 and 407; 64 of 32^3, 152 to
-    // 570, 1055 and 1056; 12 of 32^3 plain, 19 to 101, 331 and 359.
-    bool oneWorkgroup() const {
+    // over all cases where the stepping case of most candidates, whose workgroup the
+    // step waits for, has many: past the line of a single handle, moved by what the
+    // launches need for the candidates of all cases.  Whole steps, a workgroup per
+    // case against separate launches, 3 passes of perturbed hexahedra: 4 cases of
+    // 44^3, 600 to 876 candidates in the first pass, 626 us and 500 (10 passes 1020
+    // and 845); 4 of 50^3, 897 to 1303, 802 and 586; 12 of 44^3, 486 to 974, 710 and
+    // 593; 4 of 36^3, 331 to 479, 417 and 407; 64 of 32^3, 152 to 570, 1055 and 1056,
+    // 344 to 756, 1512 and 1532; 12 of 32^3 plain, 19 to 101, 331 and 359; 256 plain ones
+    // of 16^3 to 48^3 over their runs (up to 1630 in all passes of a case, 33k in all
+    // cases) 676 and 720.
+    bool oneWorkgroup(const double* dt) const {
         if (!bndSmall_) return false;
-        for (const solveVofEqu* h : c_)
-            if (bound_last(h->st_) > SMALL_CANDS) return false;
-        return true;
+        long most = 0, all = 0;
+        for (int k = 0; k < size(); ++k) {
+            if (!(dt[k] > 0.0)) continue;
+            const long n = bound_last_sum(c_[k]->st_);
+            most = std::max(most, n);
+            all += n;
+        }
+        return most <= (long)SMALL_CANDS_PER_PASS * std::min(params_.nAlphaBounds, MAX_BOUND_PASSES) + all / 32;
     }
 
     // harness: max over each case's cells of sum|phi|/V and of the same for

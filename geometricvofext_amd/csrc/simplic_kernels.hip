@@ -1749,9 +1749,11 @@ constexpr int BND_PREV_COUNT = 16;
 // whether one workgroup has taken the step's passes (k_bnd_small), so that the
 // launches queued behind it have nothing to do
 constexpr int BND_HANDLED = 17;
+// candidates of the step's passes so far
+constexpr int BND_SUM = 18;
 // (one store: the host never sees one half without the other)
 __device__ inline void bound_report(const DevState& st, int epoch, int nCand) {
-    *st.bndReport = ((unsigned long long)(unsigned)epoch << 32) | (unsigned)nCand;
+    st.bndReport[0] = ((unsigned long long)(unsigned)epoch << 32) | (unsigned)nCand;
 }
 // any cell out of bounds: sum of the spread counters (each slot is one cache
 // line, so the update kernel's blocks do not queue on a single address)
@@ -2458,6 +2460,9 @@ __device__ __attribute__((always_inline)) inline void k_bnd_apply_body(const Dev
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st.bcount[BND_PREV_COUNT] = nCand;
         if (pass == 0) bound_report(st, epoch, nCand);
+        const int sum = (pass == 0 ? 0 : st.bcount[BND_SUM]) + nCand;
+        st.bcount[BND_SUM] = sum;
+        st.bndReport[1] = (unsigned long long)sum;
         if (pass < MAX_BOUND_PASSES && nCand > 0) {
             int nAct = 0;
             for (int r = 0; r <= st.gridRounds; ++r) nAct += st.bcount[3 + r];
@@ -2518,7 +2523,7 @@ __host__ __device__ inline BndHalf bound_half(const DevState& v) {
 // update writes all of it anew).
 //
 // 10 passes of about 200 candidates (33^3 perturbed, the default dictionary):
-// 151 us, against 250 us of kernels in 40 launches and the gaps between them; 3
+// 140 us, against 250 us of kernels in 40 launches and the gaps between them; 3
 // passes of 1 to 20 (16^3): 34 us against 61.
 constexpr int SMALL_THREADS = 512;
 constexpr int SMALL_WORDS = BOUND_SMALL_CELLS / 64;
@@ -2550,7 +2555,7 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
         for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
         if (t == 0) sOob = n;
     }
-    int nPrev = bcount[BND_PREV_COUNT];
+    int nPrev = bcount[BND_PREV_COUNT], sum = 0;
     for (int pass = 0; pass < nPasses; ++pass) {
         const bool odd = (pass & 1) != 0;
         DevState st = A;   // this pass's half; `other` the one before it left
@@ -2728,8 +2733,12 @@ __device__ __attribute__((always_inline)) inline void k_bnd_small_body(const Dev
         if (d) atomicAdd(&sOob, d);
         bound_clear(m, other, nPrev, T - 1 - t, T);
         nPrev = nCand;
+        sum += nCand;
     }
-    if (t == 0) bcount[BND_PREV_COUNT] = nPrev;
+    if (t == 0) {
+        bcount[BND_PREV_COUNT] = nPrev;
+        A.bndReport[1] = (unsigned long long)sum;
+    }
 }
 
 template <int MF>
@@ -2807,28 +2816,29 @@ bool bound_small(const DevMesh& m, const DevState& st) {
 }
 
 // One workgroup takes a step's passes where they have few candidates, by the
-// first pass's count that the GPU last reported; only the time depends on it.
-// Three passes of 221, 16 and 3 (64^3): 78 us in one launch, 102 and the gaps
-// between them in twelve.  Whole steps, one workgroup against separate launches:
-// 36^3 perturbed, 3 passes, 384 candidates 216 us and 211, 666: 243 and 226,
-// 1136: 290 and 247.  A pass more is 25 us of launches and, in the workgroup, a
-// short pass of few candidates, so on those meshes the line moves with the number
-// of passes (10 passes: 363 candidates 384 and 470, 1136: 438 and 471, 1400: 458
-// and 484).
-// The count may be a few steps old.  On meshes of up to BOUND_TRUST_CELLS a count
+// counts that the GPU last reported; only the time depends on them.
+// Three passes of 221, 16 and 3 (64^3): 79 us in one launch, 102 and the gaps
+// between them in twelve.  The launches cost about 25 us a pass whatever the
+// count, the workgroup by the candidate, so the line is a mean count per pass.
+// Whole steps, one workgroup against separate launches, perturbed hexahedra: 36^3,
+// 3 passes, 384 + 331 + 337 candidates 216 us and 211, 666 + 352 + 309 243 and 226,
+// 1136 + 374 + 303 290 and 247; plain ones, 673 + 112 + 10 196 and 204; 10 passes,
+// about 320 each, 384 and 470, 1142 in the first of them 438 and 471.
+// The counts may be a few steps old.  On meshes of up to BOUND_TRUST_CELLS a count
 // that grew meanwhile costs one step a fraction of what the measured ones show.
-// On larger ones, where it may have grown much (a new alpha or flow, a longer
-// step) since the report, the workgroup looks itself, and where it declines the
-// separate launches, queued behind it in any case, do the work.
+// On larger ones the line is at the first pass's count, and where that may have
+// grown much (a new alpha or flow, a longer step) since the report, the workgroup
+// looks itself: where it declines, the separate launches, queued behind it in any
+// case, do the work.
 template <int MF>
 void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
                         const double* Su, int* passSeq, hipStream_t s) {
     int behind = 0;
     if constexpr (MF <= NS_CELL_FACES) {
         const bool trust = m.nC <= BOUND_TRUST_CELLS;
-        const int limit = trust ? std::max(SMALL_CANDS, SMALL_CANDS * nPasses / 3) : SMALL_CANDS;
         const int reported = bound_last_epoch(st);
-        if (nPasses > 0 && bound_small(m, st) && bound_last(st) <= limit) {
+        const bool few = trust ? bound_last_sum(st) <= (long)SMALL_CANDS_PER_PASS * nPasses : bound_last(st) <= SMALL_CANDS;
+        if (nPasses > 0 && bound_small(m, st) && few) {
             behind = !trust && reported <= st.bndSince;
             k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
                                                          bound_half(bound_pass_view(m, st, *passSeq + 1)), nPasses, dt,

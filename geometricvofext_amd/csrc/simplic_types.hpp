@@ -103,8 +103,8 @@ struct DevState {
     int bndGrid;        // workgroups of the grid-stride bounding kernels
     int bndFlow;        // workgroups of the one-launch dataflow pass, 0 = rounds and tail
     int bndSmall;       // cells up to which one workgroup takes all passes
-    // host memory: the last step's first bounding pass, number of its
-    // reconstruct (upper half) and candidates
+    // host memory, of the last step's bounding: number of its reconstruct
+    // (upper half) and candidates of its first pass; candidates of all passes
     unsigned long long* bndReport;
     int bndSince;       // (host) reports of reconstructs up to this one are older than the field or the flow
     int bndListWords;   // bitmap words per block of the candidate list (64..4096)
@@ -157,7 +157,9 @@ constexpr int STAGE_CLOCK_WORDS = CLOCK_STRIDE + 2 * CLOCK_SLOTS * CLOCK_STRIDE;
 // batch, and those where it takes them without a look at a count that may have
 // grown since the last report
 constexpr int BOUND_SMALL_CELLS = 524288, BOUND_SMALL_BATCH_CELLS = 131072, BOUND_TRUST_CELLS = 49152;
-constexpr int SMALL_CANDS = 512;   // more candidates are left to the separate launches
+// candidates past which the separate launches are faster: of the first pass, which
+// the workgroup itself can look at, and per pass in the mean
+constexpr int SMALL_CANDS = 512, SMALL_CANDS_PER_PASS = 350;
 
 constexpr int DETECT_BLOCK = 256;
 
@@ -359,8 +361,9 @@ size_t bound_record_bytes(int maxCellFaces);
 void launch_count_warped(const DevMesh& m, int* count, hipStream_t s);  // faces below flatness 1 - tSmall
 // whether one workgroup may take all bounding passes of this mesh
 bool bound_small(const DevMesh& m, const DevState& st);
-// what the GPU last reported of a first bounding pass
+// what the GPU last reported of a step's bounding
 inline int bound_last(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport & 0xffffffffull); }
+inline long bound_last_sum(const DevState& st) { return (long)((const volatile unsigned long long*)st.bndReport)[1]; }
 inline int bound_last_epoch(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport >> 32); }
 // the state of bounding pass number seq of a handle: the half (seq & 1) of
 // the double-buffered bounding arrays
