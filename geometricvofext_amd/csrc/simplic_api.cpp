@@ -633,18 +633,14 @@ public:
 
     void timers(double& rec, double& adv, uint64_t& nic) {
         // what the kernels of the stages noted (in ticks of the GPU's clock)
-        launch_stage_fold(st_, stream_);
+        launch_stage_fold(st_, times_.p, stream_);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipStreamSynchronize(stream_));
-        unsigned long long sum[2];
-        HIPCHECK(hipMemcpy(sum, st_.clock + 2, sizeof sum, hipMemcpyDeviceToHost));
         int rate = 0;   // kHz
         HIPCHECK(hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, device_));
-        rec = 1e-3 * (double)sum[0] / rate;
-        adv = 1e-3 * (double)sum[1] / rate;
-        unsigned long long n = 0;
-        HIPCHECK(hipMemcpy(&n, st_.nIcTotal, sizeof(n), hipMemcpyDeviceToHost));
-        nic = n;
+        rec = 1e-3 * (double)times_.p[0] / rate;
+        adv = 1e-3 * (double)times_.p[1] / rate;
+        nic = times_.p[2];
     }
 
     // Batched stepping (class caseBatch): whether this handle's step is the
@@ -700,7 +696,7 @@ public:
     double* U0_ = nullptr;
     double* phi0_ = nullptr;
     double* U0b_ = nullptr;
-    HostOut courant_, finite_, status_;   // apart: one call's words are not another's
+    HostOut courant_, finite_, status_, times_;   // apart: one call's words are not another's
     int* nonfinite_ = nullptr;   // count of warped faces
     std::vector<double> hostC_, hostCf_, hostSf_;
     // learned orientation method
@@ -1096,6 +1092,7 @@ private:
         courant_.alloc(courant_blocks(1, m_.nC));
         finite_.alloc(count_blocks(std::max<long>(m_.nF, 3L * m_.nC)));
         status_.alloc(2);
+        times_.alloc(2);
         st_.bndReport = status_.p + 2;
         st_.bndReport[0] = st_.bndReport[1] = 0;
         fieldChanged();

@@ -325,8 +325,18 @@ __global__ void __launch_bounds__(DETECT_LIST_THREADS) k_detect_list(DevMesh m, 
     k_detect_list_body(m, st, tol, nBlocks);
 }
 
-__global__ void __launch_bounds__(64) k_stage_fold(DevState st) { stage_fold(st, threadIdx.x); }
-void launch_stage_fold(const DevState& st, hipStream_t s) { k_stage_fold<<<1, 64, 0, s>>>(st); }
+// the stages' times up to here (ticks) and the running sum of mixed cells, to
+// host memory in one go, as k_status
+__global__ void __launch_bounds__(64) k_stage_fold(DevState st, unsigned long long* out) {
+    stage_fold(st, threadIdx.x);
+    if (threadIdx.x != 0) return;
+    out[0] = st.clock[2];
+    out[1] = st.clock[3];
+    out[2] = *st.nIcTotal;
+}
+void launch_stage_fold(const DevState& st, unsigned long long* out, hipStream_t s) {
+    k_stage_fold<<<1, 64, 0, s>>>(st, out);
+}
 
 void launch_detect(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s) {
     const int nb = cdiv(m.nC, DETECT_LIST_CELLS);

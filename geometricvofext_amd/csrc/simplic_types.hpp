@@ -275,7 +275,7 @@ struct BatchDims {
 
 // launchers (simplic_kernels.hip)
 void launch_geometry(const DevMesh& m, hipStream_t s);
-void launch_stage_fold(const DevState& st, hipStream_t s);
+void launch_stage_fold(const DevState& st, unsigned long long* out, hipStream_t s);
 void launch_detect(const DevMesh& m, const DevState& st, const Params& p, hipStream_t s);
 // wl/wn: optional device list of mixed-cell positions and its length
 void launch_ls_normal(const DevMesh& m, const DevState& st, hipStream_t s, const int* wl = nullptr,
