@@ -2846,10 +2846,10 @@ void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, doubl
     int behind = 0;
     if constexpr (MF <= NS_CELL_FACES) {
         const bool trust = m.nC <= BOUND_TRUST_CELLS;
-        const int reported = bound_last_epoch(st);
-        const bool few = trust ? bound_last_sum(st) <= (long)SMALL_CANDS_PER_PASS * nPasses : bound_last(st) <= SMALL_CANDS;
+        const BoundReport last = bound_last(st);
+        const bool few = trust ? bound_last_sum(st) <= (long)SMALL_CANDS_PER_PASS * nPasses : last.first <= SMALL_CANDS;
         if (nPasses > 0 && bound_small(m, st) && few) {
-            behind = !trust && reported <= st.bndSince;
+            behind = !trust && last.epoch <= st.bndSince;
             k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
                                                          bound_half(bound_pass_view(m, st, *passSeq + 1)), nPasses, dt,
                                                          Sp, Su, behind);

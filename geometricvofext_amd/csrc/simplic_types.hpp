@@ -361,10 +361,16 @@ size_t bound_record_bytes(int maxCellFaces);
 void launch_count_warped(const DevMesh& m, int* count, hipStream_t s);  // faces below flatness 1 - tSmall
 // whether one workgroup may take all bounding passes of this mesh
 bool bound_small(const DevMesh& m, const DevState& st);
-// what the GPU last reported of a step's bounding
-inline int bound_last(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport & 0xffffffffull); }
+// what the GPU last reported of a step's bounding: number of the reconstruct and
+// candidates of the first pass (one word, read once), and of all passes
+struct BoundReport {
+    int epoch, first;
+};
+inline BoundReport bound_last(const DevState& st) {
+    const unsigned long long w = *(const volatile unsigned long long*)st.bndReport;
+    return BoundReport{(int)(w >> 32), (int)(w & 0xffffffffull)};
+}
 inline long bound_last_sum(const DevState& st) { return (long)((const volatile unsigned long long*)st.bndReport)[1]; }
-inline int bound_last_epoch(const DevState& st) { return (int)(*(const volatile unsigned long long*)st.bndReport >> 32); }
 // the state of bounding pass number seq of a handle: the half (seq & 1) of
 // the double-buffered bounding arrays
 DevState bound_pass_view(const DevMesh& m, const DevState& st, int seq);
