@@ -2833,13 +2833,14 @@ bool bound_small(const DevMesh& m, const DevState& st) {
 // Whole steps, one workgroup against separate launches, perturbed hexahedra: 36^3,
 // 3 passes, 384 + 331 + 337 candidates 216 us and 211, 666 + 352 + 309 243 and 226,
 // 1136 + 374 + 303 290 and 247; plain ones, 673 + 112 + 10 196 and 204; 10 passes,
-// about 320 each, 384 and 470, 1142 in the first of them 438 and 471.
+// about 320 each, 384 and 470, 1142 in the first of them 438 and 471; 38^3, 3
+// passes, 459 + 403 + 399 237 and 214.
 // The counts may be a few steps old.  On meshes of up to BOUND_TRUST_CELLS a count
 // that grew meanwhile costs one step a fraction of what the measured ones show.
-// On larger ones the line is at the first pass's count, and where that may have
-// grown much (a new alpha or flow, a longer step) since the report, the workgroup
-// looks itself: where it declines, the separate launches, queued behind it in any
-// case, do the work.
+// On larger ones the first pass's count has a line of its own, and where it may
+// have grown much (a new alpha or flow, a longer step) since the report, the
+// workgroup looks itself: where it declines, the separate launches, queued behind
+// it in any case, do the work.
 template <int MF>
 void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, double dt, const double* Sp,
                         const double* Su, int* passSeq, hipStream_t s) {
@@ -2847,7 +2848,8 @@ void launch_bound_faces(const DevMesh& m, const DevState& st, int nPasses, doubl
     if constexpr (MF <= NS_CELL_FACES) {
         const bool trust = m.nC <= BOUND_TRUST_CELLS;
         const BoundReport last = bound_last(st);
-        const bool few = trust ? bound_last_sum(st) <= (long)SMALL_CANDS_PER_PASS * nPasses : last.first <= SMALL_CANDS;
+        const bool few = bound_last_sum(st) <= (long)SMALL_CANDS_PER_PASS * nPasses &&
+                         (trust || last.first <= SMALL_CANDS);
         if (nPasses > 0 && bound_small(m, st) && few) {
             behind = !trust && last.epoch <= st.bndSince;
             k_bnd_small<MF><<<1, SMALL_THREADS, 0, s>>>(m, bound_pass_view(m, st, *passSeq),
